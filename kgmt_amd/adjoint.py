@@ -14,8 +14,8 @@ obstacles are rows of 6 floats shared by every trajectory.
     history = refine(u, x0, goal, steps, obstacles, cfg, params)   # Adam, in place
 
 The cost J = w_e sum_t |u_t - u_ref|^2 + w_o sum_{t>=1} sum_b tau softplus((m - sd(p_t, b)) / tau)
-+ w_g |p_T - goal|^2 and its gradient are computed in FP32 by one lane per
-trajectory on the GPU; there is no CPU path.
++ w_g |p_T - goal|^2 and its gradient are computed in FP32 on the GPU (16 to
+64 lanes per trajectory); there is no CPU path.
 """
 from __future__ import annotations
 

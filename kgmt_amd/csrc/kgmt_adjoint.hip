@@ -1,380 +1,615 @@
 // kgmt_adjoint.hip — differentiable RK4 rollout of the quadcopter ODE on gfx950.
 //
-// Refinement of found control sequences (an extension beside the planner):
-// one lane per trajectory integrates x_{t+1} = RK4(x_t, u_t) forward, keeping
-// the state at every step as a checkpoint, then runs the discrete adjoint
-// backwards: each RK4 step's four stages are recomputed from its checkpoint
-// and their vector-Jacobian products chained (stage recomputation instead of
-// storing 4x12 stage values per step). The cost is
+// Refinement of found control sequences (an extension beside the planner).
+// A trajectory integrates x_{t+1} = RK4(x_t, u_t) forward and runs the
+// discrete adjoint of those steps backward. The cost is
 //   J = w_e sum |u_t - u_ref|^2 + w_o sum_{t>=1} sum_b tau softplus((m - sd(p_t, b)) / tau)
 //     + w_g |p_T - goal|^2.
-// k_adjoint<false> writes J and dJ/du; k_adjoint<true> runs Adam for
+// k_rollout<false> writes J and dJ/du; k_rollout<true> runs Adam for
 // `iterations` steps in place and records J before every step and after the
 // last. The dynamics are those of statePropagator.cu:325-370 (ode).
+//
+// What bounds it: the time steps form a chain, and a wave issues at most one
+// vector instruction every 4 cycles, so the time of a pass is the number of
+// instructions on the chain. Only what must follow the chain stays on it:
+//   1. forward chain: attitude and body velocities. The position feeds back
+//      into nothing, so it is left out. Lane c of a quad carries component c
+//      of the angles, the body velocity and the body rates; one sin/cos, one
+//      cross product and one square root serve all three components, and a
+//      step takes a quarter of the instructions that one lane would need. The
+//      four stages' states are kept for the passes below.
+//   2. positions, penalties and J, lane = (step, stage): the stages' world
+//      velocities, their sum over a step by quad permutations, a scan over the
+//      steps, then the boxes spread over the trajectory's lanes.
+//   3. backward, lane = (step, stage): the stage's vector-Jacobian product as
+//      eight rows of coefficients in LDS (the adjoints of the positions and of
+//      psi do not depend on the others: suffix sums over the steps, folded
+//      into the rows' constants), then the backward chain: lane j of a row of
+//      16 lanes holds adjoint j, and a stage is eight multiply-adds with
+//      broadcast operands.
+// The kernel that ran the whole step in every lane of a trajectory took
+// 47.2 ms for 4096 trajectories (20..80 steps, 50 Adam steps, 50 boxes),
+// 1.18 ms for one cost and gradient of them and 1.42 ms for 333 trajectories
+// among 301 boxes; this one takes 7.33, 0.21 and 0.11 ms, and its error
+// against 64 bits is smaller (gradient of the 333: 2.2e-6 to 5.8e-7).
+#include <algorithm>
+
 #include "kgmt_launch.hpp"
+
+#pragma clang fp contract(fast)
 
 namespace kgmt
 {
 
-// dynamics constants of one configuration (quad parameters, dt)
-struct QuadK
+namespace
 {
-    float h, hh, h6, h3;
-    float g, minv, nu, mu;
-    float ax, bx, ay, by, az, bz;
+
+// sin and cos as sincos_k (the same reduction and polynomials) with fused
+// multiply-adds
+__device__ __forceinline__ void sincos_fused(float x, float& s, float& c)
+{
+    const float fk = __builtin_rintf(x * 0x1.45f306p-1f);
+    float r        = __builtin_fmaf(-fk, 0x1.92p+0f, x);
+    r              = __builtin_fmaf(-fk, 0x1.fb4p-12f, r);
+    r              = __builtin_fmaf(-fk, 0x1.4442d2p-24f, r);
+    const int m    = (int)fk;
+    const float z  = r * r;
+    float ps       = __builtin_fmaf(0x1.71de3ap-19f, z, -0x1.a01a02p-13f);
+    ps             = __builtin_fmaf(ps, z, 0x1.111112p-7f);
+    ps             = __builtin_fmaf(ps, z, -0x1.555556p-3f);
+    const float sr = __builtin_fmaf(r * z, ps, r);
+    float pc       = __builtin_fmaf(0x1.1eed8ep-29f, z, -0x1.27e4fcp-22f);
+    pc             = __builtin_fmaf(pc, z, 0x1.a01a02p-16f);
+    pc             = __builtin_fmaf(pc, z, -0x1.6c16c2p-10f);
+    pc             = __builtin_fmaf(pc, z, 0x1.555556p-5f);
+    const float cr = __builtin_fmaf(z * z, pc, __builtin_fmaf(-0.5f, z, 1.0f));
+    const float a  = (m & 1) ? cr : sr;
+    const float b  = (m & 1) ? sr : cr;
+    s              = (m & 2) ? -a : a;
+    c              = ((m + 1) & 2) ? -b : b;
+}
+
+// (s, c) turned by the small angle d (|d| < 0.1: the series' first term left
+// out is below 3e-10)
+__device__ __forceinline__ void turn(float s0, float c0, float d, float& s, float& c)
+{
+    const float z  = d * d;
+    const float sd = __builtin_fmaf(d * z, __builtin_fmaf(z, 1.0f / 120.0f, -1.0f / 6.0f), d);
+    const float cm = z * __builtin_fmaf(z, __builtin_fmaf(z, -1.0f / 720.0f, 1.0f / 24.0f), -0.5f);  // cos d - 1
+    s              = __builtin_fmaf(c0, sd, __builtin_fmaf(s0, cm, s0));
+    c              = __builtin_fmaf(-s0, sd, __builtin_fmaf(c0, cm, c0));
+}
+
+// 1 / x within one ulp
+__device__ __forceinline__ float recip(float x)
+{
+    return __builtin_amdgcn_rcpf(x);
+}
+
+// v of the lane that the DPP control selects (every control used here stays
+// inside the row)
+template <int CTRL>
+__device__ __forceinline__ float dpp(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+constexpr int kQuad0 = 0x00, kQuad1 = 0x55, kQuad2 = 0xAA, kQuad3 = 0xFF;  // quad_perm: one lane to its quad
+constexpr int kNext  = 0xC9;   // quad_perm [1,2,0,3]: component c + 1 of three
+constexpr int kPrev  = 0xD2;   // quad_perm [2,0,1,3]: component c + 2
+
+// y += sum over k < 8 of x of lane k of the row times ck: eight multiply-adds
+// that read their broadcast operand by DPP (the compiler keeps a move before
+// each). A DPP read needs two wait states after the write of x: the s_nop.
+__device__ __forceinline__ void row_madd(float& y, float x, float c0, float c1, float c2, float c3, float c4, float c5,
+                                         float c6, float c7)
+{
+#define KGMT_MADD(K, R) "v_fmac_f32_dpp %0, %1, " R " row_newbcast:" K " row_mask:0xf bank_mask:0xf\n\t"
+    asm("s_nop 1\n\t" KGMT_MADD("0", "%2") KGMT_MADD("1", "%3") KGMT_MADD("2", "%4") KGMT_MADD("3", "%5")
+          KGMT_MADD("4", "%6") KGMT_MADD("5", "%7") KGMT_MADD("6", "%8") KGMT_MADD("7", "%9")
+        : "+&v"(y)  // written before the last operands are read
+        : "v"(x), "v"(c0), "v"(c1), "v"(c2), "v"(c3), "v"(c4), "v"(c5), "v"(c6), "v"(c7));
+#undef KGMT_MADD
+}
+
+__device__ __forceinline__ float quad_sum(float v)
+{
+    v += dpp<0xB1>(v);
+    return v + dpp<0x4E>(v);
+}
+
+// four values per lane -> lane c of the quad holds the quad's sum of v[c]
+__device__ __forceinline__ float quad_scatter(const float (&v)[4], int lane)
+{
+    const bool b1 = lane & 2, b0 = lane & 1;
+    const float x = (b1 ? v[2] : v[0]) + dpp<0x4E>(b1 ? v[0] : v[2]);
+    const float y = (b1 ? v[3] : v[1]) + dpp<0x4E>(b1 ? v[1] : v[3]);
+    return (b0 ? y : x) + dpp<0xB1>(b0 ? x : y);
+}
+
+// tau * softplus((margin - sd) / tau) of one box at p, and its gradient
+// (times -w): softplus(z) = max(z, 0) + log1p(e) and its derivative
+// (1 or e) / (1 + e) with e = exp(-|z|); log1p(e) = 2 atanh(e / (2 + e)).
+// The error of z (of the position, over tau) is larger than that of exp2
+// of the rounded product.
+__device__ __forceinline__ void box_penalty(float4 lo, float4 hi, float px, float py, float pz, float margin,
+                                            float itau, float tau, float w, float (&acc)[4])
+{
+    const float lx = lo.x - px, hx = px - hi.x, ly = lo.y - py, hy = py - hi.y, lz = lo.z - pz, hz = pz - hi.z;
+    const bool nx = lx > hx, ny = ly > hy, nz = lz > hz;  // nearer the low face
+    const float qx = nx ? lx : hx, qy = ny ? ly : hy, qz = nz ? lz : hz;
+    const float ox = fmaxf(qx, 0.0f), oy = fmaxf(qy, 0.0f), oz = fmaxf(qz, 0.0f);
+    const float d2 = ox * ox + oy * oy + oz * oz;
+    const float id = __builtin_amdgcn_rsqf(d2);
+    float sd       = d2 * id;
+    // outside: (ox, oy, oz) / distance; inside (rare: one vote of the active
+    // lanes skips it): the axis of the nearest face, the first of the largest
+    float vx = ox * id, vy = oy * id, vz = oz * id;
+    if(__any(!(d2 > 0.0f) | __builtin_isunordered(qx, qy) | (qz != qz)))
+        {
+            const bool out = d2 > 0.0f;
+            const bool xy = qx >= qy, ax = xy & (qx >= qz), ay = !xy & (qy >= qz);
+            sd = (out ? sd : 0.0f) + fminf(ax ? qx : ay ? qy : qz, 0.0f);
+            vx = out ? vx : ax ? 1.0f : 0.0f, vy = out ? vy : ay ? 1.0f : 0.0f;
+            vz = out ? vz : (ax | ay) ? 0.0f : 1.0f;
+        }
+    const float z = (margin - sd) * itau;
+    const float e = __builtin_amdgcn_exp2f(-1.44269504f * fabsf(z));
+    // one reciprocal for 1 / (2 + e) and 1 / (1 + e)
+    const float e1 = 1.0f + e, e2 = 2.0f + e, re = recip(e1 * e2);
+    const float s = e * e1 * re, s2 = s * s;
+    float at      = __builtin_fmaf(s2, 2.0f / 15.0f, 2.0f / 13.0f);
+    at            = __builtin_fmaf(s2, at, 2.0f / 11.0f);
+    at            = __builtin_fmaf(s2, at, 2.0f / 9.0f);
+    at            = __builtin_fmaf(s2, at, 2.0f / 7.0f);
+    at            = __builtin_fmaf(s2, at, 2.0f / 5.0f);
+    at            = __builtin_fmaf(s2, at, 2.0f / 3.0f);
+    at            = __builtin_fmaf(s2, at, 2.0f);
+    acc[0]        = __builtin_fmaf(tau, __builtin_fmaf(s, at, fmaxf(z, 0.0f)), acc[0]);
+    const float ds = -w * (z >= 0.0f ? 1.0f : e) * e2 * re;
+    acc[1]         = __builtin_fmaf(nx ? -ds : ds, vx, acc[1]);
+    acc[2]         = __builtin_fmaf(ny ? -ds : ds, vy, acc[2]);
+    acc[3]         = __builtin_fmaf(nz ? -ds : ds, vz, acc[3]);
+}
+
+constexpr int kRowWords   = 12;   // a row of coefficients: constant, then those of a3 a4 a6 a7 a8 a9 a10 a11
+constexpr int kBlockWords = 100;  // eight rows of one (step, stage), padded: 16 lanes' blocks start in distinct banks
+constexpr int kStageWords = 48;   // kept per step: angles, velocity, rates, each [4 stages][4]
+
+// box slots of the LDS for n boxes: the next four of a lane's last box fit
+__host__ __device__ constexpr uint32_t box_slots(uint32_t n)
+{
+    return n + 8;
+}
+
+struct RolloutLds
+{
+    float coef[64 * kBlockWords];
+    float ubar[64];
 };
 
-// d(ode)/d(state)^T a and d(ode)/d(control)^T a, FP32 (same derivation as
-// the oracle's FP64 orc_quad_vjp_f64)
-__device__ __forceinline__ void quad_vjp(const QuadK& K, const float* s, const float* a, float* gs, float* gc)
-{
-    const float u = s[6], v = s[7], w = s[8], p = s[9], q = s[10], r = s[11];
-    float sf, cf, st, ct, sp, cp;
-    sincos_k(s[3], sf, cf);
-    sincos_k(s[4], st, ct);
-    sincos_k(s[5], sp, cp);
-    const float tt = st / ct, ict = 1.0f / ct;
-    const float R00 = ct * cp, R01 = sf * st * cp - cf * sp, R02 = cf * st * cp + sf * sp;
-    const float R10 = ct * sp, R11 = sf * st * sp + cf * cp, R12 = cf * st * sp - sf * cp;
-    const float R20 = -st, R21 = sf * ct, R22 = cf * ct;
-    const float a0 = a[0], a1 = a[1], a2 = a[2], a3 = a[3], a4 = a[4], a5 = a[5];
-    const float a6 = a[6], a7 = a[7], a8 = a[8], a9 = a[9], a10 = a[10], a11 = a[11];
-    float g3 = 0.0f, g4 = 0.0f, g5 = 0.0f, g6, g7, g8, g9, g10, g11;
-    g6 = R00 * a0 + R10 * a1 + R20 * a2;
-    g7 = R01 * a0 + R11 * a1 + R21 * a2;
-    g8 = R02 * a0 + R12 * a1 + R22 * a2;
-    const float d0f = (cf * st * cp + sf * sp) * v + (-sf * st * cp + cf * sp) * w;
-    const float d1f = (cf * st * sp - sf * cp) * v + (-sf * st * sp - cf * cp) * w;
-    const float d2f = cf * ct * v - sf * ct * w;
-    const float d0t = -st * cp * u + sf * ct * cp * v + cf * ct * cp * w;
-    const float d1t = -st * sp * u + sf * ct * sp * v + cf * ct * sp * w;
-    const float d2t = -ct * u - sf * st * v - cf * st * w;
-    const float f0 = R00 * u + R01 * v + R02 * w, f1 = R10 * u + R11 * v + R12 * w;
-    g3 += d0f * a0 + d1f * a1 + d2f * a2;
-    g4 += d0t * a0 + d1t * a1 + d2t * a2;
-    g5 += -f1 * a0 + f0 * a1;
-    const float E = q * sf + r * cf, F = q * cf - r * sf;
-    g3 += F * tt * a3 - E * a4 + F * ict * a5;
-    g4 += E * ict * ict * a3 + E * st * ict * ict * a5;
-    g9  = a3;
-    g10 = sf * tt * a3 + cf * a4 + sf * ict * a5;
-    g11 = cf * tt * a3 - sf * a4 + cf * ict * a5;
-    g7 += r * a6 - p * a8;
-    g8 += -q * a6 + p * a7;
-    g6 += -r * a7 + q * a8;
-    g9 += w * a7 - v * a8;
-    g10 += -w * a6 + u * a8;
-    g11 += v * a6 - u * a7;
-    g4 += -K.g * ct * a6 - K.g * st * sf * a7 - K.g * st * cf * a8;
-    g3 += K.g * ct * cf * a7 - K.g * ct * sf * a8;
-    const float nv = __builtin_sqrtf(u * u + v * v + w * w);
-    const float N  = -K.nu * nv;
-    g6 += K.minv * N * a6;
-    g7 += K.minv * N * a7;
-    g8 += K.minv * N * a8;
-    if(nv > 0.0f)
-        {
-            const float k = K.minv * (-K.nu) / nv * (u * a6 + v * a7 + w * a8);
-            g6 += k * u, g7 += k * v, g8 += k * w;
-        }
-    g10 += K.ax * r * a9;
-    g11 += K.ax * q * a9;
-    g9 += K.ay * r * a10;
-    g11 += K.ay * p * a10;
-    g9 += K.az * q * a11;
-    g10 += K.az * p * a11;
-    const float nw = __builtin_sqrtf(p * p + q * q + r * r);
-    const float M  = -K.mu * nw;
-    const float b9 = K.bx * a9, b10 = K.by * a10, b11 = K.bz * a11;
-    g9 += M * b9, g10 += M * b10, g11 += M * b11;
-    if(nw > 0.0f)
-        {
-            const float k = (-K.mu) / nw * (p * b9 + q * b10 + r * b11);
-            g9 += k * p, g10 += k * q, g11 += k * r;
-        }
-    gs[0] = 0.0f, gs[1] = 0.0f, gs[2] = 0.0f;
-    gs[3] = g3, gs[4] = g4, gs[5] = g5, gs[6] = g6, gs[7] = g7, gs[8] = g8;
-    gs[9] = g9, gs[10] = g10, gs[11] = g11;
-    gc[0] = K.minv * a8;
-    gc[1] = K.bx * a9;
-    gc[2] = K.by * a10;
-    gc[3] = K.bz * a11;
-}
+}  // namespace
 
-__device__ __forceinline__ void rk4_step(const QueryDesc& qd, const QuadK& K, float* x, const float* uc)
-{
-    float k1[12], k2[12], k3[12], k4[12], st[12];
-    quad_ode(qd, x, uc, k1);
-#pragma unroll
-    for(int j = 0; j < 12; ++j) st[j] = x[j] + K.hh * k1[j];
-    quad_ode(qd, st, uc, k2);
-#pragma unroll
-    for(int j = 0; j < 12; ++j) st[j] = x[j] + K.hh * k2[j];
-    quad_ode(qd, st, uc, k3);
-#pragma unroll
-    for(int j = 0; j < 12; ++j) st[j] = x[j] + K.h * k3[j];
-    quad_ode(qd, st, uc, k4);
-#pragma unroll
-    for(int j = 0; j < 12; ++j) x[j] = x[j] + K.h6 * (k1[j] + 2.0f * k2[j] + 2.0f * k3[j] + k4[j]);
-}
-
-// xbar = J_x^T lam, ubar = J_u^T lam of one RK4 step from checkpoint x
-__device__ __forceinline__ void rk4_vjp(const QueryDesc& qd, const QuadK& K, const float* x, const float* uc,
-                                        const float* lam, float* xbar, float* ubar)
-{
-    float k[12], s2[12], s3[12], s4[12];
-    quad_ode(qd, x, uc, k);
-#pragma unroll
-    for(int j = 0; j < 12; ++j) s2[j] = x[j] + K.hh * k[j];
-    quad_ode(qd, s2, uc, k);
-#pragma unroll
-    for(int j = 0; j < 12; ++j) s3[j] = x[j] + K.hh * k[j];
-    quad_ode(qd, s3, uc, k);
-#pragma unroll
-    for(int j = 0; j < 12; ++j) s4[j] = x[j] + K.h * k[j];
-    float kb[12], gs[12], gc[4];
-#pragma unroll
-    for(int j = 0; j < 12; ++j) xbar[j] = lam[j], kb[j] = K.h6 * lam[j];
-    ubar[0] = ubar[1] = ubar[2] = ubar[3] = 0.0f;
-    // stage 4: k4 = f(s4), s4 = x + h k3
-    quad_vjp(K, s4, kb, gs, gc);
-#pragma unroll
-    for(int j = 0; j < 12; ++j) xbar[j] += gs[j], kb[j] = K.h3 * lam[j] + K.h * gs[j];
-#pragma unroll
-    for(int i = 0; i < 4; ++i) ubar[i] += gc[i];
-    // stage 3: k3 = f(s3), s3 = x + h/2 k2
-    quad_vjp(K, s3, kb, gs, gc);
-#pragma unroll
-    for(int j = 0; j < 12; ++j) xbar[j] += gs[j], kb[j] = K.h3 * lam[j] + K.hh * gs[j];
-#pragma unroll
-    for(int i = 0; i < 4; ++i) ubar[i] += gc[i];
-    // stage 2: k2 = f(s2), s2 = x + h/2 k1
-    quad_vjp(K, s2, kb, gs, gc);
-#pragma unroll
-    for(int j = 0; j < 12; ++j) xbar[j] += gs[j], kb[j] = K.h6 * lam[j] + K.hh * gs[j];
-#pragma unroll
-    for(int i = 0; i < 4; ++i) ubar[i] += gc[i];
-    // stage 1: k1 = f(x)
-    quad_vjp(K, x, kb, gs, gc);
-#pragma unroll
-    for(int j = 0; j < 12; ++j) xbar[j] += gs[j];
-#pragma unroll
-    for(int i = 0; i < 4; ++i) ubar[i] += gc[i];
-}
-
-// lanes per trajectory: they run the same rollout (same operations, same
-// bits) and split the obstacle penalty's boxes
-constexpr int kLanes = 16;
-
-// v + v of the lane the DPP control selects (all 16 lanes of the row active)
-template <int CTRL>
-__device__ __forceinline__ float dpp_add(float v)
-{
-    return v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, false));
-}
-
-// sum over a row of 16 lanes, the same bits in every lane: lane ^ 1, lane ^ 2
-// (quad permutations), then the half-row and row mirrors
-__device__ __forceinline__ float group_sum(float v)
-{
-    static_assert(kLanes == 16, "one DPP row per trajectory");
-    v = dpp_add<0xB1>(v);   // quad_perm [1,0,3,2]
-    v = dpp_add<0x4E>(v);   // quad_perm [2,3,0,1]
-    v = dpp_add<0x141>(v);  // row_half_mirror
-    v = dpp_add<0x140>(v);  // row_mirror
-    return v;
-}
-
-// sum over boxes of tau * softplus((margin - sd(p, box)) / tau), boxes
-// sub, sub + kLanes, ... in this lane, summed over the trajectory's lanes;
-// with gp, adds scale * gradient with respect to p
-__device__ __forceinline__ float penalty(const kgmt_adjoint_params& ap, const float* p, const float4* sObs, int nObs,
-                                         float scale, float* gp, int sub)
-{
-    float total = 0.0f, g0 = 0.0f, g1 = 0.0f, g2 = 0.0f;
-    for(int o = sub; o < nObs; o += kLanes)
-        {
-            const float4 lo4 = sObs[2 * o], hi4 = sObs[2 * o + 1];
-            const float lo[3] = {lo4.x, lo4.y, lo4.z}, hi[3] = {hi4.x, hi4.y, hi4.z};
-            float qv[3], sgn[3];
-#pragma unroll
-            for(int d = 0; d < 3; ++d)
-                {
-                    const float l = lo[d] - p[d], h = p[d] - hi[d];
-                    qv[d]  = l > h ? l : h;
-                    sgn[d] = l > h ? -1.0f : 1.0f;
-                }
-            const float ox = qv[0] > 0.0f ? qv[0] : 0.0f, oy = qv[1] > 0.0f ? qv[1] : 0.0f;
-            const float oz      = qv[2] > 0.0f ? qv[2] : 0.0f;
-            const float outside = __builtin_sqrtf(ox * ox + oy * oy + oz * oz);
-            const int am = qv[0] >= qv[1] ? (qv[0] >= qv[2] ? 0 : 2) : (qv[1] >= qv[2] ? 1 : 2);
-            const float inside = qv[am] < 0.0f ? qv[am] : 0.0f;
-            const float z      = (ap.margin - (outside + inside)) / ap.tau;
-            total += ap.tau * (z > 30.0f ? z : log1pf(expf(z)));
-            if(gp)
-                {
-                    const float dsd = -scale / (1.0f + expf(-z));
-                    if(outside > 0.0f)
-                        {
-                            g0 += dsd * (ox / outside) * sgn[0];
-                            g1 += dsd * (oy / outside) * sgn[1];
-                            g2 += dsd * (oz / outside) * sgn[2];
-                        }
-                    else
-                        {
-                            const float gd = dsd * sgn[am];
-                            g0 += am == 0 ? gd : 0.0f;
-                            g1 += am == 1 ? gd : 0.0f;
-                            g2 += am == 2 ? gd : 0.0f;
-                        }
-                }
-        }
-    if(gp)
-        {
-            gp[0] += group_sum(g0);
-            gp[1] += group_sum(g1);
-            gp[2] += group_sum(g2);
-        }
-    return group_sum(total);
-}
-
-// kLanes lanes per trajectory; every lane of a trajectory computes and writes
-// the same values (the same address and value from each lane)
-template <bool REFINE>
-__global__ __launch_bounds__(64) void k_adjoint(const QueryDesc* __restrict__ qdp, kgmt_adjoint_params ap,
-                                                uint32_t n, uint32_t maxT, const int32_t* __restrict__ steps,
+// LPT lanes per trajectory (64 / LPT trajectories per wave, one wave per
+// workgroup); LPT / 4 steps per round of passes 2 and 3. work: per trajectory
+// of this launch maxT * (kStageWords + 8 [+ 8]) floats: stage states, per step
+// the penalty, its gradient and the controls, and, when refining, the Adam
+// moments. (The controls are copied first: the caller's layout puts a
+// trajectory's steps 16 n bytes apart, a page each, and the chain would wait
+// for each of them.)
+template <bool REFINE, int LPT>
+__global__ __launch_bounds__(64) void k_rollout(RolloutK K, kgmt_adjoint_params ap, uint32_t i0, uint32_t n,
+                                                uint32_t maxT, const int32_t* __restrict__ steps,
                                                 const float* __restrict__ x0g, const float* __restrict__ goalg,
-                                                float* __restrict__ u, float* __restrict__ grad,
-                                                float* __restrict__ ckpt, float* __restrict__ mom,
-                                                float* __restrict__ vel, const float4* __restrict__ obs,
-                                                uint32_t nObs, float* __restrict__ cost)
+                                                float* u, float* __restrict__ grad, float* work,
+                                                const float* __restrict__ rows, uint32_t nObs,
+                                                float* __restrict__ cost)
 {
-    extern __shared__ float4 sObs[];
-    for(uint32_t k = threadIdx.x; k < 2 * nObs; k += blockDim.x) sObs[k] = obs[k];
+    constexpr int CH = LPT / 4;  // steps per round
+    extern __shared__ float4 sBox[];  // low corners, then high corners
+    __shared__ RolloutLds L;
+    const int lane = (int)threadIdx.x;
+    const uint32_t nBox = box_slots(nObs);  // the read ahead ends inside the slots (unused ones hold anything)
+    for(uint32_t k = lane; k < nObs; k += 64)
+        {
+            const float* r = rows + 6 * (size_t)k;
+            sBox[k]        = make_float4(r[0], r[1], r[2], 0.0f);
+            sBox[nBox + k] = make_float4(r[3], r[4], r[5], 0.0f);
+        }
     __syncthreads();
-    const uint32_t i = (blockIdx.x * blockDim.x + threadIdx.x) / kLanes;
-    const int sub    = (int)(threadIdx.x % kLanes);
-    if(i >= n) return;  // whole groups of kLanes lanes leave together
-    const QueryDesc& qd  = *qdp;
-    const kgmt_config& c = qd.cfg;
-    QuadK K;
-    K.h = c.dt, K.hh = 0.5f * c.dt, K.h6 = c.dt / 6.0f, K.h3 = c.dt / 3.0f;
-    K.g = c.gravity, K.minv = qd.qminv, K.nu = c.quad_nu, K.mu = c.quad_mu;
-    K.ax = qd.qax, K.bx = qd.qbx, K.ay = qd.qay, K.by = qd.qby, K.az = qd.qaz, K.bz = qd.qbz;
-    int T = steps[i];
-    if(T < 0) T = 0;
-    if(T > (int)maxT) T = (int)maxT;
-    const float gx = goalg[i], gy = goalg[(size_t)n + i], gz = goalg[2 * (size_t)n + i];
+    const uint32_t slot = (blockIdx.x * 64 + lane) / LPT;
+    const uint32_t i    = i0 + slot < n ? i0 + slot : n - 1;  // lanes past the end read the last trajectory
+    const bool act      = i0 + slot < n;                      // and write nothing
+    const int l         = lane % LPT;
+    const int tt = l >> 2, s = l & 3;  // passes 2 and 3: step of the round, stage (or control)
+    const int j  = l & 7;              // backward chain: row
+    const int gb = lane - l;           // first lane of the trajectory
+    const size_t N = n;
+    int T          = act ? steps[i] : 0;
+    T              = T < 0 ? 0 : (T > (int)maxT ? (int)maxT : T);
+    int Tm         = T;  // longest of the wave
+#pragma unroll
+    for(int o = LPT; o < 64; o <<= 1)
+        {
+            const int x = __shfl_xor(Tm, o, 64);
+            Tm          = x > Tm ? x : Tm;
+        }
+    Tm             = __builtin_amdgcn_readfirstlane(Tm);
+    float* W       = work + (size_t)slot * maxT * (kStageWords + 8 + (REFINE ? 8 : 0));
+    float* Wg      = W + (size_t)maxT * kStageWords;  // penalty (0) and its gradient (1..3) at x_{t+1}, u_t (4..7)
+    float* Wm      = Wg + (size_t)maxT * 8;           // moments [t][4] x 2
+    const float gx = goalg[i], gy = goalg[N + i], gz = goalg[2 * N + i];
+    const float p0x = x0g[i], p0y = x0g[N + i], p0z = x0g[2 * N + i];
+    const int c3     = s < 3 ? s : 2;  // forward chain: component of this lane (lane 3 repeats lane 2)
+    const float A0 = x0g[(3 + c3) * N + i], U0 = x0g[(6 + c3) * N + i], P0 = x0g[(9 + c3) * N + i];
+    const float qa = s == 0 ? K.ax : s == 1 ? K.ay : K.az, qb = s == 0 ? K.bx : s == 1 ? K.by : K.bz;
+    const float uref   = s == 0 ? ap.u_ref[0] : s == 1 ? ap.u_ref[1] : s == 2 ? ap.u_ref[2] : ap.u_ref[3];
+    const float uscale = s == 0 ? K.minv : s == 1 ? K.bx : s == 2 ? K.by : K.bz;
+    const float umin   = s == 0 ? K.cmin[0] : s == 1 ? K.cmin[1] : s == 2 ? K.cmin[2] : K.cmin[3];
+    const float umax   = s == 0 ? K.cmax[0] : s == 1 ? K.cmax[1] : s == 2 ? K.cmax[2] : K.cmax[3];
+    const float itau   = 1.0f / ap.tau;
+    const float hS     = s == 0 || s == 3 ? K.h6 : K.h3;  // weight of stage s in the step
+    const float* uF    = Wg + 4 + ((s + 1) & 3);  // forward: lane c takes control c + 1, lane 3 control 0
     const uint32_t iters = REFINE ? ap.iterations : 0;
+    for(int t0 = 0; t0 < Tm; t0 += 4 * CH)
+        {
+            float x[4];
+#pragma unroll
+            for(int k = 0; k < 4; ++k)
+                {
+                    const int t = t0 + k * CH + tt;
+                    x[k]        = u[((size_t)(t < Tm ? t : Tm - 1) * 4 + s) * N + i];
+                }
+#pragma unroll
+            for(int k = 0; k < 4; ++k)
+                {
+                    const int t = t0 + k * CH + tt;
+                    if(t < Tm) Wg[(size_t)t * 8 + 4 + s] = x[k];
+                }
+        }
+    __threadfence_block();
     float b1t = 1.0f, b2t = 1.0f;
     for(uint32_t it = 0; it <= iters; ++it)
         {
-            // forward rollout with checkpoints
-            float x[12];
-#pragma unroll
-            for(int j = 0; j < 12; ++j) x[j] = x0g[(size_t)j * n + i], ckpt[(size_t)j * n + i] = x[j];
-            float J = 0.0f;
-            for(int t = 0; t < T; ++t)
+            // 1. forward chain
+            {
+                float A = A0, U = U0, P = P0;
+                const float gd = -K.minv * K.nu, wd = -qb * K.mu;
+                float un = Tm > 0 ? uF[0] : 0.0f;
+                for(int t = 0; t < Tm; ++t)
+                    {
+                        const float uc = un;
+                        if(t + 1 < Tm) un = uF[(size_t)(t + 1) * 8];
+                        const float u0  = dpp<kQuad3>(uc);
+                        const float thr = s == 2 ? K.minv * u0 : 0.0f;
+                        const float tor = qb * uc;
+                        auto deriv = [&](float sn, float cs, float v, float w, float& da, float& dv, float& dw) {
+                            const float sph = dpp<kQuad0>(sn), cph = dpp<kQuad0>(cs);
+                            const float sth = dpp<kQuad1>(sn), cth = dpp<kQuad1>(cs);
+                            const float v1 = dpp<kNext>(v), v2 = dpp<kPrev>(v);
+                            const float w1 = dpp<kNext>(w), w2 = dpp<kPrev>(w);
+                            const float q = dpp<kQuad1>(w), r = dpp<kQuad2>(w);
+                            const float Ei = (q * sph + r * cph) * recip(cth);
+                            const float F  = q * cph - r * sph;
+                            da             = s == 0 ? w + Ei * sth : s == 1 ? F : Ei;
+                            const float gv = s == 0 ? -sth : cth * (s == 1 ? sph : cph);
+                            const float nv = __builtin_amdgcn_sqrtf(v * v + v1 * v1 + v2 * v2);
+                            dv = (w2 * v1 - w1 * v2) + K.g * gv + thr + gd * nv * v;
+                            const float nw = __builtin_amdgcn_sqrtf(w * w + w1 * w1 + w2 * w2);
+                            dw = qa * w1 * w2 + wd * nw * w + tor;
+                        };
+                        float a1, v1, w1, a2, v2, w2, a3, v3, w3, a4, v4, w4;
+                        // the stages' angles are the step's, turned by what
+                        // they advance (a fast spin or a long step: past
+                        // 0.1 rad in some lane, sin / cos of the stage's angle)
+                        float sn0, cs0, sn, cs;
+                        sincos_fused(A, sn0, cs0);
+                        auto angle = [&](float d) {
+                            if(__any(!(fabsf(d) < 0.1f)))
+                                sincos_fused(A + d, sn, cs);
+                            else
+                                turn(sn0, cs0, d, sn, cs);
+                        };
+                        // quad k of the row keeps stage k's state
+                        const int quad = (l >> 2) & 3;
+                        float kA = A, kU = U, kP = P, d, sv, sw;
+                        deriv(sn0, cs0, U, P, a1, v1, w1);
+                        d = K.hh * a1, sv = U + K.hh * v1, sw = P + K.hh * w1;
+                        angle(d);
+                        kA = quad == 1 ? A + d : kA, kU = quad == 1 ? sv : kU, kP = quad == 1 ? sw : kP;
+                        deriv(sn, cs, sv, sw, a2, v2, w2);
+                        d = K.hh * a2, sv = U + K.hh * v2, sw = P + K.hh * w2;
+                        angle(d);
+                        kA = quad == 2 ? A + d : kA, kU = quad == 2 ? sv : kU, kP = quad == 2 ? sw : kP;
+                        deriv(sn, cs, sv, sw, a3, v3, w3);
+                        d = K.h * a3, sv = U + K.h * v3, sw = P + K.h * w3;
+                        angle(d);
+                        kA = quad == 3 ? A + d : kA, kU = quad == 3 ? sv : kU, kP = quad == 3 ? sw : kP;
+                        deriv(sn, cs, sv, sw, a4, v4, w4);
+                        if(l < 16)
+                            {
+                                float* o = W + (size_t)t * kStageWords + l;
+                                o[0] = kA, o[16] = kU, o[32] = kP;
+                            }
+                        A = A + K.h6 * (a1 + 2.0f * a2 + 2.0f * a3 + a4);
+                        U = U + K.h6 * (v1 + 2.0f * v2 + 2.0f * v3 + v4);
+                        P = P + K.h6 * (w1 + 2.0f * w2 + 2.0f * w3 + w4);
+                    }
+            }
+            __threadfence_block();  // the stage states, read by other lanes below
+            // 2. positions, penalties, J
+            float px = p0x, py = p0y, pz = p0z, J = 0.0f;  // position at the end of the rounds before
+            // (each round's reads go out a round ahead)
+            const int tl = T > 0 ? T - 1 : 0;
+            float4 an, vn;
+            float dn = 0.0f;
+            auto fetch2 = [&](int t) {
+                const int tc     = t < tl ? t : tl;
+                const float4* w4 = reinterpret_cast<const float4*>(W + (size_t)tc * kStageWords);
+                an = w4[s], vn = w4[4 + s];
+                dn = Wg[(size_t)tc * 8 + 4 + s];
+            };
+            if(Tm > 0) fetch2(tt);
+            for(int t0 = 0; t0 < Tm; t0 += CH)
                 {
-                    float uc[4];
+                    const int t    = t0 + tt;
+                    const bool on  = t < T;
+                    const float4 a = an, v = vn;
+                    const float d  = dn - uref;
+                    fetch2(t + CH);
+                    float sf, cf, st, ct, sp, cp;
+                    sincos_fused(a.x, sf, cf);
+                    sincos_fused(a.y, st, ct);
+                    sincos_fused(a.z, sp, cp);
+                    // the velocity turned about x by phi, about y by theta, about z by psi
+                    const float m  = sf * v.y + cf * v.z, be = cf * v.y - sf * v.z;
+                    const float al = ct * v.x + st * m;
+                    float dx = quad_sum(hS * (cp * al - sp * be));
+                    float dy = quad_sum(hS * (sp * al + cp * be));
+                    float dz = quad_sum(hS * (ct * m - st * v.x));
+                    dx = on ? dx : 0.0f, dy = on ? dy : 0.0f, dz = on ? dz : 0.0f;
 #pragma unroll
-                    for(int k = 0; k < 4; ++k)
+                    for(int o = 4; o < LPT; o <<= 1)
                         {
-                            uc[k]         = u[((size_t)t * 4 + k) * n + i];
-                            const float d = uc[k] - ap.u_ref[k];
-                            J += ap.w_effort * d * d;
+                            const float ex = __shfl_up(dx, o, LPT), ey = __shfl_up(dy, o, LPT);
+                            const float ez = __shfl_up(dz, o, LPT);
+                            if(l >= o) dx += ex, dy += ey, dz += ez;
                         }
-                    rk4_step(qd, K, x, uc);
-#pragma unroll
-                    for(int j = 0; j < 12; ++j) ckpt[(((size_t)t + 1) * 12 + j) * n + i] = x[j];
-                    J += ap.w_obstacle * penalty(ap, x, sObs, (int)nObs, 1.0f, nullptr, sub);
+                    const float qx = px + dx, qy = py + dy, qz = pz + dz;  // x_{t+1}
+                    px = __shfl(qx, LPT - 1, LPT), py = __shfl(qy, LPT - 1, LPT), pz = __shfl(qz, LPT - 1, LPT);
+                    // boxes s, s + 4, ... against this lane's step, each read
+                    // while the one before it is worked on
+                    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                    float4 lo = sBox[s], hi = sBox[nBox + s];
+                    for(uint32_t o = s; o < nObs; o += 4)
+                        {
+                            const float4 l1 = sBox[o + 4], h1 = sBox[nBox + o + 4];
+                            box_penalty(lo, hi, qx, qy, qz, ap.margin, itau, ap.tau, ap.w_obstacle, acc);
+                            lo = l1, hi = h1;
+                        }
+                    const float mine = quad_scatter(acc, l);
+                    if(on)
+                        {
+                            J += (s == 0 ? ap.w_obstacle * mine : 0.0f) + ap.w_effort * d * d;
+                            Wg[(size_t)t * 8 + s] = mine;
+                        }
                 }
-            const float ex = x[0] - gx, ey = x[1] - gy, ez = x[2] - gz;
+#pragma unroll
+            for(int o = 1; o < LPT; o <<= 1) J += __shfl_xor(J, o, 64);
+            const float ex = px - gx, ey = py - gy, ez = pz - gz;
             J += ap.w_goal * (ex * ex + ey * ey + ez * ez);
+            if(act && l == 0) cost[(size_t)it * N + i] = J;
             if(REFINE)
                 {
-                    cost[(size_t)it * n + i] = J;
                     if(it == iters) break;
                     b1t *= ap.beta1;
                     b2t *= ap.beta2;
                 }
-            else
-                cost[i] = J;
-            // backward: lam = dJ/dx_t
-            float lam[12];
-#pragma unroll
-            for(int j = 0; j < 12; ++j) lam[j] = 0.0f;
-            lam[0] = 2.0f * ap.w_goal * ex, lam[1] = 2.0f * ap.w_goal * ey, lam[2] = 2.0f * ap.w_goal * ez;
-            if(T >= 1) penalty(ap, x, sObs, (int)nObs, ap.w_obstacle, lam, sub);
-            for(int t = T - 1; t >= 0; --t)
+            __threadfence_block();  // the penalty gradients
+            // 3. backward, the last round first. lam: adjoint j of the chain;
+            // lx, ly, lz, l5: adjoints of the position and of psi at the end
+            // of the round
+            float lam = 0.0f, l5 = 0.0f;
+            float lx = 2.0f * ap.w_goal * ex, ly = 2.0f * ap.w_goal * ey, lz = 2.0f * ap.w_goal * ez;
+            float4 wn, gn;
+            float un = 0.0f, mn = 0.0f, qn = 0.0f;
+            auto fetch3 = [&](int t) {
+                const int tc     = t < 0 ? 0 : t < tl ? t : tl;
+                const float4* w4 = reinterpret_cast<const float4*>(W + (size_t)tc * kStageWords);
+                an = w4[s], vn = w4[4 + s], wn = w4[8 + s];
+                gn = *reinterpret_cast<const float4*>(Wg + (size_t)tc * 8);
+                un = Wg[(size_t)tc * 8 + 4 + s];
+                if(REFINE && it > 0) mn = Wm[(size_t)tc * 8 + s], qn = Wm[(size_t)tc * 8 + 4 + s];
+            };
+            const int last = (Tm - 1) / CH * CH;
+            if(Tm > 0) fetch3(last + tt);
+            for(int t0 = last; t0 >= 0 && Tm > 0; t0 -= CH)
                 {
-                    float xt[12], uc[4], xbar[12], ubar[4];
+                    const int t     = t0 + tt;
+                    const bool on   = t < T;
+                    const float4 a = an, v4 = vn, w = wn, g4 = gn;
+                    const float uc = un;
+                    float mom = mn, vel = qn;
+                    fetch3(t - CH);
+                    float sf, cf, st, ct, sp, cp;
+                    sincos_fused(a.x, sf, cf);
+                    sincos_fused(a.y, st, ct);
+                    sincos_fused(a.z, sp, cp);
+                    // adjoint of x_{t+1}'s position: gradients at x_{t+1} .. x_T
+                    float hx = on ? g4.y : 0.0f, hy = on ? g4.z : 0.0f, hz = on ? g4.w : 0.0f;
 #pragma unroll
-                    for(int j = 0; j < 12; ++j) xt[j] = ckpt[((size_t)t * 12 + j) * n + i];
-#pragma unroll
-                    for(int k = 0; k < 4; ++k) uc[k] = u[((size_t)t * 4 + k) * n + i];
-                    rk4_vjp(qd, K, xt, uc, lam, xbar, ubar);
-#pragma unroll
-                    for(int k = 0; k < 4; ++k)
+                    for(int o = 4; o < LPT; o <<= 1)
                         {
-                            const float gk   = ubar[k] + 2.0f * ap.w_effort * (uc[k] - ap.u_ref[k]);
-                            const size_t idx = ((size_t)t * 4 + k) * n + i;
+                            const float fx = __shfl_down(hx, o, LPT), fy = __shfl_down(hy, o, LPT);
+                            const float fz = __shfl_down(hz, o, LPT);
+                            if(l + o < LPT) hx += fx, hy += fy, hz += fz;
+                        }
+                    hx += lx, hy += ly, hz += lz;
+                    lx = __shfl(hx, 0, LPT), ly = __shfl(hy, 0, LPT), lz = __shfl(hz, 0, LPT);
+                    const float a0 = hS * hx, a1 = hS * hy, a2 = hS * hz;
+                    const float U = v4.x, V = v4.y, Wv = v4.z, p = w.x, q = w.y, r = w.z;
+                    const float R00 = ct * cp, R01 = sf * st * cp - cf * sp, R02 = cf * st * cp + sf * sp;
+                    const float R10 = ct * sp, R11 = sf * st * sp + cf * cp, R12 = cf * st * sp - sf * cp;
+                    const float R21 = sf * ct, R22 = cf * ct;
+                    const float m  = sf * V + cf * Wv, be = cf * V - sf * Wv;
+                    const float al = ct * U + st * m, rt = ct * m - st * U;
+                    // adjoint of psi (the derivative of the world velocity by psi)
+                    const float g5 = (cp * al - sp * be) * a1 - (sp * al + cp * be) * a0;
+                    float h5       = quad_sum(g5);
+                    h5             = on ? h5 : 0.0f;
+#pragma unroll
+                    for(int o = 4; o < LPT; o <<= 1)
+                        {
+                            const float f5 = __shfl_down(h5, o, LPT);
+                            if(l + o < LPT) h5 += f5;
+                        }
+                    const float n5 = __shfl_down(h5, 4, LPT);
+                    const float m5 = l5 + (l + 4 < LPT ? n5 : 0.0f);  // of x_{t+1}
+                    l5 += __shfl(h5, 0, LPT);
+                    const float hG = s == 3 ? 0.0f : s == 2 ? K.h : K.hh;
+                    const float a5 = hS * m5 + hG * dpp<0xF9>(g5);  // quad_perm [1,2,3,3]: the stage after
+                    // the stage's rows
+                    const float ict = recip(ct), tn = st * ict;
+                    const float E = q * sf + r * cf, F = q * cf - r * sf;
+                    const float nv = __builtin_amdgcn_sqrtf(U * U + V * V + Wv * Wv);
+                    const float nw = __builtin_amdgcn_sqrtf(p * p + q * q + r * r);
+                    const float mN = -K.minv * K.nu * nv, kv = nv > 0.0f ? -K.minv * K.nu * recip(nv) : 0.0f;
+                    const float M  = -K.mu * nw, km = nw > 0.0f ? -K.mu * recip(nw) : 0.0f;
+                    const float kU = kv * U, kV = kv * V, kW = kv * Wv, kp = km * p, kq = km * q, kr = km * r;
+                    const float gct = K.g * ct, gst = K.g * st;
+                    const float d0f = R02 * V - R01 * Wv, d1f = R12 * V - R11 * Wv, d2f = R22 * V - R21 * Wv;
+                    const float d0t = cp * rt, d1t = sp * rt, d2t = -al;
+                    float* B        = L.coef + lane * kBlockWords;
+                    auto row = [&](int k, float c, float x3, float x4, float x6, float x7, float x8, float x9,
+                                   float x10, float x11) {
+                        float4* o = reinterpret_cast<float4*>(B + k * kRowWords);
+                        o[0] = make_float4(c, x3, x4, x6);
+                        o[1] = make_float4(x7, x8, x9, x10);
+                        B[k * kRowWords + 8] = x11;
+                    };
+                    row(0, d0f * a0 + d1f * a1 + d2f * a2 + F * ict * a5, F * tn, -E, 0.0f, gct * cf, -gct * sf, 0.0f,
+                        0.0f, 0.0f);
+                    row(1, d0t * a0 + d1t * a1 + d2t * a2 + E * tn * ict * a5, E * ict * ict, 0.0f, -gct, -gst * sf,
+                        -gst * cf, 0.0f, 0.0f, 0.0f);
+                    row(2, R00 * a0 + R10 * a1 - st * a2, 0.0f, 0.0f, mN + kU * U, kU * V - r, kU * Wv + q, 0.0f, 0.0f,
+                        0.0f);
+                    row(3, R01 * a0 + R11 * a1 + R21 * a2, 0.0f, 0.0f, kU * V + r, mN + kV * V, kV * Wv - p, 0.0f, 0.0f,
+                        0.0f);
+                    row(4, R02 * a0 + R12 * a1 + R22 * a2, 0.0f, 0.0f, kU * Wv - q, kV * Wv + p, mN + kW * Wv, 0.0f,
+                        0.0f, 0.0f);
+                    row(5, 0.0f, 1.0f, 0.0f, 0.0f, Wv, -V, K.bx * (M + kp * p), K.ay * r + K.by * kp * q,
+                        K.az * q + K.bz * kp * r);
+                    row(6, sf * ict * a5, sf * tn, cf, -Wv, 0.0f, U, K.ax * r + K.bx * kq * p, K.by * (M + kq * q),
+                        K.az * p + K.bz * kq * r);
+                    row(7, cf * ict * a5, cf * tn, -sf, V, -U, 0.0f, K.ax * q + K.bx * kr * p, K.ay * p + K.by * kr * q,
+                        K.bz * (M + kr * r));
+                    wave_sync();
+                    // the chain over this round's steps
+                    for(int k = (Tm - 1 - t0 < CH - 1 ? Tm - 1 - t0 : CH - 1); k >= 0; --k)
+                        {
+                            const float* B0 = L.coef + (gb + 4 * k) * kBlockWords + j * kRowWords;
+                            auto apply = [&](int stage, float x) {
+                                const float* b   = B0 + stage * kBlockWords;
+                                const float4 c0 = *reinterpret_cast<const float4*>(b);
+                                const float4 c1 = *reinterpret_cast<const float4*>(b + 4);
+                                const float c8  = b[8];
+                                float y         = c0.x;
+                                row_madd(y, x, c0.y, c0.z, c0.w, c1.x, c1.y, c1.z, c1.w, c8);
+                                return y;
+                            };
+                            float x = K.h6 * lam, sum = x;
+                            float y = apply(3, x), xb = lam + y;
+                            x = K.h3 * lam + K.h * y, sum += x;
+                            y = apply(2, x), xb += y;
+                            x = K.h3 * lam + K.hh * y, sum += x;
+                            y = apply(1, x), xb += y;
+                            x = K.h6 * lam + K.hh * y, sum += x;
+                            y = apply(0, x), xb += y;
+                            lam = t0 + k < T ? xb : lam;
+                            // rows 4..7 (a8 .. a11): the adjoints of controls 0..3, unscaled
+                            if(j >= 4) L.ubar[gb + 4 * k + j - 4] = sum;
+                        }
+                    wave_sync();
+                    const float gk = uscale * L.ubar[lane] + 2.0f * ap.w_effort * (uc - uref);
+                    const size_t iu = ((size_t)t * 4 + s) * N + i;
+                    if(on)
+                        {
                             if(REFINE)
                                 {
-                                    const float m = ap.beta1 * mom[idx] + (1.0f - ap.beta1) * gk;
-                                    const float v = ap.beta2 * vel[idx] + (1.0f - ap.beta2) * gk * gk;
-                                    mom[idx]      = m;
-                                    vel[idx]      = v;
-                                    float un      = uc[k] - ap.lr * (m / (1.0f - b1t)) /
-                                                           (__builtin_sqrtf(v / (1.0f - b2t)) + ap.adam_eps);
-                                    if(ap.clamp)
-                                        un = un < c.ctrl_min[k] ? c.ctrl_min[k] : (un > c.ctrl_max[k] ? c.ctrl_max[k] : un);
-                                    u[idx] = un;
+                                    mom = ap.beta1 * mom + (1.0f - ap.beta1) * gk;
+                                    vel = ap.beta2 * vel + (1.0f - ap.beta2) * gk * gk;
+                                    Wm[(size_t)t * 8 + s]     = mom;
+                                    Wm[(size_t)t * 8 + 4 + s] = vel;
+                                    float u1 = uc - ap.lr * (mom / (1.0f - b1t)) /
+                                                      (__builtin_sqrtf(vel / (1.0f - b2t)) + ap.adam_eps);
+                                    if(ap.clamp) u1 = u1 < umin ? umin : (u1 > umax ? umax : u1);
+                                    u[iu]                     = u1;
+                                    Wg[(size_t)t * 8 + 4 + s] = u1;
                                 }
                             else
-                                grad[idx] = gk;
+                                grad[iu] = gk;
                         }
-                    if(t >= 1) penalty(ap, xt, sObs, (int)nObs, ap.w_obstacle, xbar, sub);
-#pragma unroll
-                    for(int j = 0; j < 12; ++j) lam[j] = xbar[j];
+                    wave_sync();  // the next round rewrites the rows
                 }
+            if(REFINE) __threadfence_block();  // the controls, read by other lanes in the next pass
         }
-    if(!REFINE)
-        for(uint32_t t = (uint32_t)T; t < maxT; ++t)
-#pragma unroll
-            for(int k = 0; k < 4; ++k) grad[((size_t)t * 4 + k) * n + i] = 0.0f;
+    if(!REFINE && act)
+        for(uint32_t t = (uint32_t)T + tt; t < maxT; t += CH) grad[((size_t)t * 4 + s) * N + i] = 0.0f;
 }
 
-__global__ void k_pack_boxes(const float* __restrict__ rows, uint32_t n, float4* __restrict__ out)
+// floats of `work` per trajectory
+static size_t rollout_words(bool refine, uint32_t maxT)
 {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if(i >= n) return;
-    const float* r = rows + 6 * (size_t)i;
-    out[2 * i]     = make_float4(r[0], r[1], r[2], 0.0f);
-    out[2 * i + 1] = make_float4(r[3], r[4], r[5], 0.0f);
+    return (size_t)maxT * (kStageWords + 8 + (refine ? 8 : 0));
 }
 
-hipError_t launch_pack_boxes(const float* rows, uint32_t n, float4* out, hipStream_t s)
+// lanes per trajectory: all 64 while the waves fit the chip's SIMDs one each
+// (more lanes share the boxes and the steps of a round; the chains do not get
+// shorter), fewer above
+static uint32_t rollout_lanes(uint32_t n)
 {
-    if(n == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_pack_boxes, dim3((n + 255) / 256), dim3(256), 0, s, rows, n, out);
-    return hipGetLastError();
+    return n <= 1024 ? 64 : n <= 2048 ? 32 : 16;
 }
 
-hipError_t launch_adjoint(bool refine, const QueryDesc* qd, const kgmt_adjoint_params& ap, uint32_t n, uint32_t maxT,
-                          const int32_t* steps, const float* x0, const float* goal, float* u, float* grad, float* ckpt,
-                          float* mom, float* vel, const float4* obs, uint32_t nObs, float* cost, hipStream_t s)
+uint32_t rollout_slab(bool refine, uint32_t n, uint32_t maxT, size_t* floats)
 {
-    if(n == 0) return hipSuccess;
-    const dim3 g((uint32_t)(((uint64_t)n * kLanes + 63) / 64)), b(64);
-    const size_t lds = (size_t)(nObs ? nObs : 1) * 2 * sizeof(float4);
-    if(refine)
-        hipLaunchKernelGGL(k_adjoint<true>, g, b, lds, s, qd, ap, n, maxT, steps, x0, goal, u, grad, ckpt, mom, vel, obs,
-                           nObs, cost);
-    else
-        hipLaunchKernelGGL(k_adjoint<false>, g, b, lds, s, qd, ap, n, maxT, steps, x0, goal, u, grad, ckpt, mom, vel,
-                           obs, nObs, cost);
-    return hipGetLastError();
+    const size_t per = std::max<size_t>(rollout_words(refine, maxT), 1);
+    // trajectories per launch: whole waves, the work space within 1 GiB
+    const size_t most = std::max<size_t>((size_t(1) << 28) / per / 64 * 64, 64);
+    const uint32_t slab = (uint32_t)std::min<size_t>(((size_t)n + 63) / 64 * 64, most);
+    *floats = per * slab;
+    return slab;
+}
+
+template <bool REFINE, int LPT>
+static void launch_rollout_lanes(const RolloutK& K, const kgmt_adjoint_params& ap, uint32_t i0, uint32_t cnt,
+                                 uint32_t n, uint32_t maxT, const int32_t* steps, const float* x0, const float* goal,
+                                 float* u, float* grad, float* work, const float* rows, uint32_t nObs, float* cost,
+                                 hipStream_t s)
+{
+    const dim3 g((cnt + 64 / LPT - 1) / (64 / LPT)), b(64);
+    const size_t lds = (size_t)box_slots(nObs) * 2 * sizeof(float4);
+    hipLaunchKernelGGL((k_rollout<REFINE, LPT>), g, b, lds, s, K, ap, i0, n, maxT, steps, x0, goal, u, grad, work, rows,
+                       nObs, cost);
+}
+
+hipError_t launch_rollout(bool refine, const RolloutK& K, const kgmt_adjoint_params& ap, uint32_t n, uint32_t maxT,
+                          const int32_t* steps, const float* x0, const float* goal, float* u, float* grad, float* work,
+                          uint32_t slab, const float* rows, uint32_t nObs, float* cost, hipStream_t s)
+{
+    for(uint32_t i0 = 0; i0 < n; i0 += std::min(slab, n - i0))
+        {
+            const uint32_t cnt = std::min(slab, n - i0);
+            auto go            = [&](auto kernel) { kernel(K, ap, i0, cnt, n, maxT, steps, x0, goal, u, grad, work, rows, nObs, cost, s); };
+            switch(rollout_lanes(cnt))
+                {
+                    case 64: refine ? go(launch_rollout_lanes<true, 64>) : go(launch_rollout_lanes<false, 64>); break;
+                    case 32: refine ? go(launch_rollout_lanes<true, 32>) : go(launch_rollout_lanes<false, 32>); break;
+                    default: refine ? go(launch_rollout_lanes<true, 16>) : go(launch_rollout_lanes<false, 16>); break;
+                }
+            const hipError_t e = hipGetLastError();
+            if(e != hipSuccess) return e;
+        }
+    return hipSuccess;
 }
 
 }  // namespace kgmt

@@ -1583,24 +1583,20 @@ static int adjoint_common(bool refine, const kgmt_config* cfg, const kgmt_adjoin
     if(!(ap->tau > 0.0f)) return fail(KGMT_E_ARG, "tau must be positive");
     if(refine && ap->iterations > 100000) return fail(KGMT_E_ARG, "too many iterations");
     if(n == 0) return KGMT_OK;
-    StageDesc sd((hipStream_t)stream);
-    int rc = sd.make(cfg);
+    int rc = check_config(cfg);
     if(rc) return rc;
-    const size_t ck = ((size_t)max_steps + 1) * 12 * n, mv = (size_t)max_steps * 4 * n;
-    float *ckpt = nullptr, *mom = nullptr, *vel = nullptr;
-    float4* boxes = nullptr;
-    AsyncBuffers a(sd.s);  // released on every return path
-    if((rc = a.get(ckpt, ck)) || (rc = a.get(boxes, 2 * (size_t)std::max<uint32_t>(n_obs, 1)))) return rc;
-    if(refine)
-        {
-            if((rc = a.get(mom, mv)) || (rc = a.get(vel, mv))) return rc;
-            HIP_TRY(hipMemsetAsync(mom, 0, mv * sizeof(float), sd.s));
-            HIP_TRY(hipMemsetAsync(vel, 0, mv * sizeof(float), sd.s));
-        }
-    hipError_t e = launch_pack_boxes(d_obstacles, n_obs, boxes, sd.s);
-    if(e == hipSuccess)
-        e = launch_adjoint(refine, sd.d, *ap, n, max_steps, d_steps, d_x0, d_goal, d_u, d_grad, ckpt, mom, vel, boxes,
-                           n_obs, d_cost, sd.s);
+    QueryDesc qd;
+    fill_desc(qd, *cfg);
+    RolloutK K{cfg->dt, 0.5f * cfg->dt, cfg->dt / 6.0f, cfg->dt / 3.0f, cfg->gravity, qd.qminv, cfg->quad_nu,
+               cfg->quad_mu, qd.qax, qd.qbx, qd.qay, qd.qby, qd.qaz, qd.qbz, {}, {}};
+    for(int k = 0; k < 4; ++k) K.cmin[k] = cfg->ctrl_min[k], K.cmax[k] = cfg->ctrl_max[k];
+    AsyncBuffers a((hipStream_t)stream);  // released on every return path
+    size_t floats       = 0;
+    const uint32_t slab = rollout_slab(refine, n, max_steps, &floats);
+    float* work         = nullptr;
+    if((rc = a.get(work, floats))) return rc;
+    const hipError_t e = launch_rollout(refine, K, *ap, n, max_steps, d_steps, d_x0, d_goal, d_u, d_grad, work, slab,
+                                        d_obstacles, n_obs, d_cost, a.s);
     if(e != hipSuccess) return fail(KGMT_E_HIP, std::string("adjoint: ") + hipGetErrorString(e));
     return KGMT_OK;
 }

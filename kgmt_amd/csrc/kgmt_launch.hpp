@@ -94,10 +94,20 @@ hipError_t launch_stage_compact(const uint8_t* flags, uint32_t n, uint32_t* out,
 hipError_t launch_stage_repeat(const uint32_t* ids, const uint32_t* counts, uint32_t n, uint32_t* out,
                                uint32_t outCap, uint32_t* total, uint32_t* tmp, hipStream_t s);
 
-// trajectory refinement (kgmt_adjoint.hip)
-hipError_t launch_pack_boxes(const float* rows, uint32_t n, float4* out, hipStream_t s);
-hipError_t launch_adjoint(bool refine, const QueryDesc* qd, const kgmt_adjoint_params& ap, uint32_t n, uint32_t maxT,
-                          const int32_t* steps, const float* x0, const float* goal, float* u, float* grad, float* ckpt,
-                          float* mom, float* vel, const float4* obs, uint32_t nObs, float* cost, hipStream_t s);
+// trajectory refinement (kgmt_adjoint.hip): the quadcopter's constants, and
+// the launches over slabs of trajectories that share one work space
+struct RolloutK
+{
+    float h, hh, h6, h3;
+    float g, minv, nu, mu;
+    float ax, bx, ay, by, az, bz;
+    float cmin[4], cmax[4];
+};
+// trajectories per launch and the floats of work space they take
+uint32_t rollout_slab(bool refine, uint32_t n, uint32_t maxT, size_t* floats);
+// rows: nObs boxes of 6 floats
+hipError_t launch_rollout(bool refine, const RolloutK& K, const kgmt_adjoint_params& ap, uint32_t n, uint32_t maxT,
+                          const int32_t* steps, const float* x0, const float* goal, float* u, float* grad, float* work,
+                          uint32_t slab, const float* rows, uint32_t nObs, float* cost, hipStream_t s);
 
 }  // namespace kgmt
