@@ -31,6 +31,20 @@ constexpr uint32_t kGroupBatch = 4;  // groups tested together (scenes pad to a 
 // float4 pairs: at most 1692 pairs = 54.1 KB (+ 58.5 KB of tile state and
 // candidate lists for a 512-thread propagate tile: 113 KB of gfx950's 160 KB)
 constexpr int32_t kNoGoal   = 0x7fffffff;
+// Box masks of a scene: the workspace cut into kSlabs slabs per axis; row
+// (axis, side, slab) has one bit per box: side 0, the boxes whose low face
+// lies in this slab or a lower one; side 1, those whose high face lies in it
+// or a higher one. Words per row for n boxes: whole 64-bit words, whole
+// 128-bit words past 64 boxes.
+constexpr uint32_t kSlabs = 16;
+__host__ __device__ constexpr uint32_t mask_row(uint32_t n)
+{
+    return n == 0 ? 0u : n <= 64 ? 2u : (n + 127u) / 128u * 4u;
+}
+__host__ __device__ constexpr uint32_t mask_pairs(uint32_t n)  // of a scene's masks, in (lo, hi) float4 pairs
+{
+    return 6u * kSlabs * mask_row(n) / 8u;
+}
 
 // -------------------------------------------------------------------------
 // Per-query descriptor (read-only during a plan) and mutable state.
@@ -50,11 +64,13 @@ struct QueryDesc
     uint32_t obsOff, nObs, nGrp;     // first pair, boxes, groups (multiple of 4) of the scene in the pool
     uint32_t pathOff;                // float offset of the path rows ((max_iter+2)*D)
     float r1size, vol;               // W_R1_SIZE, W_R1_VOL
+    float slabScale;                 // kSlabs / (ws_max - ws_min): slabs of the box masks
     float invSpan, invR1, invP;      // exact 1 / (ws_max - ws_min), 1 / r1size, 1 / P when powers of two, else 0
     float goal[3];
     float start[KGMT_MAX_SAMPLE];
     float qminv, qax, qbx, qay, qby, qaz, qbz;  // quad: 1/m, (Iy-Iz)/Ix, 1/Ix, ...
     uint32_t rowOff;                 // first obstacle row (2 * wdim floats) of the query in the scene's source rows
+    uint32_t masks;                  // the scene has box masks (the query's tiles run the mask check)
     int32_t wdim;                    // workspace dimension W_DIM: 2 (planar: x y, z = 0) or 3
 };
 
@@ -63,6 +79,15 @@ struct QueryDesc
 __host__ __device__ constexpr int row_words(int D)
 {
     return (D + 5) & ~3;
+}
+
+// Whether the rows of a 32-child segment's flagged children lie densely from
+// the segment's start, else each at its child's index: a quadcopter tile
+// finishes its children in no order, and a row of 20 words is most of a
+// cache line anyway.
+__host__ __device__ constexpr bool dense_rows(int model)
+{
+    return model != KGMT_MODEL_QUADCOPTER;
 }
 
 struct QueryState
@@ -154,6 +179,7 @@ struct WorkLists
     uint32_t* jobStart;    // 2 x (nq + 1): update jobs
     uint32_t* active;      // 2: queries not done in each list
     uint32_t* counter;     // arrivals of k_init's workgroups (the last builds the first work lists)
+    uint32_t* tileClaim;   // 2 (by parity): propagate tiles taken past the first of each workgroup
     uint32_t* claim;       // 2 (by parity): update jobs taken in a launch (the launch before zeroes it)
     uint32_t* allDone;     // host-mapped word: 1 once every query is done
     uint32_t* error;       // 1 once an update job's look-back wait ran out (host-mapped for plans)
@@ -162,7 +188,9 @@ struct WorkLists
     HostResult* result;    // host-mapped result of a single-query plan (null: batch, or no early result)
     float* hostPath;       // host-mapped goal -> root rows of that plan ((max_iter + 2) x D floats)
     uint32_t nq;
-    uint32_t tile;         // children per propagate tile (= its workgroup size)
+    uint32_t tile;         // children per propagate tile (= its workgroup size / lanes per child)
+    uint32_t quads;        // 1 when a query is a quadcopter's
+    uint32_t refill;       // children from which a quadcopter query's tiles hold twice as many (0: never)
 
     __device__ __forceinline__ const uint32_t* tiles(uint32_t parity) const { return tileStart + parity * (nq + 1); }
     __device__ __forceinline__ const uint32_t* jobs(uint32_t parity) const { return jobStart + parity * (nq + 1); }
@@ -493,6 +521,110 @@ struct LaneCandCheck
     }
 };
 
+// slab of a coordinate: monotone in v, so a box that meets a segment on an
+// axis has its low face in the slab of the segment's high end or a lower one
+// and its high face in the slab of the low end or a higher one
+__device__ __forceinline__ int slab_of(float v, float wsMin, float scale)
+{
+    // (NaN: fmaxf gives 0)
+    return (int)fminf(fmaxf((v - wsMin) * scale, 0.0f), (float)(kSlabs - 1));
+}
+
+// A scene staged for the mask check: the lo corners of its boxes (whole
+// groups, dummies last), their hi corners, then the masks.
+struct MaskScene
+{
+    const float4* lo;
+    const float4* hi;
+    const uint32_t* mask;
+    int nw;    // words per mask row
+    int nBox;  // boxes, dummies included
+};
+
+// Segment checks of one lane against the boxes its masks leave
+// (collisionCheck.cu:49-62 per step): the boxes whose extent meets the slabs
+// of the segment on every axis, six row reads and their AND for 128 boxes at
+// a time, then those alone by separated(). Every box that the segment meets
+// is among them, so the verdict is the one of testing every box.
+// The slabs of a step's start are those of the last step's end.
+struct MaskWalk
+{
+    int ix, iy, iz;  // slabs of the position
+    __device__ __forceinline__ void start(const QueryDesc& qd, float x, float y, float z)
+    {
+        const float w = qd.cfg.ws_min, c = qd.slabScale;
+        ix = slab_of(x, w, c), iy = slab_of(y, w, c), iz = slab_of(z, w, c);
+    }
+    // whether the segment from (ax, ay, az), the position before, meets a
+    // box; need: lanes whose verdict matters
+    __device__ __forceinline__ bool hit(const QueryDesc& qd, const MaskScene& sc, float ax, float ay, float az,
+                                        float bx, float by, float bz, bool need)
+    {
+        const float w = qd.cfg.ws_min, c = qd.slabScale;
+        const int jx = slab_of(bx, w, c), jy = slab_of(by, w, c), jz = slab_of(bz, w, c);
+        const float mnx = ax > bx ? bx : ax, mxx = ax > bx ? ax : bx;
+        const float mny = ay > by ? by : ay, mxy = ay > by ? ay : by;
+        const float mnz = az > bz ? bz : az, mxz = az > bz ? az : bz;
+        const float sum = (ax + ay + az) + (bx + by + bz);
+        bool found      = false;
+        if(__any(need & (sum != sum)))
+            {
+                // a NaN coordinate has no slab: every box
+                for(int b = 0; b < sc.nBox; ++b) found |= !separated(mnx, mny, mnz, mxx, mxy, mxz, sc.lo[b], sc.hi[b]);
+            }
+        else
+            {
+                const int nw = sc.nw, n = (int)kSlabs * nw;
+                const uint32_t* r0 = sc.mask + max(ix, jx) * nw;
+                const uint32_t* r1 = sc.mask + n + min(ix, jx) * nw;
+                const uint32_t* r2 = sc.mask + 2 * n + max(iy, jy) * nw;
+                const uint32_t* r3 = sc.mask + 3 * n + min(iy, jy) * nw;
+                const uint32_t* r4 = sc.mask + 4 * n + max(iz, jz) * nw;
+                const uint32_t* r5 = sc.mask + 5 * n + min(iz, jz) * nw;
+                auto test = [&](uint64_t m, int b0) {
+                    while(__any(m != 0))
+                        {
+                            const int b = m ? b0 + __ffsll((unsigned long long)m) - 1 : 0;
+                            found |= (m != 0) & !separated(mnx, mny, mnz, mxx, mxy, mxz, sc.lo[b], sc.hi[b]);
+                            m &= m - 1;
+                        }
+                };
+                if(nw == 2)
+                    {
+                        auto two = [](const uint32_t* p) { return *reinterpret_cast<const uint64_t*>(p); };
+                        const uint64_t m = two(r0) & two(r1) & two(r2) & two(r3) & two(r4) & two(r5);
+                        test(need ? m : 0ull, 0);
+                    }
+                else
+                    for(int k = 0; k < nw; k += 4)
+                        {
+                            auto four = [&](const uint32_t* p) { return *reinterpret_cast<const uint4*>(p + k); };
+                            const uint4 a = four(r0), b = four(r1), c4 = four(r2), d = four(r3), e = four(r4), f = four(r5);
+                            const uint32_t m0 = a.x & b.x & c4.x & d.x & e.x & f.x, m1 = a.y & b.y & c4.y & d.y & e.y & f.y;
+                            const uint32_t m2 = a.z & b.z & c4.z & d.z & e.z & f.z, m3 = a.w & b.w & c4.w & d.w & e.w & f.w;
+                            if(!__any(need & ((m0 | m1 | m2 | m3) != 0u))) continue;
+                            test(need ? ((uint64_t)m1 << 32) | m0 : 0ull, 32 * k);
+                            test(need ? ((uint64_t)m3 << 32) | m2 : 0ull, 32 * k + 64);
+                        }
+            }
+        ix = jx, iy = jy, iz = jz;
+        return found;
+    }
+};
+
+// copy a scene's boxes and masks (stored as nGrp group pairs, box pairs,
+// masks at pool + 2 off) into LDS in the layout of MaskScene
+__device__ __forceinline__ MaskScene stage_masks(const float4* __restrict__ pool, uint32_t off, uint32_t nGrp,
+                                                 uint32_t nObs, float4* sObs, bool copy)
+{
+    const uint32_t nBox = nGrp * kGroup, nw = mask_row(nObs), m4 = 6u * kSlabs * nw / 4u;
+    const float4* src   = pool + 2 * ((size_t)off + nGrp);
+    if(copy)
+        for(uint32_t i = threadIdx.x; i < 2 * nBox + m4; i += blockDim.x)
+            sObs[i < 2 * nBox ? (i & 1u) * nBox + (i >> 1) : i] = src[i];
+    return MaskScene{sObs, sObs + nBox, reinterpret_cast<const uint32_t*>(sObs + 2 * nBox), (int)nw, (int)nBox};
+}
+
 // bitwise ORs: every comparison is evaluated (no short-circuit branches)
 __device__ __forceinline__ bool ws_out(const kgmt_config& c, float x, float y, float z)
 {
@@ -731,40 +863,172 @@ __device__ __forceinline__ void quad_ode(const QueryDesc& qd, const float* st, c
     xd[11]          = qd.qaz * p * q + qd.qbz * LMN * r + qd.qbz * uc[3];
 }
 
+// one RK4 step, statePropagator.cu:246-301
+__device__ __forceinline__ void quad_step(const QueryDesc& qd, float* s, const float* uc)
+{
+    const float h = qd.cfg.dt, hh = 0.5f * h, h6 = h / 6.0f;
+    float k1[12], k2[12], k3[12], k4[12], st[12];
+    quad_ode(qd, s, uc, k1);
+#pragma unroll
+    for(int j = 0; j < 12; ++j) st[j] = s[j] + hh * k1[j];
+    quad_ode(qd, st, uc, k2);
+#pragma unroll
+    for(int j = 0; j < 12; ++j) st[j] = s[j] + hh * k2[j];
+    quad_ode(qd, st, uc, k3);
+#pragma unroll
+    for(int j = 0; j < 12; ++j) st[j] = s[j] + h * k3[j];
+    quad_ode(qd, st, uc, k4);
+#pragma unroll
+    for(int j = 0; j < 12; ++j) s[j] = s[j] + h6 * (k1[j] + 2.0f * k2[j] + 2.0f * k3[j] + k4[j]);
+}
+
+// body velocity or workspace bounds left (bitwise: no branches)
+__device__ __forceinline__ bool quad_out(const kgmt_config& c, const float* s)
+{
+    return (s[6] < c.v_min) | (s[6] > c.v_max) | (s[7] < c.v_min) | (s[7] > c.v_max) | (s[8] < c.v_min) |
+           (s[8] > c.v_max) | ws_out(c, s[0], s[1], s[2]);
+}
+
 // statePropagator.cu:246-323
 template <class CHK>
 __device__ __forceinline__ bool prop_quad(const QueryDesc& qd, float* s, const float* uc, int steps, CHK& chk)
 {
-    const kgmt_config& c = qd.cfg;
-    const float h = c.dt, hh = 0.5f * h, h6 = h / 6.0f;
-    bool valid = true;
     for(int i = 0; i < steps; ++i)
         {
             const float px = s[0], py = s[1], pz = s[2];
-            float k1[12], k2[12], k3[12], k4[12], st[12];
-            quad_ode(qd, s, uc, k1);
-#pragma unroll
-            for(int j = 0; j < 12; ++j) st[j] = s[j] + hh * k1[j];
-            quad_ode(qd, st, uc, k2);
-#pragma unroll
-            for(int j = 0; j < 12; ++j) st[j] = s[j] + hh * k2[j];
-            quad_ode(qd, st, uc, k3);
-#pragma unroll
-            for(int j = 0; j < 12; ++j) st[j] = s[j] + h * k3[j];
-            quad_ode(qd, st, uc, k4);
-#pragma unroll
-            for(int j = 0; j < 12; ++j) s[j] = s[j] + h6 * (k1[j] + 2.0f * k2[j] + 2.0f * k3[j] + k4[j]);
+            quad_step(qd, s, uc);
             // body velocity, workspace, segment: each ends the edge, so one branch
             const bool free = chk(px, py, pz, s[0], s[1], s[2]);
-            if((s[6] < c.v_min) | (s[6] > c.v_max) | (s[7] < c.v_min) | (s[7] > c.v_max) | (s[8] < c.v_min) |
-               (s[8] > c.v_max) | ws_out(c, s[0], s[1], s[2]) | !free)
-                {
-                    valid = false;
-                    break;
-                }
+            if(quad_out(qd.cfg, s) | !free) return false;
         }
-    return valid;
+    return true;
 }
+
+// ---------------------------------------------------------------------------
+// One quadcopter by a quad of lanes: lane c (lane 3 as lane 2) holds
+// component c of position, angles, body velocity and rates. A step is the
+// operations of quad_ode and quad_step, each evaluated in the lane whose
+// component it belongs to (the three sin / cos, the two divisions and the two
+// square roots side by side), so the results have the same bits; it takes
+// about half the instructions of one lane's step, for four times the lanes.
+// ---------------------------------------------------------------------------
+template <int CTRL>
+__device__ __forceinline__ float quad_perm(float v)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xF, 0xF, true));
+}
+template <int CTRL>
+__device__ __forceinline__ uint32_t quad_perm(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, 0xF, 0xF, true);
+}
+
+// both values are evaluated (no branch)
+__device__ __forceinline__ float pick(bool b, float x, float y)
+{
+    return b ? x : y;
+}
+
+struct QuadLane
+{
+    float x, a, v, w;      // component of position, angles, velocity, rates
+    float thr, tor;        // thrust and torque terms of the derivative
+    float qa, qb;          // inertia terms of this component
+    int c;                 // component
+
+    // every lane of the quad
+    __device__ __forceinline__ void ode(const QueryDesc& qd, float a_, float v_, float w_, float& dx, float& da,
+                                        float& dv, float& dw) const
+    {
+        constexpr int L0 = 0x00, L1 = 0x55, L2 = 0xAA;    // one lane's value
+        constexpr int NEXT = 0x09, PREV = 0x52;           // components c + 1 and c + 2 of three
+        constexpr int FST = 0x01, SND = 0x5A;             // the two other rates, in the order of the reference
+        const kgmt_config& k = qd.cfg;
+        float sn, cs;
+        sincos_k(a_, sn, cs);
+        const float sph = quad_perm<L0>(sn), cph = quad_perm<L0>(cs);
+        const float sth = quad_perm<L1>(sn), cth = quad_perm<L1>(cs);
+        const float sps = quad_perm<L2>(sn), cps = quad_perm<L2>(cs);
+        const float u = quad_perm<L0>(v_), v = quad_perm<L1>(v_), wv = quad_perm<L2>(v_);
+        const float p = quad_perm<L0>(w_), q = quad_perm<L1>(w_), r = quad_perm<L2>(w_);
+        const float E = q * sph + r * cph;
+        const float F = q * cph - r * sph;
+        const bool c0 = c == 0, c1 = c == 1, c2 = c == 2;
+        const float d = pick(c0, sth, E) / cth;
+        da            = pick(c0, w_ + E * d, pick(c1, F, d));
+        // rows of the rotation: y is x with (cos, sin) of psi turned by 90 degrees
+        const float X = pick(c0, cps, sps), Y = pick(c0, sps, -cps);
+        const float A = pick(c2, -sth, cth * X);
+        const float B = pick(c2, sph * cth, sph * sth * X - cph * Y);
+        const float C = pick(c2, cph * cth, cph * sth * X + sph * Y);
+        dx            = A * u + B * v + C * wv;
+        const float n = __builtin_sqrtf(pick(c0, u * u + v * v + wv * wv, p * p + q * q + r * r));
+        const float XYZ = -k.quad_nu * quad_perm<L0>(n), LMN = -k.quad_mu * quad_perm<L1>(n);
+        const float cr  = quad_perm<PREV>(w_) * quad_perm<NEXT>(v_) - quad_perm<NEXT>(w_) * quad_perm<PREV>(v_);
+        const float g   = k.gravity, gc = g * cth;
+        dv              = cr + pick(c0, -(g * sth), gc * pick(c1, sph, cph)) + qd.qminv * XYZ * v_;
+        dv              = pick(c2, dv + thr, dv);
+        dw              = qa * quad_perm<FST>(w_) * quad_perm<SND>(w_) + qb * LMN * w_ + tor;
+    }
+
+    __device__ __forceinline__ void step(const QueryDesc& qd)
+    {
+        const float h = qd.cfg.dt, hh = 0.5f * h, h6 = h / 6.0f;
+        float x1, a1, v1, w1, x2, a2, v2, w2, x3, a3, v3, w3, x4, a4, v4, w4;
+        ode(qd, a, v, w, x1, a1, v1, w1);
+        ode(qd, a + hh * a1, v + hh * v1, w + hh * w1, x2, a2, v2, w2);
+        ode(qd, a + hh * a2, v + hh * v2, w + hh * w2, x3, a3, v3, w3);
+        ode(qd, a + h * a3, v + h * v3, w + h * w3, x4, a4, v4, w4);
+        x = x + h6 * (x1 + 2.0f * x2 + 2.0f * x3 + x4);
+        a = a + h6 * (a1 + 2.0f * a2 + 2.0f * a3 + a4);
+        v = v + h6 * (v1 + 2.0f * v2 + 2.0f * v3 + v4);
+        w = w + h6 * (w1 + 2.0f * w2 + 2.0f * w3 + w4);
+    }
+
+    // bounds left, or a box met by the segment from position component px;
+    // the same verdict in every lane of the quad. i: slab of px, then of x.
+    __device__ __forceinline__ bool ends(const QueryDesc& qd, const MaskScene& sc, float px, int& i) const
+    {
+        constexpr int L0 = 0x00, L1 = 0x55, L2 = 0xAA;
+        const kgmt_config& k = qd.cfg;
+        auto any3 = [](bool t) {
+            const uint32_t b = t ? 1u : 0u;
+            return (quad_perm<L0>(b) | quad_perm<L1>(b) | quad_perm<L2>(b)) != 0u;
+        };
+        const bool out = any3((v < k.v_min) | (v > k.v_max) | (x < k.ws_min) | (x > k.ws_max));
+        const float mn = px > x ? x : px, mx = px > x ? px : x;
+        const int j = slab_of(x, k.ws_min, qd.slabScale);
+        const float* lo = reinterpret_cast<const float*>(sc.lo) + c;
+        const float* hi = reinterpret_cast<const float*>(sc.hi) + c;
+        bool hit = false;
+        auto test = [&](int b) { return !any3((mx <= lo[4 * b]) | (hi[4 * b] <= mn)); };
+        if(__any(!out & (__builtin_isunordered(px, x))))
+            {
+                for(int b = 0; b < sc.nBox; ++b) hit |= test(b);
+            }
+        else
+            {
+                const int n        = (int)kSlabs * sc.nw;
+                const uint32_t* r0 = sc.mask + 2 * c * n + max(i, j) * sc.nw;
+                const uint32_t* r1 = sc.mask + (2 * c + 1) * n + min(i, j) * sc.nw;
+                for(int w0 = 0; w0 < sc.nw; w0 += 2)
+                    {
+                        const uint32_t a0 = r0[w0] & r1[w0], a1 = r0[w0 + 1] & r1[w0 + 1];
+                        const uint32_t b0 = quad_perm<L0>(a0) & quad_perm<L1>(a0) & quad_perm<L2>(a0);
+                        const uint32_t b1 = quad_perm<L0>(a1) & quad_perm<L1>(a1) & quad_perm<L2>(a1);
+                        uint64_t m        = out ? 0ull : ((uint64_t)b1 << 32) | b0;
+                        while(__any(m != 0))
+                            {
+                                const int b = m ? 32 * w0 + __ffsll((unsigned long long)m) - 1 : 0;
+                                hit |= test(b) & (m != 0);
+                                m &= m - 1;
+                            }
+                    }
+            }
+        i = j;
+        return out | hit;
+    }
+};
 
 template <int MODEL, class CHK>
 __device__ __forceinline__ bool propagate_with(const QueryDesc& qd, float* s, const float* u, int steps, CHK& chk)

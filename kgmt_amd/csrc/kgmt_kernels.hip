@@ -294,10 +294,18 @@ __device__ __forceinline__ void launch_regime(const QueryDesc& qd, uint32_t R, u
     nChildren         = nc > qd.cap ? qd.cap : (uint32_t)nc;
 }
 
+// children per tile of a query: a workgroup's lanes, or twice as many for a
+// quadcopter query whose children fill the chip anyway
+__device__ __forceinline__ uint32_t tile_children(const QueryDesc& qd, const WorkLists& W, uint32_t nC)
+{
+    return W.refill && qd.cfg.model == KGMT_MODEL_QUADCOPTER && nC >= W.refill ? 2u * W.tile : W.tile;
+}
+
 // Work lists of the next iteration into buffer `parity` (block of NT threads,
 // run by the last workgroup to arrive).
 template <int NT>
-__device__ void build_worklists(const QueryState* sts, const WorkLists& W, uint32_t parity, uint32_t* sbuf)
+__device__ void build_worklists(const QueryDesc* __restrict__ qds, const QueryState* sts, const WorkLists& W,
+                                uint32_t parity, uint32_t* sbuf)
 {
     const uint32_t nq = W.nq;
     uint32_t* tileStart = W.tileStart + parity * (nq + 1);
@@ -316,7 +324,8 @@ __device__ void build_worklists(const QueryState* sts, const WorkLists& W, uint3
                                                                   __HIP_MEMORY_SCOPE_AGENT);
                             const uint32_t tr = __hip_atomic_load(&sts[q].treeSizeN, __ATOMIC_RELAXED,
                                                                   __HIP_MEMORY_SCOPE_AGENT);
-                            tiles             = (nc + W.tile - 1) / W.tile;
+                            const uint32_t tc = tile_children(qds[q], W, nc);
+                            tiles             = (nc + tc - 1) / tc;
                             jobs              = (nc + kChunk - 1) / kChunk + (tr + kChunk - 1) / kChunk;
                             alive             = 1;
                         }
@@ -477,6 +486,28 @@ __device__ __forceinline__ uint32_t tab_slot(int32_t* keys, int32_t key)
         }
 }
 
+// row v of flagged children: parent and grandparent bits, sample, zero
+// padding, in whole float4 stores
+template <int S, int C>
+__device__ __forceinline__ void store_row(float* rows, uint32_t v, int32_t p, int32_t gp, const float* s,
+                                          const float* uc, float dur)
+{
+    constexpr int D = S + C + 1, RW = row_words(D);
+    float w[RW];
+    w[0] = __int_as_float(p);
+    w[1] = __int_as_float(gp);
+#pragma unroll
+    for(int d = 0; d < S; ++d) w[2 + d] = s[d];
+#pragma unroll
+    for(int k = 0; k < C; ++k) w[2 + S + k] = uc[k];
+    w[D + 1] = dur;
+#pragma unroll
+    for(int e = D + 2; e < RW; ++e) w[e] = 0.0f;
+    float4* row = reinterpret_cast<float4*>(rows + (size_t)v * RW);
+#pragma unroll
+    for(int j = 0; j < RW / 4; ++j) row[j] = make_float4(w[4 * j], w[4 * j + 1], w[4 * j + 2], w[4 * j + 3]);
+}
+
 // One tile of TC = NT / K children u = base .. base + TC - 1 of a query (TC
 // divides kChunk, so a tile never straddles two chunks), K lanes per child.
 // Every child writes its flag and region; a flagged child (the only ones the
@@ -495,7 +526,7 @@ __device__ __forceinline__ void child_tile(const QueryDesc& qd, const QueryState
                                            const Pools& P, float4* sObs, TileLds<NT, K>& L, uint32_t fb,
                                            bool stage)
 {
-    constexpr int S = ModelDims<MODEL>::S, C = ModelDims<MODEL>::C, D = S + C + 1;
+    constexpr int S = ModelDims<MODEL>::S, C = ModelDims<MODEL>::C;
     constexpr uint32_t TC = NT / K;
     const uint32_t nC  = st.nChildrenN;
     const uint32_t cap = qd.cap;
@@ -683,23 +714,11 @@ __device__ __forceinline__ void child_tile(const QueryDesc& qd, const QueryState
     __syncthreads();
     if(fn)
         {
-            // row slot: segment start + flagged children before it; the row
-            // (parent bits, sample, zero padding) in whole float4 stores
-            constexpr int RW = row_words(D);
-            const uint32_t v = base + (i & ~31u) + (uint32_t)__popc(L.fbits[fb][i >> 5] & ((1u << (i & 31u)) - 1u));
-            float w[RW];
-            w[0] = __int_as_float((int32_t)p);
-            w[1] = __int_as_float(gp);
-#pragma unroll
-            for(int d = 0; d < S; ++d) w[2 + d] = s[d];
-#pragma unroll
-            for(int k = 0; k < C; ++k) w[2 + S + k] = uc[k];
-            w[D + 1] = qd.cfg.dt * (float)steps;
-#pragma unroll
-            for(int e = D + 2; e < RW; ++e) w[e] = 0.0f;
-            float4* row = reinterpret_cast<float4*>(P.childR + qd.rowOffC + (size_t)v * RW);
-#pragma unroll
-            for(int j = 0; j < RW / 4; ++j) row[j] = make_float4(w[4 * j], w[4 * j + 1], w[4 * j + 2], w[4 * j + 3]);
+            // row slot: segment start + flagged children before it
+            const uint32_t v = !dense_rows(MODEL) ? u
+                               : base + (i & ~31u) +
+                                   (uint32_t)__popc(L.fbits[fb][i >> 5] & ((1u << (i & 31u)) - 1u));
+            store_row<S, C>(P.childR + qd.rowOffC, v, (int32_t)p, gp, s, uc, qd.cfg.dt * (float)steps);
         }
     {
         const int32_t rk = L.rkey[t];
@@ -717,6 +736,333 @@ __device__ __forceinline__ void child_tile(const QueryDesc& qd, const QueryState
     __syncthreads();  // L is reused by the next tile
 }
 
+// ---------------------------------------------------------------------------
+// quadcopter tiles, one lane per child
+// ---------------------------------------------------------------------------
+// Most edges of a quadcopter end long before their drawn 10 to 50 steps (out
+// of the workspace, past a speed bound, in a box: 8 to 16 steps on average on
+// the configured queries), and a step is about 1300 instructions, so a wave
+// that runs until its longest edge ends leaves more than half of its lanes
+// idle (2.0 to 2.5 times the steps needed). A tile's lanes are therefore
+// looked over every kQuadSteps steps: with children left, once 64 lanes are
+// free they take new ones; with none left, the lanes still running move out
+// of the last wave as soon as the waves before it have room, and the wave
+// idles (its SIMD goes to other workgroups): 1.3 to 1.6 times the steps needed.
+// The last 64 children take a quad of lanes each: a lone wave's step costs the
+// launch its whole length (160 children: 50 steps). Where each child runs does
+// not change its result. With the mask check in place of the group bounds:
+// three configured quadcopter queries 29.2 -> 19.9 ms a plan, the mixed batch
+// of 512 queries 112 -> 35.7 ms (propagate launches 444 -> 295 and 1154 ->
+// about 340 us); bound by vector issue (63 % of its slots in the single
+// query's launches), then by the length of the longest edge.
+constexpr int kQuadSteps = 4;
+constexpr int kMoveWords = 20;  // a running child: state, controls, frontier uniform, steps left, index and steps, parent
+
+template <int NT>
+struct QuadRunLds
+{
+    float move[kMoveWords][64];
+    uint32_t order[64];        // slots of the last children, most steps left first
+    uint32_t cnt[2][NT / 64];  // running lanes per wave, alternating
+};
+
+// A child of a quadcopter tile
+struct QuadChild
+{
+    float s[12], u[4], uf;  // state (at the start, then at the end of the edge), controls, frontier uniform
+    int left;               // steps left; 0: the edge ended valid; -1: invalid
+    uint32_t meta;          // index in the tile | steps << 10
+    uint32_t p;             // parent
+};
+
+// Runs the children 0 .. count - 1 (at most 1024) of a workgroup of NT threads:
+// take(i, ch) fills a child (state, controls, steps into left), done(ch) takes
+// the finished one; each is called once per child, in any order and lane.
+// Barriers inside, the last before the last calls of done: call uniformly.
+template <int NT, class TAKE, class DONE>
+__device__ __forceinline__ void quad_run(const QueryDesc& qd, uint32_t count, const MaskScene& sc, QuadRunLds<NT>& L,
+                                         TAKE take, DONE done)
+{
+    constexpr int S = 12, C = 4, NW = NT / 64;
+    // children left when a quad of lanes takes each: a quad's step costs half
+    // an instruction more per child than half a wave of single lanes
+    constexpr int kTail = NT / 4 < 64 ? NT / 4 : 64;
+    const int t    = (int)threadIdx.x;
+    const int wave = __builtin_amdgcn_readfirstlane(t / 64);
+    QuadChild ch;
+    bool held = false, run = false;  // a child in this lane; still running
+    MaskWalk walk{0, 0, 0};
+#pragma unroll
+    for(int d = 0; d < S; ++d) ch.s[d] = 0.0f;
+#pragma unroll
+    for(int k = 0; k < C; ++k) ch.u[k] = 0.0f;
+    ch.uf = 0.0f, ch.left = 0, ch.meta = 0u, ch.p = 0u;
+    // the child's words into / out of slot m of L.move
+    auto put = [&](uint32_t m) {
+#pragma unroll
+        for(int d = 0; d < S; ++d) L.move[d][m] = ch.s[d];
+#pragma unroll
+        for(int k = 0; k < C; ++k) L.move[S + k][m] = ch.u[k];
+        L.move[16][m] = ch.uf, L.move[17][m] = __int_as_float(ch.left);
+        L.move[18][m] = __uint_as_float(ch.meta), L.move[19][m] = __uint_as_float(ch.p);
+    };
+    auto get = [&](uint32_t m) {
+#pragma unroll
+        for(int d = 0; d < S; ++d) ch.s[d] = L.move[d][m];
+#pragma unroll
+        for(int k = 0; k < C; ++k) ch.u[k] = L.move[S + k][m];
+        ch.uf = L.move[16][m], ch.left = __float_as_int(L.move[17][m]);
+        ch.meta = __float_as_uint(L.move[18][m]), ch.p = __float_as_uint(L.move[19][m]);
+    };
+    uint32_t next = 0;   // children taken
+    uint32_t rest = 0;   // children left to the quads of lanes
+    int W         = NW;  // waves that may hold running lanes
+    uint32_t par  = 0;
+    while(true)
+        {
+            // running lanes of every wave (the first round's barrier also
+            // covers what the caller staged)
+            const uint64_t mine = __ballot(run);
+            if(lane_id() == 0) L.cnt[par][wave] = (uint32_t)__popcll(mine);
+            __syncthreads();
+            const uint32_t* now = L.cnt[par];
+            uint32_t cw[NW], total = 0;
+#pragma unroll
+            for(int k = 0; k < NW; ++k) cw[k] = now[k], total += cw[k];
+            par ^= 1u;
+            const bool more = next < count;
+            const bool fill = more && (NT - total >= 64u);
+            while(!more && W > 1 && now[W - 1] == 0u) --W;
+            const bool end  = !more && total <= (uint32_t)kTail;
+            const bool drop = !end && !more && W > 1 && total <= 64u * (uint32_t)(W - 1);
+            if(fill || drop || end)
+                {
+                    if(held && !run)
+                        {
+                            held = false;
+                            done(ch);
+                        }
+                    const uint64_t lower = (1ull << lane_id()) - 1ull;
+                    if(end)
+                        {
+                            // the children still running, to the quads below
+                            uint32_t rank = (uint32_t)__popcll(mine & lower);
+#pragma unroll
+                            for(int k = 0; k < NW; ++k) rank += k < wave ? cw[k] : 0u;
+                            if(run) put(rank);
+                            rest = total;
+                            break;
+                        }
+                    // rank among the lanes that take something
+                    uint32_t rank = (uint32_t)__popcll(~mine & lower);
+#pragma unroll
+                    for(int k = 0; k < NW; ++k) rank += k < wave ? 64u - cw[k] : 0u;
+                    if(fill)
+                        {
+                            const uint32_t i = next + rank;
+                            if(!run && i < count)
+                                {
+                                    take(i, ch);
+                                    walk.start(qd, ch.s[0], ch.s[1], ch.s[2]);
+                                    ch.meta = i | (uint32_t)ch.left << 10;
+                                    held    = true;
+                                    run     = ch.left > 0;
+                                }
+                            next = next + (NT - total) < count ? next + (NT - total) : count;
+                        }
+                    else
+                        {
+                            // the last wave's lanes to the free lanes before it
+                            --W;
+                            const uint32_t movers = now[W];
+                            if(wave == W && run)
+                                {
+                                    put((uint32_t)__popcll(mine & lower));
+                                    held = run = false;
+                                }
+                            __syncthreads();
+                            if(wave < W && !run && rank < movers)
+                                {
+                                    get(rank);
+                                    walk.start(qd, ch.s[0], ch.s[1], ch.s[2]);
+                                    held = run = true;
+                                }
+                        }
+                }
+            for(int k = 0; k < kQuadSteps; ++k)
+                {
+                    if(!__any(run)) break;
+                    if(run)
+                        {
+                            const float px = ch.s[0], py = ch.s[1], pz = ch.s[2];
+                            quad_step(qd, ch.s, ch.u);
+                            const bool out = quad_out(qd.cfg, ch.s);
+                            const bool hit = walk.hit(qd, sc, px, py, pz, ch.s[0], ch.s[1], ch.s[2], !out);
+                            ch.left        = (out | hit) ? -1 : ch.left - 1;
+                            run            = ch.left > 0;
+                        }
+                }
+        }
+    if(!rest) return;
+    // the last children, a quad of lanes each, until they end; the longest
+    // first, so that a wave's 16 end together
+    __syncthreads();
+    const uint32_t m = (uint32_t)t / 4u;
+    const int c      = (t & 3) < 3 ? (t & 3) : 2;
+    run              = m < rest;
+    if(run)
+        {
+            // children before child m: more steps left, or as many and a lower slot
+            const int own   = __float_as_int(L.move[17][m]);
+            uint32_t before = 0;
+            for(uint32_t k = (uint32_t)t & 3u; k < rest; k += 4)
+                {
+                    const int o = __float_as_int(L.move[17][k]);
+                    before += o > own || (o == own && k < m) ? 1u : 0u;
+                }
+            before += quad_perm<0xB1>(before);
+            before += quad_perm<0x4E>(before);
+            L.order[before] = m;
+        }
+    __syncthreads();
+    const uint32_t r = run ? L.order[m] : 0u;
+    QuadLane ql;
+    ql.c = c;
+    ql.x = L.move[c][r], ql.a = L.move[3 + c][r], ql.v = L.move[6 + c][r], ql.w = L.move[9 + c][r];
+    ql.qa  = c == 0 ? qd.qax : c == 1 ? qd.qay : qd.qaz;
+    ql.qb  = c == 0 ? qd.qbx : c == 1 ? qd.qby : qd.qbz;
+    ql.thr = qd.qminv * L.move[12][r], ql.tor = ql.qb * L.move[13 + c][r];
+    int left = __float_as_int(L.move[17][r]);
+    int i    = slab_of(ql.x, qd.cfg.ws_min, qd.slabScale);
+    while(__any(run))
+        {
+            if(run)
+                {
+                    const float px = ql.x;
+                    ql.step(qd);
+                    left = ql.ends(qd, sc, px, i) ? -1 : left - 1;
+                    run  = left > 0;
+                }
+        }
+    if(m < rest)
+        {
+            if((t & 3) < 3)
+                L.move[c][r] = ql.x, L.move[3 + c][r] = ql.a, L.move[6 + c][r] = ql.v, L.move[9 + c][r] = ql.w;
+            else
+                L.move[17][r] = __int_as_float(left);
+        }
+    wave_sync();  // a child's words stay within its quad
+    if(m < rest && (t & 3) == 0)
+        {
+            get(r);
+            done(ch);
+        }
+}
+
+template <int NT>
+struct QuadLds
+{
+    static constexpr int kTile = 2 * NT;  // most children of a tile
+    // sums per region and bitset word, as in TileLds
+    int32_t rkey[kTile];
+    uint32_t rtot[kTile], rval[kTile];
+    int32_t wkey[kTile];
+    uint32_t wmask[kTile];
+    QuadRunLds<NT> run;
+};
+
+template <int NT>
+__device__ __forceinline__ void quad_tile(const QueryDesc& qd, const QueryState& st, uint32_t base, uint32_t tile,
+                                          const Pools& P, float4* sObs, QuadLds<NT>& L, bool stage)
+{
+    constexpr int S = 12, C = 4;
+    constexpr int kT   = QuadLds<NT>::kTile;
+    const uint32_t nC  = st.nChildrenN, per = st.perN, itr = st.itrN;
+    const uint32_t cap = qd.cap;
+    const size_t nodeO = qd.nodeOff;
+    const float* T     = P.treeS + qd.sampleOff;
+    for(int k = (int)threadIdx.x; k < kT; k += NT)
+        {
+            L.rkey[k] = -1, L.rtot[k] = 0, L.rval[k] = 0;
+            L.wkey[k] = -1, L.wmask[k] = 0;
+        }
+    const MaskScene sc = stage_masks(P.obs, qd.obsOff, qd.nGrp, qd.nObs, sObs, stage);
+    quad_run<NT>(
+      qd, nC - base < tile ? nC - base : tile, sc, L.run,
+      [&](uint32_t i, QuadChild& ch) {
+          const uint32_t u = base + i;
+          ch.p             = P.repIdx[nodeO + u / per];
+          draw_child<C>(qd.cfg, qd.cfg.query_id, itr, u, ch.u, ch.left, ch.uf);
+#pragma unroll
+          for(int d = 0; d < S; ++d) ch.s[d] = T[(size_t)d * cap + ch.p];
+      },
+      [&](const QuadChild& ch) {
+          const uint32_t u = base + (ch.meta & 1023u);
+          const bool ok    = ch.left == 0;
+          bool fn = false, setBit = false;
+          uint32_t r2bit = 0;
+          int ix, iy, iz;
+          const int r1 = region_of(qd, ch.s[0], ch.s[1], ch.s[2], ix, iy, iz);
+          if(ok)
+              {
+                  const int r2    = subregion_of(qd, ch.s[0], ch.s[1], ch.s[2], r1, ix, iy, iz);
+                  const bool seen = test_bit(P.actPrev + qd.subOff, (uint32_t)r2);
+                  fn              = (ch.uf < P.score[qd.regOff + r1]) || !seen;
+                  setBit          = !seen;
+                  r2bit           = (uint32_t)r2;
+              }
+          if(u % per == 0) P.frontier[nodeO + ch.p] = 0;
+          P.r1child[nodeO + u] = r1;
+          P.fnext[nodeO + u]   = fn ? 1 : 0;
+          const uint32_t e     = tab_slot<kT>(L.rkey, r1);
+          atomicAdd(&L.rtot[e], 1u);
+          if(ok) atomicAdd(&L.rval[e], 1u);
+          if(setBit)
+              {
+                  const uint32_t f = tab_slot<kT>(L.wkey, (int32_t)(r2bit >> 5));
+                  atomicOr(&L.wmask[f], 1u << (r2bit & 31u));
+              }
+          // the tile lies inside one 1024-element chunk
+          const uint64_t fm = __ballot(fn);
+          if(fn)
+              {
+                  if((int)lane_id() == __ffsll((unsigned long long)fm) - 1)
+                      atomicAdd(&P.partA[qd.chunkOff + base / kChunk], (uint32_t)__popcll(fm));
+                  store_row<S, C>(P.childR + qd.rowOffC, u, (int32_t)ch.p, P.parent[nodeO + ch.p], ch.s, ch.u,
+                                  qd.cfg.dt * (float)(ch.meta >> 10));
+              }
+      });
+    __syncthreads();
+    for(int k = (int)threadIdx.x; k < kT; k += NT)
+        {
+            const int32_t rk = L.rkey[k];
+            if(rk >= 0)
+                {
+                    atomicAdd(&P.total[qd.regOff + rk], (int32_t)L.rtot[k]);
+                    if(L.rval[k]) atomicAdd(&P.validc[qd.regOff + rk], (int32_t)L.rval[k]);
+                }
+            const int32_t wk = L.wkey[k];
+            if(wk >= 0) atomicOr(&P.actNext[qd.subOff + (uint32_t)wk], L.wmask[k]);
+        }
+}
+
+// LDS of a propagate workgroup: its model's tile state
+template <int MODEL, int NT, int K>
+union PropagateLds
+{
+    TileLds<NT, K> tile;
+    QuadLds<NT> quad;
+};
+template <int NT>
+union PropagateLds<KGMT_MODEL_QUADCOPTER, NT, 1>
+{
+    QuadLds<NT> quad;
+};
+template <int MODEL, int NT, int K>
+constexpr bool kUseTile = !(MODEL == KGMT_MODEL_QUADCOPTER && K == 1);
+template <int MODEL, int NT, int K>
+constexpr bool kUseQuad = (MODEL == KGMT_MODEL_QUADCOPTER || MODEL < 0) && K == 1;
+
 template <int MODEL, int NT, int K>
 __global__ __launch_bounds__(NT, 4) void k_propagate(const QueryDesc* __restrict__ qds,
                                                   QueryState* __restrict__ sts, Pools P, WorkLists W,
@@ -724,7 +1070,7 @@ __global__ __launch_bounds__(NT, 4) void k_propagate(const QueryDesc* __restrict
 {
     static_assert(NT % 64 == 0 && kChunk % (NT / K) == 0, "tile size");
     extern __shared__ float4 sObs[];
-    __shared__ TileLds<NT, K> L;
+    __shared__ PropagateLds<MODEL, NT, K> L;
     const uint32_t nq        = W.nq;
     // the first workgroup commits the next-state fields (written when the
     // last iteration closed) to the current ones, which the update kernel
@@ -737,40 +1083,73 @@ __global__ __launch_bounds__(NT, 4) void k_propagate(const QueryDesc* __restrict
     uint32_t fb              = 0;  // flag buffer of the next tile
     // the tables and both flag buffers start empty (each tile empties them
     // again after its flush; the first tile's staging barrier comes before
-    // any insert)
-    clear_tables(L, 0u);
-    clear_tables(L, 1u);
-    for(uint32_t t = blockIdx.x; t < nTiles; t += gridDim.x)
+    // any insert); used: by a quadcopter tile's state since
+    bool used = false;
+    if constexpr(kUseTile<MODEL, NT, K>) clear_tables(L.tile, 0u), clear_tables(L.tile, 1u);
+    // Workgroup j takes tile j, then, with more tiles than workgroups, every
+    // gridDim.x-th tile; where quadcopter tiles are among them (they differ
+    // several times in length), the next from a counter instead, fetched while
+    // a tile runs (the mixed batch: 45.6 to 41.0 ms a plan; the other models'
+    // tiles are short and even, and the fetch at their start cost them 2 to
+    // 4 %). The other parity's counter starts at zero for the next launch.
+    constexpr bool claim = kUseQuad<MODEL, NT, K>;
+    __shared__ uint32_t sNext[2];
+    if(claim && blockIdx.x == 0 && threadIdx.x == 0) W.tileClaim[parity ^ 1u] = 0u;
+    uint32_t turn = 0;
+    for(uint32_t t = blockIdx.x; t < nTiles; t = claim ? sNext[turn] : t + gridDim.x, turn ^= 1u)
         {
+            if(claim && threadIdx.x == 0)
+                sNext[turn] = nTiles > gridDim.x ? gridDim.x + __hip_atomic_fetch_add(W.tileClaim + parity, 1u,
+                                                                                      __ATOMIC_RELAXED,
+                                                                                      __HIP_MEMORY_SCOPE_AGENT)
+                                                 : nTiles;
             const uint32_t q    = locate(tileList, nq, t);
-            if(sts[q].doneN) continue;  // stale list entry of a finished query
+            if(sts[q].doneN)
+                {
+                    if(claim) __syncthreads();
+                    continue;  // stale list entry of a finished query
+                }
             const QueryDesc& qd = qds[q];
             // a new query's scene: the tile stages it (after the barrier
             // that ends the last tile, so no wave still reads the old one)
             const bool stage = q != staged;
             staged           = q;
-            const uint32_t base = (t - tileList[q]) * (NT / K);
-            if constexpr(MODEL >= 0)
-                child_tile<MODEL, NT, K>(qd, sts[q], base, P, sObs, L, fb, stage);
-            else
+            const int model  = MODEL >= 0 ? MODEL : qd.cfg.model;
+            if constexpr(kUseQuad<MODEL, NT, K>)
+                if(model == KGMT_MODEL_QUADCOPTER)
+                    {
+                        const uint32_t tile = tile_children(qd, W, sts[q].nChildrenN);
+                        quad_tile<NT>(qd, sts[q], (t - tileList[q]) * tile, tile, P, sObs, L.quad, stage);
+                        used = true;
+                        continue;
+                    }
+            if constexpr(kUseTile<MODEL, NT, K>)
                 {
-                    switch(qd.cfg.model)
+                    if(used)
                         {
-                            case KGMT_MODEL_DOUBLE_INTEGRATOR:
-                                child_tile<KGMT_MODEL_DOUBLE_INTEGRATOR, NT, K>(qd, sts[q], base, P, sObs, L, fb, stage);
-                                break;
-                            case KGMT_MODEL_DUBINS_AIRPLANE:
-                                child_tile<KGMT_MODEL_DUBINS_AIRPLANE, NT, K>(qd, sts[q], base, P, sObs, L, fb, stage);
-                                break;
-                            case KGMT_MODEL_DUBINS_5D:
-                                child_tile<KGMT_MODEL_DUBINS_5D, NT, K>(qd, sts[q], base, P, sObs, L, fb, stage);
-                                break;
+                            __syncthreads();
+                            clear_tables(L.tile, 0u), clear_tables(L.tile, 1u);
+                            __syncthreads();
+                            used = false;
+                        }
+                    const uint32_t base = (t - tileList[q]) * (NT / K);
+                    if constexpr(MODEL >= 0)
+                        child_tile<MODEL, NT, K>(qd, sts[q], base, P, sObs, L.tile, fb, stage);
+                    else
+                        {
                             // (a batch never mixes planar and 3D queries, so
                             // a mixed batch holds no unicycle)
-                            default: child_tile<KGMT_MODEL_QUADCOPTER, NT, K>(qd, sts[q], base, P, sObs, L, fb, stage); break;
+                            if(model == KGMT_MODEL_DOUBLE_INTEGRATOR)
+                                child_tile<KGMT_MODEL_DOUBLE_INTEGRATOR, NT, K>(qd, sts[q], base, P, sObs, L.tile, fb, stage);
+                            else if(model == KGMT_MODEL_DUBINS_AIRPLANE)
+                                child_tile<KGMT_MODEL_DUBINS_AIRPLANE, NT, K>(qd, sts[q], base, P, sObs, L.tile, fb, stage);
+                            else if(model == KGMT_MODEL_DUBINS_5D)
+                                child_tile<KGMT_MODEL_DUBINS_5D, NT, K>(qd, sts[q], base, P, sObs, L.tile, fb, stage);
+                            else if constexpr(!kUseQuad<MODEL, NT, K>)
+                                child_tile<KGMT_MODEL_QUADCOPTER, NT, K>(qd, sts[q], base, P, sObs, L.tile, fb, stage);
                         }
+                    fb ^= 1u;
                 }
-            fb ^= 1u;
         }
 }
 
@@ -824,14 +1203,17 @@ __device__ __forceinline__ void count_closed(const WorkLists& W)
 
 // Work lists of a single-query table for its next iteration (parity
 // buffer), from the next-state fields (one thread).
-__device__ __forceinline__ void single_worklists(const QueryState& st, const WorkLists& W, uint32_t parity)
+template <bool QUADS>
+__device__ __forceinline__ void single_worklists(const QueryDesc& qd, const QueryState& st, const WorkLists& W,
+                                                 uint32_t parity)
 {
     uint32_t* tileStart = W.tileStart + parity * 2;
     uint32_t* jobStart  = W.jobStart + parity * 2;
     const bool alive    = st.doneN == 0;
     tileStart[0]        = 0;
     jobStart[0]         = 0;
-    tileStart[1]        = alive ? (st.nChildrenN + W.tile - 1) / W.tile : 0u;
+    const uint32_t tc   = QUADS ? tile_children(qd, W, st.nChildrenN) : W.tile;
+    tileStart[1]        = alive ? (st.nChildrenN + tc - 1) / tc : 0u;
     jobStart[1] = alive ? (st.nChildrenN + kChunk - 1) / kChunk + (st.treeSizeN + kChunk - 1) / kChunk : 0u;
     W.active[parity] = alive ? 1u : 0u;
 }
@@ -1280,6 +1662,7 @@ __device__ __forceinline__ void react_job(const QueryDesc& qd, const QueryState&
 // (KGMT.cu:336-339); goal: this thread's smallest appended index within
 // goal_thresh (kLbNone if none). pAll / pBefore: this thread's share of the
 // chunk counts of all chunks / of the chunks before c.
+template <bool QUADS>
 __device__ __forceinline__ void append_job(const QueryDesc& qd, const QueryState& st, uint32_t c, const Pools& P,
                                            uint32_t pAll, uint32_t pBefore, uint32_t* sbuf, uint32_t (&node)[kPer],
                                            uint32_t (&rep)[kPer], uint32_t& goal, uint32_t& nAcc, int32_t& apar)
@@ -1310,7 +1693,8 @@ __device__ __forceinline__ void append_job(const QueryDesc& qd, const QueryState
     // the flagged children before it in the segment (the 32 threads of half
     // a wave).
     const uint32_t nf = (uint32_t)__popc(fl);
-    uint32_t slot     = (u0 & ~31u) + half_incl_scan(nf) - nf;
+    uint32_t slot     = half_incl_scan(nf) - nf;
+    slot              = QUADS && !dense_rows(qd.cfg.model) ? u0 : (u0 & ~31u) + slot;
 #pragma unroll
     for(uint32_t k = 0; k < kPer; ++k)
         if((fl >> k) & 1u)
@@ -1368,6 +1752,7 @@ __device__ __forceinline__ void append_job(const QueryDesc& qd, const QueryState
 // One job of query q (li: its index among the query's jobs). own: the
 // scores come from the region counts (the planner); otherwise from P.score
 // (the stage entry, which is given them).
+template <bool QUADS>
 __device__ void update_job(const QueryDesc* __restrict__ qds, QueryState* __restrict__ sts, const Pools& P,
                            const WorkLists& W, uint32_t parity, uint32_t q, uint32_t li, bool own, UpdateLds& L)
 {
@@ -1429,7 +1814,7 @@ __device__ void update_job(const QueryDesc* __restrict__ qds, QueryState* __rest
             react_job(qd, st, li, P, fw, rr, u, own, L.raw, L.sum, faccept(qd, st.itr, tree, next), node, rep);
         }
     else
-        append_job(qd, st, c, P, pAll, pBefore, L.sbuf, node, rep, goal, nAcc, apar);
+        append_job<QUADS>(qd, st, c, P, pAll, pBefore, L.sbuf, node, rep, goal, nAcc, apar);
     uint32_t total, jobGoal;
     const uint32_t ex = block_excl_scan_min<kUpd>(rep[0], goal, L.sbuf, total, jobGoal);
     if(threadIdx.x == 0)
@@ -1556,7 +1941,7 @@ __device__ void update_job(const QueryDesc* __restrict__ qds, QueryState* __rest
                     if(nq == 1)
                         {
                             finish_query(qd, st, R);
-                            single_worklists(st, W, parity ^ 1u);
+                            single_worklists<QUADS>(qd, st, W, parity ^ 1u);
                             count_closed(W);
                             if(st.doneN && !st.successN)
                                 {
@@ -1568,6 +1953,8 @@ __device__ void update_job(const QueryDesc* __restrict__ qds, QueryState* __rest
         }
 }
 
+// QUADS: some query is a quadcopter's
+template <bool QUADS>
 __global__ __launch_bounds__(kUpd) void k_update(const QueryDesc* __restrict__ qds, QueryState* __restrict__ sts,
                                                    Pools P, WorkLists W, uint32_t parity, uint32_t own)
 {
@@ -1599,7 +1986,7 @@ __global__ __launch_bounds__(kUpd) void k_update(const QueryDesc* __restrict__ q
                 }
             const uint32_t q = nq > 1 ? locate(jobList, nq, j) : 0u;
             // (a stale list entry of a finished query has nothing to do)
-            if(!sts[q].done) update_job(qds, sts, P, W, parity, q, nq > 1 ? j - jobList[q] : j, own != 0, L);
+            if(!sts[q].done) update_job<QUADS>(qds, sts, P, W, parity, q, nq > 1 ? j - jobList[q] : j, own != 0, L);
             if(!more) return;
             __syncthreads();  // L is rewritten by the next job
         }
@@ -1616,7 +2003,7 @@ __global__ __launch_bounds__(kBlock) void k_finish(const QueryDesc* __restrict__
     for(uint32_t q = threadIdx.x; q < W.nq; q += kBlock)
         if(!sts[q].done) finish_query(qds[q], sts[q], sts[q].R);
     __syncthreads();
-    build_worklists<kBlock>(sts, W, parity ^ 1u, sbuf);
+    build_worklists<kBlock>(qds, sts, W, parity ^ 1u, sbuf);
     if(threadIdx.x == 0) count_closed(W);
 }
 
@@ -1724,9 +2111,12 @@ __device__ __forceinline__ float row_face(const float* __restrict__ rows, uint32
         return k == 2 ? -1.0f : k == 5 ? 1.0f : rows[4 * (size_t)i + (k < 3 ? k : k - 1)];
 }
 
-template <int W>
-__device__ void build_scene_wg(const float* __restrict__ rows, uint32_t n, uint32_t nGrp, float4* __restrict__ out,
-                               SceneLds& L)
+// mask (null: none): the box masks too, for a workspace from wsMin with
+// slabScale slabs per unit.
+template <int W, bool MASKS = false>
+__device__ __forceinline__ void build_scene_wg(const float* __restrict__ rows, uint32_t n, uint32_t nGrp, float4* __restrict__ out,
+                               SceneLds& L, uint32_t* __restrict__ mask = nullptr, float wsMin = 0.0f,
+                               float slabScale = 0.0f)
 {
     // bounds of the finite centres
     float lo[3] = {INFINITY, INFINITY, INFINITY}, hi[3] = {-INFINITY, -INFINITY, -INFINITY};
@@ -1815,6 +2205,48 @@ __device__ void build_scene_wg(const float* __restrict__ rows, uint32_t n, uint3
             out[2 * g]     = make_float4(gl[0], gl[1], gl[2], 0.0f);
             out[2 * g + 1] = make_float4(gh[0], gh[1], gh[2], 0.0f);
         }
+    if(!MASKS || !mask) return;
+    // 64 boxes per wave and round: the ballot of "low face in slab g or
+    // lower" is their two words of row (axis, 0, g), "high face in slab g or
+    // higher" of row (axis, 1, g); a NaN face belongs to every row of its side
+    const uint32_t nw = mask_row(n), lane = lane_id();
+    for(uint32_t wp = threadIdx.x / 64; wp < nw / 2; wp += kBlock / 64)
+        {
+            const uint32_t k = 64 * wp + lane;
+            for(int d = 0; d < 3; ++d)
+                {
+                    int lo = (int)kSlabs, hi = -1;
+                    if(k < n)
+                        {
+                            const float h = L.box[k][3 + d];
+                            lo            = slab_of(L.box[k][d], wsMin, slabScale);  // NaN: 0
+                            hi            = h == h ? slab_of(h, wsMin, slabScale) : (int)kSlabs - 1;
+                        }
+                    uint64_t keep = 0;
+#pragma unroll
+                    for(int g = 0; g < (int)kSlabs; ++g)
+                        {
+                            const uint64_t a = __ballot(lo <= g), b = __ballot(hi >= g);
+                            keep             = (int)lane == g ? a : (int)lane == (int)kSlabs + g ? b : keep;
+                        }
+                    if(lane < 2 * kSlabs)
+                        *reinterpret_cast<uint64_t*>(mask + (size_t)(2 * kSlabs * d + lane) * nw + 2 * wp) = keep;
+                }
+        }
+}
+
+// a query's scene from its rows, with its masks where MASKS and it has them
+template <bool MASKS>
+__device__ __forceinline__ void build_query_scene(const QueryDesc& qd, const float* __restrict__ rows, const Pools& P, SceneLds& L)
+{
+    float4* out    = P.obs + 2 * (size_t)qd.obsOff;
+    uint32_t* mask = MASKS && qd.masks ? reinterpret_cast<uint32_t*>(out + 2 * (size_t)qd.nGrp * (1 + kGroup)) : nullptr;
+    if(qd.wdim == 2)
+        build_scene_wg<2, MASKS>(rows + 4 * (size_t)qd.rowOff, qd.nObs, qd.nGrp, out, L, mask, qd.cfg.ws_min,
+                                 qd.slabScale);
+    else
+        build_scene_wg<3, MASKS>(rows + 6 * (size_t)qd.rowOff, qd.nObs, qd.nGrp, out, L, mask, qd.cfg.ws_min,
+                                 qd.slabScale);
 }
 
 // ---------------------------------------------------------------------------
@@ -1831,24 +2263,19 @@ __global__ __launch_bounds__(kBlock) void k_init(const QueryDesc* __restrict__ q
     __shared__ uint32_t sflag;
     const uint32_t q    = blockIdx.x;
     const QueryDesc& qd = qds[q];
-    if(rows && qd.nObs)
-        {
-            if(qd.wdim == 2)
-                build_scene_wg<2>(rows + 4 * (size_t)qd.rowOff, qd.nObs, qd.nGrp, P.obs + 2 * (size_t)qd.obsOff, L);
-            else
-                build_scene_wg<3>(rows + 6 * (size_t)qd.rowOff, qd.nObs, qd.nGrp, P.obs + 2 * (size_t)qd.obsOff, L);
-        }
+    if(rows && qd.nObs) build_query_scene<true>(qd, rows, P, L);
     clear_query(qd, P, threadIdx.x, kBlock);
     root_query(qd, sts[q], P);
-    if(q == 0 && threadIdx.x < 2) W.claim[threadIdx.x] = 0u;
+    if(q == 0 && threadIdx.x < 2) W.claim[threadIdx.x] = W.tileClaim[threadIdx.x] = 0u;
     if(q == 0 && threadIdx.x == 0) *W.closedDev = 0u;
-    if(last_arrival(W.counter, nq, &sflag)) build_worklists<kBlock>(sts, W, 0, sbuf);
+    if(last_arrival(W.counter, nq, &sflag)) build_worklists<kBlock>(qds, sts, W, 0, sbuf);
 }
 
 // k_init of a single query, its descriptor a kernel argument that the first
 // thread stores for the kernels after it (no upload before the launch):
 // workgroup 0 builds the scene, the root, the state and the first work
 // lists (no hand-off between workgroups), workgroups 1.. clear the counters
+template <bool MASKS>
 __global__ __launch_bounds__(kBlock) void k_init_one(const QueryDesc qd, QueryDesc* __restrict__ dq,
                                                      QueryState* __restrict__ sts, Pools P, WorkLists W,
                                                      const float* __restrict__ rows)
@@ -1860,20 +2287,14 @@ __global__ __launch_bounds__(kBlock) void k_init_one(const QueryDesc qd, QueryDe
             return;
         }
     if(threadIdx.x == 0) *dq = qd;
-    if(rows && qd.nObs)
-        {
-            if(qd.wdim == 2)
-                build_scene_wg<2>(rows + 4 * (size_t)qd.rowOff, qd.nObs, qd.nGrp, P.obs + 2 * (size_t)qd.obsOff, L);
-            else
-                build_scene_wg<3>(rows + 6 * (size_t)qd.rowOff, qd.nObs, qd.nGrp, P.obs + 2 * (size_t)qd.obsOff, L);
-        }
+    if(rows && qd.nObs) build_query_scene<MASKS>(qd, rows, P, L);
     root_query(qd, sts[0], P);
-    if(threadIdx.x < 2) W.claim[threadIdx.x] = 0u;
+    if(threadIdx.x < 2) W.claim[threadIdx.x] = W.tileClaim[threadIdx.x] = 0u;
     // the first thread wrote the state: it builds the first work lists
     if(threadIdx.x == 0)
         {
             *W.closedDev = 0u;
-            single_worklists(sts[0], W, 0u);
+            single_worklists<MASKS>(qd, sts[0], W, 0u);
         }
 }
 
@@ -2049,7 +2470,7 @@ __global__ __launch_bounds__(kBlock) void k_stage_fu_nodes(const QueryDesc* __re
     P.fnext[i]   = f ? 1 : 0;
     P.r1child[i] = region_of(qd, child[i], child[(size_t)nC + i], child[2 * (size_t)nC + i], ix, iy, iz);
     if(!f) return;
-    const uint32_t s0 = i & ~31u;
+    const uint32_t s0 = dense_rows(qd.cfg.model) ? i & ~31u : i;
     uint32_t before   = 0;
     for(uint32_t k = s0; k < i; ++k) before += fnext[k] ? 1u : 0u;
     const int32_t p  = childParent[i];
@@ -2255,7 +2676,10 @@ hipError_t launch_init_one(const QueryDesc& qd, QueryDesc* dq, QueryState* sts, 
     // about 4 K words to clear per clearing workgroup
     const uint32_t words = 3u * (uint32_t)qd.R1 + 2u * (uint32_t)qd.R2words + 9u * (qd.nChunks + 1u);
     const uint32_t clear = std::min(32u, std::max(1u, (words + 4095u) / 4096u));
-    hipLaunchKernelGGL(k_init_one, dim3(1 + clear), dim3(kBlock), 0, s, qd, dq, sts, P, W, rows);
+    if(qd.masks)
+        hipLaunchKernelGGL(k_init_one<true>, dim3(1 + clear), dim3(kBlock), 0, s, qd, dq, sts, P, W, rows);
+    else
+        hipLaunchKernelGGL(k_init_one<false>, dim3(1 + clear), dim3(kBlock), 0, s, qd, dq, sts, P, W, rows);
     return hipGetLastError();
 }
 
@@ -2313,7 +2737,11 @@ hipError_t launch_propagate(int model, const QueryDesc* qds, QueryState* sts, co
 hipError_t launch_update(const QueryDesc* qds, QueryState* sts, const Pools& P, const WorkLists& W,
                          uint32_t parity, const Launch& L, bool own, hipStream_t s)
 {
-    hipLaunchKernelGGL(k_update, dim3(L.chunkGrid), dim3(kUpd), 0, s, qds, sts, P, W, parity, own ? 1u : 0u);
+    const dim3 g(L.chunkGrid), b(kUpd);
+    if(W.quads)
+        hipLaunchKernelGGL(k_update<true>, g, b, 0, s, qds, sts, P, W, parity, own ? 1u : 0u);
+    else
+        hipLaunchKernelGGL(k_update<false>, g, b, 0, s, qds, sts, P, W, parity, own ? 1u : 0u);
     return hipGetLastError();
 }
 
