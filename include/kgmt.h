@@ -336,11 +336,9 @@ int kgmt_propagate_collide(const kgmt_config* cfg, const int32_t* d_parent_idx,
 /* kgmt_propagate_collide without any device allocation: no counterpart in
  * the reference; for callers that cannot allocate (code under HIP graph
  * capture, serving loops, harnesses that forbid hipMalloc). Same arguments,
- * outputs and bits as kgmt_propagate_collide; the obstacle scene goes into a
- * library-held device array of one scene of at most 1500 boxes per GPU
- * (54 KB, kept until the process ends), and n_obs > 1500 is rejected with
- * KGMT_E_CAPACITY. Calls on one GPU share that array: calls that overlap on
- * one GPU race. Asynchronous on `stream`. */
+ * outputs and bits as kgmt_propagate_collide, which allocates nothing either;
+ * n_obs > 1500 is rejected with KGMT_E_CAPACITY. Calls may overlap.
+ * Asynchronous on `stream`. */
 int kgmt_propagate_collide_noalloc(const kgmt_config* cfg, const int32_t* d_parent_idx,
                                    const float* d_parent_states, uint32_t n_parents,
                                    const float* d_controls, const int32_t* d_steps, uint32_t n_children,

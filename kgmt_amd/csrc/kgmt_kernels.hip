@@ -2093,6 +2093,40 @@ __device__ __forceinline__ uint32_t morton10(uint32_t x, uint32_t y, uint32_t z)
     return code;
 }
 
+// The masks of n boxes (device.hpp, kSlabs) by a workgroup of kBlock threads;
+// face(k, d): face d (0..2 low, 3..5 high) of box k. 64 boxes per wave and
+// round: the ballot of "low face in slab g or lower" is their two words of row
+// (axis, 0, g), "high face in slab g or higher" of row (axis, 1, g); a NaN
+// face belongs to every row of its side.
+template <class FACE>
+__device__ __forceinline__ void box_masks(uint32_t n, float wsMin, float slabScale, uint32_t* mask, FACE face)
+{
+    const uint32_t nw = mask_row(n), lane = lane_id();
+    for(uint32_t wp = threadIdx.x / 64; wp < nw / 2; wp += kBlock / 64)
+        {
+            const uint32_t k = 64 * wp + lane;
+            for(int d = 0; d < 3; ++d)
+                {
+                    int lo = (int)kSlabs, hi = -1;
+                    if(k < n)
+                        {
+                            const float h = face(k, 3 + d);
+                            lo            = slab_of(face(k, d), wsMin, slabScale);  // NaN: 0
+                            hi            = h == h ? slab_of(h, wsMin, slabScale) : (int)kSlabs - 1;
+                        }
+                    uint64_t keep = 0;
+#pragma unroll
+                    for(int g = 0; g < (int)kSlabs; ++g)
+                        {
+                            const uint64_t a = __ballot(lo <= g), b = __ballot(hi >= g);
+                            keep             = (int)lane == g ? a : (int)lane == (int)kSlabs + g ? b : keep;
+                        }
+                    if(lane < 2 * kSlabs)
+                        *reinterpret_cast<uint64_t*>(mask + (size_t)(2 * kSlabs * d + lane) * nw + 2 * wp) = keep;
+                }
+        }
+}
+
 struct SceneLds
 {
     float box[kMaxObs][6];
@@ -2206,33 +2240,7 @@ __device__ __forceinline__ void build_scene_wg(const float* __restrict__ rows, u
             out[2 * g + 1] = make_float4(gh[0], gh[1], gh[2], 0.0f);
         }
     if(!MASKS || !mask) return;
-    // 64 boxes per wave and round: the ballot of "low face in slab g or
-    // lower" is their two words of row (axis, 0, g), "high face in slab g or
-    // higher" of row (axis, 1, g); a NaN face belongs to every row of its side
-    const uint32_t nw = mask_row(n), lane = lane_id();
-    for(uint32_t wp = threadIdx.x / 64; wp < nw / 2; wp += kBlock / 64)
-        {
-            const uint32_t k = 64 * wp + lane;
-            for(int d = 0; d < 3; ++d)
-                {
-                    int lo = (int)kSlabs, hi = -1;
-                    if(k < n)
-                        {
-                            const float h = L.box[k][3 + d];
-                            lo            = slab_of(L.box[k][d], wsMin, slabScale);  // NaN: 0
-                            hi            = h == h ? slab_of(h, wsMin, slabScale) : (int)kSlabs - 1;
-                        }
-                    uint64_t keep = 0;
-#pragma unroll
-                    for(int g = 0; g < (int)kSlabs; ++g)
-                        {
-                            const uint64_t a = __ballot(lo <= g), b = __ballot(hi >= g);
-                            keep             = (int)lane == g ? a : (int)lane == (int)kSlabs + g ? b : keep;
-                        }
-                    if(lane < 2 * kSlabs)
-                        *reinterpret_cast<uint64_t*>(mask + (size_t)(2 * kSlabs * d + lane) * nw + 2 * wp) = keep;
-                }
-        }
+    box_masks(n, wsMin, slabScale, mask, [&](uint32_t k, int d) { return L.box[k][d]; });
 }
 
 // a query's scene from its rows, with its masks where MASKS and it has them
@@ -2345,20 +2353,132 @@ __global__ __launch_bounds__(kBlock) void k_stage_draw(const QueryDesc* __restri
     ufront[i] = uf;
 }
 
-template <int MODEL>
-__global__ __launch_bounds__(kBlock) void k_stage_propagate(const QueryDesc* __restrict__ qdp,
-                                                            const int32_t* __restrict__ parentIdx,
-                                                            const float* __restrict__ parentStates,
-                                                            uint32_t nParents, const float* __restrict__ controls,
-                                                            const int32_t* __restrict__ steps, uint32_t n,
-                                                            const float4* __restrict__ obs, uint32_t nGrp,
-                                                            float* child, uint8_t* valid, int32_t* r1o, int32_t* r2o)
+// Segment check of the dynamics by box masks
+struct MaskCheck
 {
-    extern __shared__ float4 sObs[];
-    stage_scene(obs, 0, nGrp, sObs);
+    const QueryDesc& qd;
+    const MaskScene& sc;
+    MaskWalk walk;
+    __device__ __forceinline__ bool operator()(float px, float py, float pz, float x, float y, float z)
+    {
+        return !walk.hit(qd, sc, px, py, pz, x, y, z, true);
+    }
+};
+
+// LDS pairs of a stage's scene: its boxes in the caller's order, their masks
+static uint32_t stage_pairs(uint32_t nObs)
+{
+    return nObs + mask_pairs(nObs);
+}
+
+template <int W>
+__device__ __forceinline__ MaskScene stage_scene_masks(const QueryDesc& qd, const float* __restrict__ rows, uint32_t n,
+                                                       float4* sObs)
+{
+    float4 *lo = sObs, *hi = sObs + n;
+    uint32_t* mask = reinterpret_cast<uint32_t*>(sObs + 2 * n);
+    for(uint32_t i = threadIdx.x; i < n; i += kBlock)
+        {
+            lo[i] = make_float4(row_face<W>(rows, i, 0), row_face<W>(rows, i, 1), row_face<W>(rows, i, 2), 0.0f);
+            hi[i] = make_float4(row_face<W>(rows, i, 3), row_face<W>(rows, i, 4), row_face<W>(rows, i, 5), 0.0f);
+        }
     __syncthreads();
-    stage_propagate_child<MODEL>(*qdp, parentIdx, parentStates, nParents, controls, steps, n, sObs, nGrp, child,
-                                 valid, r1o, r2o);
+    box_masks(n, qd.cfg.ws_min, qd.slabScale, mask, [&](uint32_t k, int d) {
+        const float4& f = d < 3 ? lo[k] : hi[k];
+        const int e     = d < 3 ? d : d - 3;
+        return e == 0 ? f.x : e == 1 ? f.y : f.z;
+    });
+    __syncthreads();
+    return MaskScene{lo, hi, mask, (int)mask_row(n), (int)n};
+}
+
+// kgmt_propagate_collide: one launch. Every workgroup builds the scene's
+// masks in its LDS (about 2 us for 200 boxes; a scene kernel before this one
+// took 10.6 and the sort its group bounds need grows with the square of the
+// boxes) and takes every gridDim.x-th tile of kBlock children: one per lane,
+// or, for the quadcopter, as the planner's tiles do. 100003 quadcopter edges
+// among 200 boxes: kernels 539 + 10.6 -> 235 us, the call 580 -> 233; 100003 of
+// the other models 102 to 246 -> 22 to 47 us, 1000 of them 55 to 65 -> 12 to 20.
+template <int MODEL>
+__global__ __launch_bounds__(kBlock, 4) void k_stage_propagate(const QueryDesc qd, const int32_t* __restrict__ parentIdx,
+                                                               const float* __restrict__ parentStates,
+                                                               uint32_t nParents, const float* __restrict__ controls,
+                                                               const int32_t* __restrict__ steps, uint32_t n,
+                                                               const float* __restrict__ rows, uint32_t nObs,
+                                                               float* __restrict__ child, uint8_t* __restrict__ valid,
+                                                               int32_t* __restrict__ r1o, int32_t* __restrict__ r2o)
+{
+    constexpr int S = ModelDims<MODEL>::S, C = ModelDims<MODEL>::C, D = S + C + 1;
+    extern __shared__ float4 sObs[];
+    const MaskScene sc = stage_scene_masks<MODEL == KGMT_MODEL_UNICYCLE ? 2 : 3>(qd, rows, nObs, sObs);
+    auto parent = [&](uint32_t i) {
+        const int32_t p = parentIdx[i];
+        return p >= 0 && (uint32_t)p < nParents ? p : -1;
+    };
+    auto write = [&](uint32_t i, int32_t p, const float* s, const float* u, bool ok) {
+        if(p < 0)
+            {
+                // caller index out of range: no state is read; flagged by r1 = r2 = -1
+                for(int d = 0; d < D; ++d) child[(size_t)d * n + i] = 0.0f;
+                valid[i] = 0;
+                r1o[i]   = -1;
+                r2o[i]   = -1;
+                return;
+            }
+#pragma unroll
+        for(int d = 0; d < S; ++d) child[(size_t)d * n + i] = s[d];
+#pragma unroll
+        for(int k = 0; k < C; ++k) child[(size_t)(S + k) * n + i] = u[k];
+        child[(size_t)(D - 1) * n + i] = qd.cfg.dt * (float)steps[i];
+        int ix, iy, iz;
+        const int r1 = region_of(qd, s[0], s[1], s[2], ix, iy, iz);
+        valid[i]     = ok ? 1 : 0;
+        r1o[i]       = r1;
+        r2o[i]       = subregion_of(qd, s[0], s[1], s[2], r1, ix, iy, iz);
+    };
+    if constexpr(MODEL == KGMT_MODEL_QUADCOPTER)
+        {
+            __shared__ QuadRunLds<kBlock> L;
+            for(uint32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock)
+                {
+                    quad_run<kBlock>(
+                      qd, n - base < kBlock ? n - base : kBlock, sc, L,
+                      [&](uint32_t k, QuadChild& ch) {
+                          const uint32_t i = base + k;
+                          const int32_t p  = parent(i);
+                          ch.p             = (uint32_t)p;
+#pragma unroll
+                          for(int d = 0; d < S; ++d) ch.s[d] = p < 0 ? 0.0f : parentStates[(size_t)d * nParents + p];
+#pragma unroll
+                          for(int c = 0; c < C; ++c) ch.u[c] = controls[(size_t)c * n + i];
+                          const int32_t st = steps[i];
+                          ch.uf            = 0.0f;
+                          ch.left          = p < 0 || st < 0 ? 0 : st;
+                      },
+                      [&](const QuadChild& ch) {
+                          write(base + (ch.meta & 1023u), (int32_t)ch.p, ch.s, ch.u, ch.left == 0);
+                      });
+                    __syncthreads();  // L is used again
+                }
+        }
+    else
+        for(uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock)
+            {
+                const int32_t p = parent(i);
+                float s[S], u[C];
+                bool ok = false;
+#pragma unroll
+                for(int d = 0; d < S; ++d) s[d] = p < 0 ? 0.0f : parentStates[(size_t)d * nParents + p];
+#pragma unroll
+                for(int k = 0; k < C; ++k) u[k] = controls[(size_t)k * n + i];
+                if(p >= 0)
+                    {
+                        MaskCheck chk{qd, sc, MaskWalk{0, 0, 0}};
+                        chk.walk.start(qd, s[0], s[1], pos_z<MODEL>(s));
+                        ok = propagate_with<MODEL>(qd, s, u, steps[i], chk);
+                    }
+                write(i, p, s, u, ok);
+            }
 }
 
 // The planner's per-child path on caller buffers: children in waves of 64
@@ -2792,18 +2912,19 @@ hipError_t launch_stage_draw(const QueryDesc* qd, int C, uint32_t query, uint32_
     return hipGetLastError();
 }
 
-hipError_t launch_stage_propagate(int model, const QueryDesc* qd, const int32_t* parentIdx, const float* parentStates,
+hipError_t launch_stage_propagate(int model, const QueryDesc& qd, const int32_t* parentIdx, const float* parentStates,
                                   uint32_t nParents, const float* controls, const int32_t* steps, uint32_t n,
-                                  const float4* obs, uint32_t nGrp, uint32_t nObs, float* child, uint8_t* valid,
-                                  int32_t* r1, int32_t* r2, hipStream_t s)
+                                  const float* rows, uint32_t nObs, float* child, uint8_t* valid, int32_t* r1,
+                                  int32_t* r2, hipStream_t s)
 {
     if(n == 0) return hipSuccess;
-    const dim3 g((n + kBlock - 1) / kBlock), b(kBlock);
-    const size_t lds = (size_t)(nGrp ? nGrp * (1 + kGroup) : 1) * 2 * sizeof(float4);
-    (void)nObs;
+    // more workgroups than the chip holds would build the masks again
+    const uint32_t most = model == KGMT_MODEL_QUADCOPTER ? 1024u : 2048u;
+    const dim3 g(std::min((n - 1) / kBlock + 1, most)), b(kBlock);
+    const size_t lds = (size_t)std::max<uint32_t>(stage_pairs(nObs), 1) * 2 * sizeof(float4);
 #define KGMT_STAGE_PROP(M)                                                                                     \
     hipLaunchKernelGGL(k_stage_propagate<M>, g, b, lds, s, qd, parentIdx, parentStates, nParents, controls, steps, \
-                       n, obs, nGrp, child, valid, r1, r2)
+                       n, rows, nObs, child, valid, r1, r2)
     switch(model)
         {
             case KGMT_MODEL_DOUBLE_INTEGRATOR: KGMT_STAGE_PROP(KGMT_MODEL_DOUBLE_INTEGRATOR); break;
