@@ -27,6 +27,8 @@
 // the kernels write into host memory.
 #include "kgmt_launch.hpp"
 
+#include <utility>
+
 namespace kgmt
 {
 
@@ -1218,84 +1220,100 @@ __device__ __forceinline__ void single_worklists(const QueryDesc& qd, const Quer
     W.active[parity] = alive ? 1u : 0u;
 }
 
-__device__ void walk_path(const QueryDesc& qd, QueryState& st, const Pools& P, float* __restrict__ out, int32_t goal);
+// f(0), .., f(N - 1) with constant indices from the start: an array that only
+// they index is split into registers before anything takes it for a vector
+template <class F, int... I>
+__device__ __forceinline__ void static_for_impl(F&& f, std::integer_sequence<int, I...>)
+{
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f)
+{
+    static_for_impl(f, std::make_integer_sequence<int, N>{});
+}
 
-// goal -> root rows of a solved single query by one wave (every lane): the
-// chain is followed six levels per round of loads (parent, grandparent and
-// the ancestors at 3..6), lane l takes the row of the l-th node, and the
-// rows go out together; cost and length are summed in walk order, so they
-// have the bits of walk_path's. Paths of more than 64 rows take walk_path.
-__device__ void walk_path_wave(const QueryDesc& qd, QueryState& st, const Pools& P, float* __restrict__ out,
-                               int32_t goal)
+// goal -> root rows of a solved query by one wave (every lane): the chain is
+// followed six levels per round of loads (parent, grandparent and the
+// ancestors at 3..6), lane l takes the row of the l-th node, and up to 64 rows
+// go out together; cost and length (of the edge durations and of the segments
+// between node positions) are summed in walk order.
+__device__ __forceinline__ void walk_path_wave(const QueryDesc& qd, QueryState& st, const Pools& P,
+                                               float* __restrict__ out, int32_t goal)
 {
     const uint32_t lane    = lane_id();
     const uint32_t cap     = qd.cap;
     const int D            = qd.D;
     const uint32_t maxRows = qd.cfg.max_iter + 2;
-    const uint32_t lim     = maxRows < 64u ? maxRows : 64u;
     const int32_t* par     = P.parent + qd.nodeOff;
     const int32_t* gpar    = P.grand + qd.nodeOff;
     const int4* anc        = P.anc + qd.nodeOff;
-    int32_t mine = lane == 0 ? goal : -1;  // this lane's node
-    int32_t f    = goal;                    // the last node found
-    uint32_t cnt = 1;                       // nodes found
-    bool root    = false;                   // the chain ended at the root
-    while(!root && cnt < lim)
-        {
-            const int32_t p = par[f], g = gpar[f];
-            const int4 a    = anc[f];
-            const int32_t up[6] = {p, g, a.x, a.y, a.z, a.w};
-#pragma unroll
-            for(int j = 0; j < 6; ++j)
-                if(!root && cnt < lim)
-                    {
-                        if(up[j] < 0 || (uint32_t)up[j] >= cap)  // -1: past the root
-                            root = true;
-                        else
-                            {
-                                if(lane == cnt) mine = up[j];
-                                f = up[j];
-                                ++cnt;
-                            }
-                    }
-        }
-    // stopped at the plan's bound of rows: the last row's parent decides
-    // whether its duration counts
-    if(!root && cnt >= maxRows) root = par[f] == -1;
-    if(!root && cnt < maxRows)
-        {
-            // longer than one wave's rows
-            if(lane == 0) walk_path(qd, st, P, out, goal);
-            return;
-        }
     const float* __restrict__ T = P.treeS + qd.sampleOff;
-    float r[KGMT_MAX_SAMPLE] = {};
-    float dn = 0.0f;
-    if(lane < cnt)
+    uint32_t rows = 0;  // rows out
+    int32_t head  = goal;
+    float pc = 0.0f, pl = 0.0f, px = 0.0f, py = 0.0f, pz = 0.0f;
+    while(true)
         {
+            const uint32_t lim = maxRows - rows < 64u ? maxRows - rows : 64u;
+            int32_t mine = lane == 0 ? head : -1;  // this lane's node
+            int32_t f    = head;                    // the last node found
+            uint32_t cnt = 1;                       // nodes found
+            bool root    = false;                   // the chain ended at the root
+            while(!root && cnt < lim)
+                {
+                    const int32_t p = par[f], g = gpar[f];
+                    const int4 a    = anc[f];
+                    const int32_t up[6] = {p, g, a.x, a.y, a.z, a.w};
 #pragma unroll
-            for(int k = 0; k < KGMT_MAX_SAMPLE; ++k)
-                if(k < D) r[k] = T[(size_t)k * cap + mine];
-            dn = T[(size_t)(D - 1) * cap + mine];
-#pragma unroll
-            for(int k = 0; k < KGMT_MAX_SAMPLE; ++k)
-                if(k < D) out[lane * D + k] = r[k];
-        }
-    // segment length from the row before (lane l - 1) to this one
-    const float qx = __shfl_up(r[0], 1, 64), qy = __shfl_up(r[1], 1, 64), qz = __shfl_up(r[2], 1, 64);
-    const float e  = lane > 0 && lane < cnt ? pos_dist(qd, qx, qy, qz, r[0], r[1], r[2]) : 0.0f;
-    // a node's edge duration counts when it has a parent: every node but the
-    // root
-    float pc = 0.0f, pl = 0.0f;
-    for(uint32_t l = 0; l < cnt; ++l)
-        {
-            const float dl = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dn), l));
-            if(!(root && l == cnt - 1)) pc = pc + dl;
-            if(l > 0) pl = pl + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), l));
+                    for(int j = 0; j < 6; ++j)
+                        if(!root && cnt < lim)
+                            {
+                                if(up[j] < 0 || (uint32_t)up[j] >= cap)  // -1: past the root
+                                    root = true;
+                                else
+                                    {
+                                        if(lane == cnt) mine = up[j];
+                                        f = up[j];
+                                        ++cnt;
+                                    }
+                            }
+                }
+            if(!root)
+                {
+                    head = par[f];
+                    root = head < 0 || (uint32_t)head >= cap;
+                }
+            // a dimension past the sample's repeats the first (never stored)
+            float r[KGMT_MAX_SAMPLE];
+            const uint32_t node = mine < 0 ? (uint32_t)f : (uint32_t)mine;
+            static_for<KGMT_MAX_SAMPLE>([&](auto K) { r[K] = T[(size_t)(K < D ? K : 0) * cap + node]; });
+            const float dn = T[(size_t)(D - 1) * cap + node];
+            if(lane < cnt)
+                static_for<KGMT_MAX_SAMPLE>([&](auto K) {
+                    if(K < D) out[(rows + lane) * D + K] = r[K];
+                });
+            // segment length from the row before (lane l - 1, or the last of
+            // the rows before) to this one
+            float qx = __shfl_up(r[0], 1, 64), qy = __shfl_up(r[1], 1, 64), qz = __shfl_up(r[2], 1, 64);
+            if(lane == 0) qx = px, qy = py, qz = pz;
+            const float e = pos_dist(qd, qx, qy, qz, r[0], r[1], r[2]);
+            // a node's edge duration counts when it has a parent: every node
+            // but the root
+            for(uint32_t l = 0; l < cnt; ++l)
+                {
+                    const float dl = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(dn), l));
+                    if(!(root && l == cnt - 1)) pc = pc + dl;
+                    if(rows + l > 0) pl = pl + __int_as_float(__builtin_amdgcn_readlane(__float_as_int(e), l));
+                }
+            rows += cnt;
+            if(root || rows >= maxRows) break;
+            px = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r[0]), cnt - 1));
+            py = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r[1]), cnt - 1));
+            pz = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r[2]), cnt - 1));
         }
     if(lane == 0)
         {
-            st.pathRows = cnt;
+            st.pathRows = rows;
             st.pathCost = pc;
             st.pathLen  = pl;
         }
@@ -1309,20 +1327,18 @@ struct Outcome
     uint64_t expanded, flagged;
 };
 
-// End of a single-query plan (one thread): the goal path rows and the result
-// into host-mapped memory, then the completion word, so the host can return
-// without waiting for the launches it queued past the last iteration (they
-// find the query done and exit). Without a host result buffer only the
-// completion word is set.
-__device__ void publish_single(const QueryDesc& qd, QueryState& st, const Pools& P, const WorkLists& W,
-                               const Outcome& r)
+// End of a single-query plan (one thread; a solved plan's path rows are out
+// already, walk_path_wave): the result into host-mapped memory, then the
+// completion word, so the host can return without waiting for the launches it
+// queued past the last iteration (they find the query done and exit). Without
+// a host result buffer only the completion word is set.
+__device__ __forceinline__ void publish_single(const QueryState& st, const WorkLists& W, const Outcome& r)
 {
     if(!W.result)
         {
             __hip_atomic_store(W.allDone, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
             return;
         }
-    if(r.success && st.pathRows == 0) walk_path(qd, st, P, W.hostPath, r.goal);
     HostResult* h = W.result;
     h->success    = r.success;
     h->iterations = r.iterations;
@@ -1376,6 +1392,31 @@ constexpr uint32_t kLbNone        = (1u << 27) - 1;  // no goal node (node indic
 constexpr uint64_t kLbAggregate   = 1ull << 62;
 constexpr uint64_t kLbInclusive   = 2ull << 62;
 constexpr uint32_t kLookBackPolls = 1u << 20;
+
+// Arguments of k_update; read in place (fresh), not copied into registers.
+struct UpdateArgs
+{
+    const QueryDesc* qds;
+    QueryState* sts;
+    Pools P;
+    WorkLists W;
+    uint32_t parity, own;
+};
+
+// v, in constant memory (kernel arguments, a descriptor), as a reference whose
+// fields are loaded where they are used after this point. Without it the
+// compiler loads every field that a job needs anywhere before the job loop,
+// runs out of scalar registers and moves them through vector lanes: 87 writes
+// in front of the loop and some 150 reads a job, each issued by all 16 waves
+// (k_update: 33 Dubins queries 11.4 to 10.1 us a launch, one 11.6 to 10.9,
+// one double integrator 10.0 to 9.1, 512 mixed queries 30.0 to 27.7).
+template <class T>
+__device__ __forceinline__ const T& fresh(const T& v)
+{
+    const __attribute__((address_space(4))) T* p = (const __attribute__((address_space(4))) T*)&v;
+    asm volatile("" : "+s"(p));
+    return *(const T*)p;
+}
 
 // LDS of an update workgroup
 struct UpdateLds
@@ -1511,7 +1552,7 @@ __device__ __forceinline__ uint32_t block_excl_scan_min(uint32_t v, uint32_t m, 
 // (nAcc, acc: this thread's share of the chunk counts) into L.nAcc.
 // KB regions per thread and round. Barriers inside: call uniformly.
 template <int KB>
-__device__ void job_scores(const QueryDesc& qd, const Pools& P, uint32_t acc, UpdateLds& L)
+__device__ __forceinline__ void job_scores(const QueryDesc& qd, const Pools& P, uint32_t acc, UpdateLds& L)
 {
     const int R1             = qd.R1;
     const uint32_t Pn        = (uint32_t)qd.P;
@@ -1701,13 +1742,14 @@ __device__ __forceinline__ void append_job(const QueryDesc& qd, const QueryState
             {
                 vcount[k]         = P.validc[qd.regOff + r1[k]];
                 const float4* row = reinterpret_cast<const float4*>(P.childR + qd.rowOffC + (size_t)slot * RW);
-#pragma unroll
-                for(int j = 0; j < kRowMax / 4; ++j)
+                static_for<kRowMax / 4>([&](auto J) {
+                    constexpr int j = J;
                     if(4 * j < RW)
                         {
                             const float4 x = row[j];
                             v[k][4 * j] = x.x, v[k][4 * j + 1] = x.y, v[k][4 * j + 2] = x.z, v[k][4 * j + 3] = x.w;
                         }
+                });
                 ++slot;
             }
     // one scan: ranks inside the chunk, flagged children of all chunks and
@@ -1730,9 +1772,10 @@ __device__ __forceinline__ void append_job(const QueryDesc& qd, const QueryState
                 {
                     if(rank < next)
                         {
-#pragma unroll
-                            for(int d = 0; d < KGMT_MAX_SAMPLE; ++d)
+                            static_for<KGMT_MAX_SAMPLE>([&](auto I) {
+                                constexpr int d = I;
                                 if(d < D) T[(size_t)d * cap + t] = v[k][2 + d];
+                            });
                             P.parent[nodeO + t]   = __float_as_int(v[k][0]);
                             P.grand[nodeO + t]    = __float_as_int(v[k][1]);
                             apar                  = __float_as_int(v[k][0]);
@@ -1753,11 +1796,15 @@ __device__ __forceinline__ void append_job(const QueryDesc& qd, const QueryState
 // scores come from the region counts (the planner); otherwise from P.score
 // (the stage entry, which is given them).
 template <bool QUADS>
-__device__ void update_job(const QueryDesc* __restrict__ qds, QueryState* __restrict__ sts, const Pools& P,
-                           const WorkLists& W, uint32_t parity, uint32_t q, uint32_t li, bool own, UpdateLds& L)
+__device__ __forceinline__ void update_job(const UpdateArgs& A0, uint32_t q, uint32_t li, UpdateLds& L)
 {
-    QueryState& st      = sts[q];
-    const QueryDesc& qd = qds[q];
+    const UpdateArgs& A = fresh(A0);
+    QueryState& st      = A.sts[q];
+    const QueryDesc& qd = fresh(A.qds[q]);
+    const WorkLists& W  = A.W;
+    const Pools& P      = A.P;
+    const bool own      = A.own != 0u;
+    const uint32_t parity = A.parity;
     const uint32_t nq   = W.nq;
     const uint32_t tree = st.treeSize, nC = st.nChildren, cap = qd.cap;
     const uint32_t nOC  = (tree + kChunk - 1) / kChunk;
@@ -1925,7 +1972,7 @@ __device__ void update_job(const QueryDesc* __restrict__ qds, QueryState* __rest
             if(nq == 1 && jobGoal != kLbNone && goalBefore == kLbNone)
                 {
                     const Outcome r{1u, st.itr, tree + next, (int32_t)jobGoal, st.expanded + nC, st.flagged + nAcc};
-                    publish_single(qd, st, P, W, r);
+                    publish_single(st, W, r);
                 }
             // the last job knows the list size and the goal: it closes the
             // iteration of a single query (the next-state fields and work
@@ -1946,7 +1993,7 @@ __device__ void update_job(const QueryDesc* __restrict__ qds, QueryState* __rest
                             if(st.doneN && !st.successN)
                                 {
                                     const Outcome r{0u, st.finishItrN, st.treeSizeN, -1, st.expandedN, st.flaggedN};
-                                    publish_single(qd, st, P, W, r);
+                                    publish_single(st, W, r);
                                 }
                         }
                 }
@@ -1955,10 +2002,14 @@ __device__ void update_job(const QueryDesc* __restrict__ qds, QueryState* __rest
 
 // QUADS: some query is a quadcopter's
 template <bool QUADS>
-__global__ __launch_bounds__(kUpd) void k_update(const QueryDesc* __restrict__ qds, QueryState* __restrict__ sts,
-                                                   Pools P, WorkLists W, uint32_t parity, uint32_t own)
+__global__ __launch_bounds__(kUpd) void k_update(UpdateArgs)
 {
     __shared__ UpdateLds L;
+    const UpdateArgs& A = *(const UpdateArgs*)__builtin_amdgcn_kernarg_segment_ptr();
+    const WorkLists& W  = A.W;
+    const QueryDesc* __restrict__ qds = A.qds;
+    QueryState* __restrict__ sts      = A.sts;
+    const uint32_t parity             = A.parity;
     const uint32_t nq       = W.nq;
     const uint32_t* jobList = W.jobs(parity);
     // one query: its jobs 0 .. nJ-1 straight from its state (the list holds
@@ -1984,9 +2035,9 @@ __global__ __launch_bounds__(kUpd) void k_update(const QueryDesc* __restrict__ q
                     j = L.job;
                     if(j >= nJobs) return;
                 }
-            const uint32_t q = nq > 1 ? locate(jobList, nq, j) : 0u;
+            const uint32_t q = nq > 1 ? (uint32_t)__builtin_amdgcn_readfirstlane((int)locate(jobList, nq, j)) : 0u;
             // (a stale list entry of a finished query has nothing to do)
-            if(!sts[q].done) update_job<QUADS>(qds, sts, P, W, parity, q, nq > 1 ? j - jobList[q] : j, own != 0, L);
+            if(!sts[q].done) update_job<QUADS>(A, q, nq > 1 ? j - jobList[q] : j, L);
             if(!more) return;
             __syncthreads();  // L is rewritten by the next job
         }
@@ -2008,74 +2059,19 @@ __global__ __launch_bounds__(kBlock) void k_finish(const QueryDesc* __restrict__
 }
 
 // ---------------------------------------------------------------------------
-// paths: goal -> root rows of every solved query, exact depth (Q13); path
-// cost = sum of edge durations, length = sum of segment lengths between the
-// node positions
+// paths: goal -> root rows of every solved query, exact depth (Q13), one wave
+// per query (512 mixed queries: 40.4 us with one thread per query and two
+// levels a round)
 // ---------------------------------------------------------------------------
-// goal -> root rows of a solved query (pathRows etc. of st); two levels per
-// round of loads: a and its parent b are known, their rows, b's parent c and
-// grandparent d are loaded together
-__device__ void walk_path(const QueryDesc& qd, QueryState& st, const Pools& P, float* __restrict__ out, int32_t goal)
-{
-    const uint32_t cap            = qd.cap;
-    const int D                   = qd.D;
-    const float* __restrict__ T   = P.treeS + qd.sampleOff;
-    const float* __restrict__ dur = T + (size_t)(D - 1) * cap;  // edge durations
-    const int32_t* par            = P.parent + qd.nodeOff;
-    const int32_t* gpar           = P.grand + qd.nodeOff;
-    uint32_t rows                 = 0;
-    float pc = 0.0f, pl = 0.0f, px = 0.0f, py = 0.0f, pz = 0.0f;
-    const uint32_t maxRows = qd.cfg.max_iter + 2;
-    // one node's row, in walk order (its parent pn decides whether its edge
-    // duration dn counts); indices into r are compile-time constants
-    auto emit = [&](const float* r, float dn, int32_t pn) {
-#pragma unroll
-        for(int k = 0; k < KGMT_MAX_SAMPLE; ++k)
-            if(k < D) out[rows * D + k] = r[k];
-        if(pn != -1) pc = pc + dn;
-        if(rows > 0) pl = pl + pos_dist(qd, px, py, pz, r[0], r[1], r[2]);
-        px = r[0], py = r[1], pz = r[2];
-        ++rows;
-    };
-    int32_t a = goal;
-    int32_t b = par[a];
-    while(a != -1 && rows < maxRows)
-        {
-            float ra[KGMT_MAX_SAMPLE], rb[KGMT_MAX_SAMPLE];
-            float da = dur[a], db = 0.0f;
-            int32_t c = -1, d = -1;
-#pragma unroll
-            for(int k = 0; k < KGMT_MAX_SAMPLE; ++k)
-                if(k < D) ra[k] = T[(size_t)k * cap + a];
-            if(b != -1)
-                {
-#pragma unroll
-                    for(int k = 0; k < KGMT_MAX_SAMPLE; ++k)
-                        if(k < D) rb[k] = T[(size_t)k * cap + b];
-                    db = dur[b];
-                    c  = par[b];
-                    d  = gpar[b];
-                }
-            emit(ra, da, b);
-            if(b == -1 || rows >= maxRows) break;
-            emit(rb, db, c);
-            a = c;
-            b = d;
-        }
-    st.pathRows = rows;
-    st.pathCost = pc;
-    st.pathLen  = pl;
-}
-
 __global__ __launch_bounds__(64) void k_paths(const QueryDesc* __restrict__ qds, QueryState* __restrict__ sts,
                                               Pools P, uint32_t nq)
 {
-    const uint32_t q = blockIdx.x * 64 + threadIdx.x;
-    if(q >= nq) return;
-    QueryState& st = sts[q];
-    commit_state(st);  // the closed last iteration
-    if(!st.success || st.pathRows) return;
-    walk_path(qds[q], st, P, P.path + qds[q].pathOff, st.goalIdx);
+    const uint32_t q = blockIdx.x;
+    QueryState& st   = sts[q];
+    if(threadIdx.x == 0) commit_state(st);  // the closed last iteration
+    if(!st.successN || st.pathRows) return;
+    const QueryDesc& qd = qds[q];
+    walk_path_wave(qd, st, P, P.path + qd.pathOff, st.goalIdx);
 }
 
 // ---------------------------------------------------------------------------
@@ -2858,10 +2854,11 @@ hipError_t launch_update(const QueryDesc* qds, QueryState* sts, const Pools& P, 
                          uint32_t parity, const Launch& L, bool own, hipStream_t s)
 {
     const dim3 g(L.chunkGrid), b(kUpd);
+    const UpdateArgs a{qds, sts, P, W, parity, own ? 1u : 0u};
     if(W.quads)
-        hipLaunchKernelGGL(k_update<true>, g, b, 0, s, qds, sts, P, W, parity, own ? 1u : 0u);
+        hipLaunchKernelGGL(k_update<true>, g, b, 0, s, a);
     else
-        hipLaunchKernelGGL(k_update<false>, g, b, 0, s, qds, sts, P, W, parity, own ? 1u : 0u);
+        hipLaunchKernelGGL(k_update<false>, g, b, 0, s, a);
     return hipGetLastError();
 }
 
@@ -2884,7 +2881,7 @@ hipError_t launch_finish(const QueryDesc* qds, QueryState* sts, const WorkLists&
 hipError_t launch_paths(const QueryDesc* qds, QueryState* sts, const Pools& P, uint32_t nq, hipStream_t s)
 {
     if(nq == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_paths, dim3((nq + 63) / 64), dim3(64), 0, s, qds, sts, P, nq);
+    hipLaunchKernelGGL(k_paths, dim3(nq), dim3(64), 0, s, qds, sts, P, nq);
     return hipGetLastError();
 }
 
