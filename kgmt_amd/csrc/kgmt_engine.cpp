@@ -127,7 +127,10 @@ void fill_desc(QueryDesc& qd, const kgmt_config& c)
     qd.R1      = (int32_t)ipow(c.r1_len, qd.wdim);
     qd.P       = (int32_t)ipow(c.r2_len, qd.wdim);
     qd.R2      = qd.R1 * qd.P;
-    qd.R2words = (qd.R2 + 31) / 32;
+    // the planner's bitsets: whole words per region
+    qd.regShift = region_shift((uint32_t)qd.R1);
+    qd.actW     = (uint32_t)(qd.P + 31) / 32;
+    qd.R2words  = (int32_t)((qd.actW <= 2 ? 16u << qd.regShift : (uint32_t)qd.R1) * qd.actW);
     qd.cap     = c.capacity;
     qd.nChunks = (c.capacity + kChunk - 1) / kChunk;
     // W_R1_SIZE and W_R1_VOL as the float macros of config.h:247-251 evaluate
@@ -326,7 +329,7 @@ struct Engine
                 rows += (uint64_t)row_words(qd.D) * qd.cap;
                 nodes += ((uint64_t)qd.cap + kNodeAlign - 1) / kNodeAlign * kNodeAlign;
                 chunks += qd.nChunks + 1;
-                regs += (uint32_t)qd.R1;
+                regs += 16u << qd.regShift;
                 subs += (uint32_t)qd.R2words;
                 paths += (uint64_t)(cfgs[q].max_iter + 2) * qd.D;
                 if(paths > 0xffffffffull) return fail(KGMT_E_CAPACITY, "path pool too large");
@@ -344,8 +347,8 @@ struct Engine
            (rc = dev_alloc(P.r1child, nodes, owned)) ||
            (rc = dev_alloc(P.fnext, nodes, owned)) || (rc = dev_alloc(P.react, nodes, owned)) ||
            (rc = dev_alloc(P.repIdx, nodes, owned)) || (rc = dev_alloc(P.partA, chunks, owned)) ||
-           (rc = dev_alloc(P.look, 4 * (size_t)chunks, owned)) || (rc = dev_alloc(P.total, regs, owned)) ||
-           (rc = dev_alloc(P.validc, regs, owned)) || (rc = dev_alloc(P.score, regs, owned)) ||
+           (rc = dev_alloc(P.look, 4 * (size_t)chunks, owned)) || (rc = dev_alloc(P.cnt, regs, owned)) ||
+           (rc = dev_alloc(P.score, regs, owned)) ||
            (rc = dev_alloc(P.actPrev, subs, owned)) || (rc = dev_alloc(P.actNext, subs, owned)) ||
            (rc = dev_alloc(P.path, paths, owned)) || (rc = dev_alloc(W.tileStart, 2 * (size_t)(n + 1), owned)) ||
            (rc = dev_alloc(W.jobStart, 2 * (size_t)(n + 1), owned)) || (rc = dev_alloc(W.active, 2, owned)) ||
@@ -746,6 +749,23 @@ struct Engine
         return KGMT_OK;
     }
 
+    // per-region counters of query q, in region order
+    int region_counts(uint32_t q, std::vector<int32_t>* total, std::vector<int32_t>* valid) const
+    {
+        const QueryDesc& qd = hq[q];
+        std::vector<uint64_t> c(16u << qd.regShift);
+        HIP_TRY(hipMemcpy(c.data(), P.cnt + qd.regOff, sizeof(uint64_t) * c.size(), hipMemcpyDeviceToHost));
+        if(total) total->resize(qd.R1);
+        if(valid) valid->resize(qd.R1);
+        for(uint32_t r = 0; r < (uint32_t)qd.R1; ++r)
+            {
+                const uint64_t v = c[region_slot(r, qd.regShift)];
+                if(total) (*total)[r] = (int32_t)(uint32_t)v;
+                if(valid) (*valid)[r] = (int32_t)(v >> 32);
+            }
+        return KGMT_OK;
+    }
+
     // frontier flags and repeat counts of query q's tree nodes after the
     // last iteration: 1 for an old node it re-activated, 15 or 1 for a node it
     // appended (its region's valid count, final for that iteration, below
@@ -765,12 +785,12 @@ struct Engine
             {
                 const uint32_t next = std::min(st.next, ts), old = ts - next;
                 std::vector<uint8_t> react(old);
-                std::vector<int32_t> r1(next), valid(qd.R1);
+                std::vector<int32_t> r1(next), valid;
                 if(old) HIP_TRY(hipMemcpy(react.data(), P.react + qd.nodeOff, old, hipMemcpyDeviceToHost));
                 if(next)
                     HIP_TRY(hipMemcpy(r1.data(), P.r1node + qd.nodeOff + old, sizeof(int32_t) * next,
                                       hipMemcpyDeviceToHost));
-                HIP_TRY(hipMemcpy(valid.data(), P.validc + qd.regOff, sizeof(int32_t) * qd.R1, hipMemcpyDeviceToHost));
+                if(int rc = region_counts(q, nullptr, &valid)) return rc;
                 for(uint32_t i = 0; i < old; ++i) repeat[i] = react[i] ? 1u : 0u;
                 for(uint32_t j = 0; j < next; ++j)
                     repeat[old + j] = valid[r1[j]] < qd.cfg.sparse_valid_below ? qd.cfg.repeat_sparse
@@ -1221,8 +1241,13 @@ int kgmt_get_regions(kgmt_ctx* ctx, int32_t* total, int32_t* valid, float* score
     if(n) *n = (uint32_t)qd.R1;
     if(cap < (uint32_t)qd.R1 && (total || valid || score)) return fail(KGMT_E_CAPACITY, "region buffer too small");
     HIP_TRY(hipStreamSynchronize(e.stream));  // a plan returns before its trailing launches drain
-    if(total) HIP_TRY(hipMemcpy(total, e.P.total + qd.regOff, sizeof(int32_t) * qd.R1, hipMemcpyDeviceToHost));
-    if(valid) HIP_TRY(hipMemcpy(valid, e.P.validc + qd.regOff, sizeof(int32_t) * qd.R1, hipMemcpyDeviceToHost));
+    if(total || valid)
+        {
+            std::vector<int32_t> t, v;
+            if(int rc = e.region_counts(0, &t, &v)) return rc;
+            if(total) std::copy(t.begin(), t.end(), total);
+            if(valid) std::copy(v.begin(), v.end(), valid);
+        }
     if(score) HIP_TRY(hipMemcpy(score, e.P.score + qd.regOff, sizeof(float) * qd.R1, hipMemcpyDeviceToHost));
     return KGMT_OK;
 }
@@ -1511,7 +1536,7 @@ int kgmt_frontier_update(const kgmt_config* cfg, uint32_t itr, uint32_t tree_siz
        (rc = a.get(P.frontier, nodes)) || (rc = a.get(P.r1node, nodes)) || (rc = a.get(P.r1child, nodes)) ||
        (rc = a.get(P.fnext, nodes)) || (rc = a.get(P.react, nodes)) || (rc = a.get(P.repIdx, nodes)) ||
        (rc = a.get(P.partA, h.nChunks + 1)) || (rc = a.get(P.look, 4 * ((size_t)h.nChunks + 1))) ||
-       (rc = a.get(P.validc, h.R1)) || (rc = a.get(P.score, h.R1)) || (rc = a.get(W.tileStart, 4)) ||
+       (rc = a.get(P.cnt, 16u << h.regShift)) || (rc = a.get(P.score, h.R1)) || (rc = a.get(W.tileStart, 4)) ||
        (rc = a.get(W.jobStart, 4)) || (rc = a.get(W.active, 2)) || (rc = a.get(W.counter, 1)) ||
        (rc = a.get(W.claim, 2)) || (rc = a.get(W.allDone, 1)) || (rc = a.get(W.error, 1)) ||
        (rc = a.get(W.closed, 1)) || (rc = a.get(W.closedDev, 1)))
@@ -1525,10 +1550,9 @@ int kgmt_frontier_update(const kgmt_config* cfg, uint32_t itr, uint32_t tree_siz
     HIP_TRY(hipMemcpyAsync(P.parent, d_parents, sizeof(int32_t) * cap, hipMemcpyDeviceToDevice, s));
     HIP_TRY(hipMemcpyAsync(P.cost, d_costs, sizeof(float) * cap, hipMemcpyDeviceToDevice, s));
     HIP_TRY(hipMemcpyAsync(P.frontier, d_frontier, cap, hipMemcpyDeviceToDevice, s));
-    HIP_TRY(hipMemcpyAsync(P.validc, d_valid_count, sizeof(int32_t) * h.R1, hipMemcpyDeviceToDevice, s));
     HIP_TRY(hipMemcpyAsync(P.score, d_score, sizeof(float) * h.R1, hipMemcpyDeviceToDevice, s));
-    hipError_t e = launch_stage_frontier_update(dq, ds, P, W, itr, tree_size, d_child_samples, d_child_parent,
-                                                d_fnext, n_children, info, s);
+    hipError_t e = launch_stage_frontier_update(dq, ds, P, W, (uint32_t)h.R1, itr, tree_size, d_child_samples,
+                                                d_child_parent, d_fnext, n_children, d_valid_count, info, s);
     if(e != hipSuccess) return fail(KGMT_E_HIP, std::string("frontier update: ") + hipGetErrorString(e));
     HIP_TRY(hipMemcpyAsync(d_tree_samples, P.treeS, sizeof(float) * h.D * cap, hipMemcpyDeviceToDevice, s));
     HIP_TRY(hipMemcpyAsync(d_parents, P.parent, sizeof(int32_t) * cap, hipMemcpyDeviceToDevice, s));

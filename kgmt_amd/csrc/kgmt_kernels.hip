@@ -381,11 +381,10 @@ __device__ __forceinline__ bool last_arrival(uint32_t* counter, uint32_t expecte
 // job words of one query: thread `rank` of `ranks` clears every ranks-th word
 __device__ void clear_query(const QueryDesc& qd, const Pools& P, uint32_t rank, uint32_t ranks)
 {
-    for(uint32_t r = rank; r < (uint32_t)qd.R1; r += ranks)
+    for(uint32_t r = rank; r < 16u << qd.regShift; r += ranks)
         {
-            P.total[qd.regOff + r]  = 0;
-            P.validc[qd.regOff + r] = 0;
-            P.score[qd.regOff + r]  = 0.0f;
+            P.cnt[qd.regOff + r]   = 0ull;
+            P.score[qd.regOff + r] = 0.0f;
         }
     for(uint32_t w = rank; w < (uint32_t)qd.R2words; w += ranks)
         {
@@ -508,6 +507,23 @@ __device__ __forceinline__ void store_row(float* rows, uint32_t v, int32_t p, in
     float4* row = reinterpret_cast<float4*>(rows + (size_t)v * RW);
 #pragma unroll
     for(int j = 0; j < RW / 4; ++j) row[j] = make_float4(w[4 * j], w[4 * j + 1], w[4 * j + 2], w[4 * j + 3]);
+}
+
+// word and bit of subregion r2 (r1 P + local) in the planner's bitsets
+__device__ __forceinline__ void subregion_bit(const QueryDesc& qd, int r1, int r2, uint32_t& word, uint32_t& bit)
+{
+    const uint32_t sub = (uint32_t)(r2 - r1 * qd.P);
+    word               = region_word((uint32_t)r1, qd.regShift, qd.actW) + (sub >> 5);
+    bit                = 1u << (sub & 31u);
+}
+
+// a tile's children and valid children of region r, one atomic for both
+// (the low word would carry past 2^32 children of one region in a plan)
+__device__ __forceinline__ void count_region(const QueryDesc& qd, const Pools& P, uint32_t r, uint32_t total,
+                                             uint32_t valid)
+{
+    atomicAdd(reinterpret_cast<unsigned long long*>(P.cnt + qd.regOff + region_slot(r, qd.regShift)),
+              (unsigned long long)valid << 32 | total);
 }
 
 // One tile of TC = NT / K children u = base .. base + TC - 1 of a query (TC
@@ -635,7 +651,7 @@ __device__ __forceinline__ void child_tile(const QueryDesc& qd, const QueryState
     int r1              = 0;
     bool ok = false, fn = false;
     bool setBit   = false;  // valid child in a subregion unseen at iteration start
-    uint32_t r2bit = 0;
+    uint32_t word = 0, bit = 0;  // of the subregion
     uint32_t p         = 0;
     int32_t gp         = -1;  // parent of the parent
     float s[S], uc[C];
@@ -685,11 +701,11 @@ __device__ __forceinline__ void child_tile(const QueryDesc& qd, const QueryState
                     r1 = region_of(qd, s[0], s[1], s[2], ix, iy, iz);
                     if(ok)
                         {
-                            const int r2    = subregion_of(qd, s[0], s[1], s[2], r1, ix, iy, iz);
-                            const bool seen = test_bit(P.actPrev + qd.subOff, (uint32_t)r2);
+                            const int r2 = subregion_of(qd, s[0], s[1], s[2], r1, ix, iy, iz);
+                            subregion_bit(qd, r1, r2, word, bit);
+                            const bool seen = (P.actPrev[qd.subOff + word] & bit) != 0u;
                             fn              = (uf < P.score[qd.regOff + r1]) || !seen;
                             setBit          = !seen;
-                            r2bit           = (uint32_t)r2;
                         }
                     if(u % per == 0) P.frontier[nodeO + p] = 0;
                     P.r1child[nodeO + u] = r1;
@@ -707,8 +723,8 @@ __device__ __forceinline__ void child_tile(const QueryDesc& qd, const QueryState
         }
     if(setBit)
         {
-            const uint32_t e = tab_slot<NT>(L.wkey, (int32_t)(r2bit >> 5));
-            atomicOr(&L.wmask[e], 1u << (r2bit & 31u));
+            const uint32_t e = tab_slot<NT>(L.wkey, (int32_t)word);
+            atomicOr(&L.wmask[e], bit);
         }
     // the tile lies inside one 1024-element chunk
     const uint64_t fm = __ballot(fn);
@@ -724,11 +740,7 @@ __device__ __forceinline__ void child_tile(const QueryDesc& qd, const QueryState
         }
     {
         const int32_t rk = L.rkey[t];
-        if(rk >= 0)
-            {
-                atomicAdd(&P.total[qd.regOff + rk], (int32_t)L.rtot[t]);
-                if(L.rval[t]) atomicAdd(&P.validc[qd.regOff + rk], (int32_t)L.rval[t]);
-            }
+        if(rk >= 0) count_region(qd, P, (uint32_t)rk, L.rtot[t], L.rval[t]);
         const int32_t wk = L.wkey[t];
         if(wk >= 0) atomicOr(&P.actNext[qd.subOff + (uint32_t)wk], L.wmask[t]);
         // empty for the next tile, which uses the other flag buffer (this
@@ -1002,16 +1014,16 @@ __device__ __forceinline__ void quad_tile(const QueryDesc& qd, const QueryState&
           const uint32_t u = base + (ch.meta & 1023u);
           const bool ok    = ch.left == 0;
           bool fn = false, setBit = false;
-          uint32_t r2bit = 0;
+          uint32_t word = 0, bit = 0;
           int ix, iy, iz;
           const int r1 = region_of(qd, ch.s[0], ch.s[1], ch.s[2], ix, iy, iz);
           if(ok)
               {
-                  const int r2    = subregion_of(qd, ch.s[0], ch.s[1], ch.s[2], r1, ix, iy, iz);
-                  const bool seen = test_bit(P.actPrev + qd.subOff, (uint32_t)r2);
+                  const int r2 = subregion_of(qd, ch.s[0], ch.s[1], ch.s[2], r1, ix, iy, iz);
+                  subregion_bit(qd, r1, r2, word, bit);
+                  const bool seen = (P.actPrev[qd.subOff + word] & bit) != 0u;
                   fn              = (ch.uf < P.score[qd.regOff + r1]) || !seen;
                   setBit          = !seen;
-                  r2bit           = (uint32_t)r2;
               }
           if(u % per == 0) P.frontier[nodeO + ch.p] = 0;
           P.r1child[nodeO + u] = r1;
@@ -1021,8 +1033,8 @@ __device__ __forceinline__ void quad_tile(const QueryDesc& qd, const QueryState&
           if(ok) atomicAdd(&L.rval[e], 1u);
           if(setBit)
               {
-                  const uint32_t f = tab_slot<kT>(L.wkey, (int32_t)(r2bit >> 5));
-                  atomicOr(&L.wmask[f], 1u << (r2bit & 31u));
+                  const uint32_t f = tab_slot<kT>(L.wkey, (int32_t)word);
+                  atomicOr(&L.wmask[f], bit);
               }
           // the tile lies inside one 1024-element chunk
           const uint64_t fm = __ballot(fn);
@@ -1038,11 +1050,7 @@ __device__ __forceinline__ void quad_tile(const QueryDesc& qd, const QueryState&
     for(int k = (int)threadIdx.x; k < kT; k += NT)
         {
             const int32_t rk = L.rkey[k];
-            if(rk >= 0)
-                {
-                    atomicAdd(&P.total[qd.regOff + rk], (int32_t)L.rtot[k]);
-                    if(L.rval[k]) atomicAdd(&P.validc[qd.regOff + rk], (int32_t)L.rval[k]);
-                }
+            if(rk >= 0) count_region(qd, P, (uint32_t)rk, L.rtot[k], L.rval[k]);
             const int32_t wk = L.wkey[k];
             if(wk >= 0) atomicOr(&P.actNext[qd.subOff + (uint32_t)wk], L.wmask[k]);
         }
@@ -1418,13 +1426,21 @@ __device__ __forceinline__ const T& fresh(const T& v)
     return *(const T*)p;
 }
 
+// Place of a region's raw score in LDS: rows of 16 counter slots, padded to 17
+// words, so that threads in slot order (the counters' loads) and threads in
+// region order (the score tree) both spread over the banks
+__device__ __forceinline__ uint32_t raw_index(uint32_t r, uint32_t shift)
+{
+    return (r & ((1u << shift) - 1u)) * 17u + (r >> shift);
+}
+
 // LDS of an update workgroup
 struct UpdateLds
 {
     union
     {
-        float raw[kMaxRegions];        // raw region scores (-1: no valid child) of a re-activation job
-        uint32_t stage[kMaxRegions];   // then the job's expansion-list entries
+        float raw[17 * (kMaxRegions / 16)];  // raw region scores (-1: no valid child), at raw_index
+        uint32_t stage[kMaxRegions];         // then the job's expansion-list entries
     };
     float part[kUpd];                   // the score tree's partial sums
     uint32_t sbuf[3 * (kUpd / 64)];     // block scans
@@ -1550,47 +1566,64 @@ __device__ __forceinline__ uint32_t block_excl_scan_min(uint32_t v, uint32_t m, 
 // query's own padded size add zeros, which leave every partial sum's bits
 // unchanged), into L.sum; with the flagged children of the iteration
 // (nAcc, acc: this thread's share of the chunk counts) into L.nAcc.
-// KB regions per thread and round. Barriers inside: call uniformly.
+// KB regions per thread (KB kUpd cover the query's). Barriers inside: call
+// uniformly.
 template <int KB>
 __device__ __forceinline__ void job_scores(const QueryDesc& qd, const Pools& P, uint32_t acc, UpdateLds& L)
 {
-    const int R1             = qd.R1;
-    const uint32_t Pn        = (uint32_t)qd.P;
-    const int t              = (int)threadIdx.x;
-    const int32_t* total     = P.total + qd.regOff;
-    const int32_t* validc    = P.validc + qd.regOff;
-    const uint32_t* act      = P.actNext + qd.subOff;
-    // KB regions per thread and round: every load of a round is issued
-    // before any is used (indices clamped into the query's regions, so no
-    // load sits behind a branch)
-    const bool oneWord   = Pn <= 32u && 32u % Pn == 0u;
-    for(int k0 = t; k0 < R1; k0 += KB * (int)kUpd)
+    const uint32_t R1    = (uint32_t)qd.R1;
+    const int t          = (int)threadIdx.x;
+    const uint32_t sh    = qd.regShift, actW = qd.actW;
+    const uint32_t slots = 16u << sh;
+    const uint64_t* cnt  = P.cnt + qd.regOff;
+    const uint32_t* act  = P.actNext + qd.subOff;
+    // KB counter slots per thread, every load issued before any is used
+    // (indices clamped into the query's slots, so no load sits behind a
+    // branch); up to 64 subregion bits per region lie at the same slots
+    uint64_t c[KB];
+    uint32_t n[KB];  // active subregions
+#pragma unroll
+    for(int k = 0; k < KB; ++k)
         {
-            int32_t vc[KB], tc[KB];
-            uint32_t aw[KB];
+            const uint32_t i = (uint32_t)t + (uint32_t)k * kUpd;
+            c[k]             = cnt[i < slots ? i : slots - 1u];
+        }
+    auto bits = [&](auto x) {  // x: a region's bits
+        using T = decltype(x);
 #pragma unroll
+        for(int k = 0; k < KB; ++k)
+            {
+                const uint32_t i = (uint32_t)t + (uint32_t)k * kUpd;
+                n[k]             = (uint32_t)__popcll(reinterpret_cast<const T*>(act)[i < slots ? i : slots - 1u]);
+            }
+    };
+    if(actW == 1u)
+        bits(uint32_t{});
+    else if(actW == 2u)
+        bits(uint64_t{});
+    else
+        {
+            // more (in region order): their counts at the places of this
+            // thread's raw scores
+#pragma unroll 1
             for(int k = 0; k < KB; ++k)
                 {
-                    const int r  = k0 + k * (int)kUpd;
-                    const int rr = r < R1 ? r : R1 - 1;
-                    vc[k]        = validc[rr];
-                    tc[k]        = total[rr];
-                    aw[k]        = oneWord ? act[((uint32_t)rr * Pn) >> 5] : 0u;
+                    const uint32_t i = (uint32_t)t + (uint32_t)k * kUpd, r = slot_region(i, sh);
+                    uint32_t m       = 0u;
+                    if(i < slots && r < R1)
+                        for(uint32_t w = 0; w < actW; ++w) m += (uint32_t)__popc(act[(size_t)r * actW + w]);
+                    if(i < slots) L.raw[(i >> 4) * 17u + (i & 15u)] = __uint_as_float(m);
                 }
+        }
 #pragma unroll
-            for(int k = 0; k < KB; ++k)
-                {
-                    const int r = k0 + k * (int)kUpd;
-                    if(r < R1 && vc[k] > 0)
-                        {
-                            const uint32_t b   = (uint32_t)r * Pn;
-                            const uint32_t m   = Pn == 32u ? 0xffffffffu : ((1u << (Pn & 31u)) - 1u) << (b & 31u);
-                            const uint32_t cnt = oneWord ? (uint32_t)__popc(aw[k] & m) : count_bits(act, b, Pn);
-                            L.raw[r]           = region_raw_score(qd, vc[k], tc[k], cnt);
-                        }
-                    else if(r < R1)
-                        L.raw[r] = -1.0f;
-                }
+    for(int k = 0; k < KB; ++k)
+        {
+            const uint32_t i = (uint32_t)t + (uint32_t)k * kUpd;
+            const uint32_t r = slot_region(i, sh);
+            const int32_t vc = (int32_t)(c[k] >> 32), tc = (int32_t)(uint32_t)c[k];
+            float& raw       = L.raw[(i >> 4) * 17u + (i & 15u)];  // raw_index(r)
+            if(i < slots && r < R1)
+                raw = vc > 0 ? region_raw_score(qd, vc, tc, actW > 2u ? __float_as_uint(raw) : n[k]) : -1.0f;
         }
     // the flagged children of the iteration, per wave (used after the tree)
     const uint32_t lane    = lane_id();
@@ -1600,17 +1633,16 @@ __device__ __forceinline__ void job_scores(const QueryDesc& qd, const Pools& P, 
     __syncthreads();
     // the thread's leaves t + k kUpd; the levels with stride >= kUpd add
     // the thread's own registers
-    constexpr int KR = kMaxRegions / (int)kUpd;
-    float sv[KR];
+    float sv[KB];
 #pragma unroll
-    for(int k = 0; k < KR; ++k)
+    for(int k = 0; k < KB; ++k)
         {
-            const int r = t + k * (int)kUpd;
-            const float x = r < R1 ? L.raw[r] : 0.0f;
-            sv[k]         = x < 0.0f ? 0.0f : x;
+            const uint32_t r = (uint32_t)t + (uint32_t)k * kUpd;
+            const float x    = r < R1 ? L.raw[raw_index(r, sh)] : 0.0f;
+            sv[k]            = x < 0.0f ? 0.0f : x;
         }
 #pragma unroll
-    for(int m = KR / 2; m >= 1; m >>= 1)
+    for(int m = KB / 2; m >= 1; m >>= 1)
         {
 #pragma unroll
             for(int k = 0; k < m; ++k) sv[k] = sv[k] + sv[k + m];
@@ -1677,7 +1709,7 @@ __device__ __forceinline__ void react_job(const QueryDesc& qd, const QueryState&
     for(uint32_t k = 0; k < kPer; ++k)
         {
             const bool cand = i0 + k < tree && ((fw >> (8 * k)) & 0xffu) == 0;
-            sc[k] = !cand ? 0.0f : own ? region_score(qd, raw[r[k]], sum) : P.score[qd.regOff + r[k]];
+            sc[k] = !cand ? 0.0f : own ? region_score(qd, raw[raw_index((uint32_t)r[k], qd.regShift)], sum) : P.score[qd.regOff + r[k]];
         }
     uint32_t rw = 0;
 #pragma unroll
@@ -1740,7 +1772,8 @@ __device__ __forceinline__ void append_job(const QueryDesc& qd, const QueryState
     for(uint32_t k = 0; k < kPer; ++k)
         if((fl >> k) & 1u)
             {
-                vcount[k]         = P.validc[qd.regOff + r1[k]];
+                vcount[k] = reinterpret_cast<const int32_t*>(
+                  P.cnt + qd.regOff)[2 * region_slot((uint32_t)r1[k], qd.regShift) + 1];  // valid children
                 const float4* row = reinterpret_cast<const float4*>(P.childR + qd.rowOffC + (size_t)slot * RW);
                 static_for<kRowMax / 4>([&](auto J) {
                     constexpr int j = J;
@@ -1923,12 +1956,24 @@ __device__ __forceinline__ void update_job(const UpdateArgs& A0, uint32_t q, uin
         }
     // (work that no job of this launch reads) the other parity's words start
     // empty for the next launch; job 0 stores the scores and the subregion
-    // snapshot for the next propagate
+    // snapshot for the next propagate (four loads in flight a thread)
     for(size_t i = (size_t)li * kUpd + threadIdx.x; i < wpq; i += (size_t)nJ * kUpd) wordsNext[i] = 0ull;
     if(li == 0 && own)
         {
-            for(int r = threadIdx.x; r < qd.R1; r += kUpd) P.score[qd.regOff + r] = region_score(qd, L.raw[r], L.sum);
-            for(int w = threadIdx.x; w < qd.R2words; w += kUpd) P.actPrev[qd.subOff + w] = P.actNext[qd.subOff + w];
+            const uint32_t* act  = P.actNext + qd.subOff;
+            uint32_t* prev       = P.actPrev + qd.subOff;
+            const uint32_t words = (uint32_t)qd.R2words;
+            for(uint32_t w0 = threadIdx.x; w0 < words; w0 += 4 * kUpd)
+                {
+                    uint32_t x[4];
+#pragma unroll
+                    for(uint32_t k = 0; k < 4; ++k) x[k] = act[w0 + k * kUpd < words ? w0 + k * kUpd : w0];
+#pragma unroll
+                    for(uint32_t k = 0; k < 4; ++k)
+                        if(w0 + k * kUpd < words) prev[w0 + k * kUpd] = x[k];
+                }
+            for(int r = threadIdx.x; r < qd.R1; r += kUpd)
+                P.score[qd.regOff + r] = region_score(qd, L.raw[raw_index((uint32_t)r, qd.regShift)], L.sum);
         }
     __syncthreads();
     const uint32_t before = L.before, goalBefore = L.goalBefore;
@@ -2573,12 +2618,14 @@ __global__ __launch_bounds__(kBlock) void k_stage_propagate_planner(
 __global__ __launch_bounds__(kBlock) void k_stage_fu_nodes(const QueryDesc* __restrict__ qdp, Pools P, uint32_t tree,
                                                            const float* __restrict__ child,
                                                            const int32_t* __restrict__ childParent,
-                                                           const uint8_t* __restrict__ fnext, uint32_t nC)
+                                                           const uint8_t* __restrict__ fnext, uint32_t nC,
+                                                           const int32_t* __restrict__ valid)
 {
     const QueryDesc& qd = *qdp;
     const uint32_t i    = blockIdx.x * kBlock + threadIdx.x;
     const uint32_t cap  = qd.cap;
     int ix, iy, iz;
+    if(i < (uint32_t)qd.R1) P.cnt[region_slot(i, qd.regShift)] = (uint64_t)(uint32_t)valid[i] << 32;
     if(i < tree)
         P.r1node[i] = region_of(qd, P.treeS[i], P.treeS[(size_t)cap + i], P.treeS[2 * (size_t)cap + i], ix, iy, iz);
     if(i >= nC) return;
@@ -2790,7 +2837,7 @@ hipError_t launch_init_one(const QueryDesc& qd, QueryDesc* dq, QueryState* sts, 
                            const float* rows, hipStream_t s)
 {
     // about 4 K words to clear per clearing workgroup
-    const uint32_t words = 3u * (uint32_t)qd.R1 + 2u * (uint32_t)qd.R2words + 9u * (qd.nChunks + 1u);
+    const uint32_t words = (48u << qd.regShift) + 2u * (uint32_t)qd.R2words + 9u * (qd.nChunks + 1u);
     const uint32_t clear = std::min(32u, std::max(1u, (words + 4095u) / 4096u));
     if(qd.masks)
         hipLaunchKernelGGL(k_init_one<true>, dim3(1 + clear), dim3(kBlock), 0, s, qd, dq, sts, P, W, rows);
@@ -2961,12 +3008,13 @@ hipError_t launch_stage_propagate_planner(int model, const QueryDesc* qd, const 
 }
 
 hipError_t launch_stage_frontier_update(const QueryDesc* qd, QueryState* st, const Pools& P, const WorkLists& W,
-                                        uint32_t itr, uint32_t tree, const float* child, const int32_t* childParent,
-                                        const uint8_t* fnext, uint32_t nC, int32_t* info, hipStream_t s)
+                                        uint32_t R1, uint32_t itr, uint32_t tree, const float* child,
+                                        const int32_t* childParent, const uint8_t* fnext, uint32_t nC,
+                                        const int32_t* valid, int32_t* info, hipStream_t s)
 {
-    const uint32_t n = tree > nC ? tree : nC;
-    if(n) hipLaunchKernelGGL(k_stage_fu_nodes, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, qd, P, tree, child,
-                             childParent, fnext, nC);
+    const uint32_t n = std::max(std::max(tree, nC), R1);
+    hipLaunchKernelGGL(k_stage_fu_nodes, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, qd, P, tree, child,
+                       childParent, fnext, nC, valid);
     hipLaunchKernelGGL(k_stage_fu_state, dim3(1), dim3(kBlock), 0, s, qd, st, P, W, itr, tree, nC);
     Launch L;
     L.chunkGrid = 256;

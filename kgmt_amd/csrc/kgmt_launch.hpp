@@ -69,12 +69,13 @@ hipError_t launch_stage_propagate_planner(int model, const QueryDesc* qd, const 
                                           float* child, uint8_t* valid, int32_t* r1, int32_t* r2, uint8_t* check,
                                           float* box, hipStream_t s);
 // frontier update of one iteration on a one-query pool (the caller's tree
-// already in P.treeS / parent / cost / frontier, region counts and scores in
-// P.validc / P.score): staging kernels, then the planner's k_update;
+// already in P.treeS / parent / cost / frontier, the scores in P.score; valid:
+// its R1 valid counts): staging kernels, then the planner's k_update;
 // info[4] = {appended, multiset size, goal node or -1, re-activated}
 hipError_t launch_stage_frontier_update(const QueryDesc* qd, QueryState* st, const Pools& P, const WorkLists& W,
-                                        uint32_t itr, uint32_t tree, const float* child, const int32_t* childParent,
-                                        const uint8_t* fnext, uint32_t nC, int32_t* info, hipStream_t s);
+                                        uint32_t R1, uint32_t itr, uint32_t tree, const float* child,
+                                        const int32_t* childParent, const uint8_t* fnext, uint32_t nC,
+                                        const int32_t* valid, int32_t* info, hipStream_t s);
 hipError_t launch_stage_region_update(const QueryDesc* qd, const int32_t* r1, const int32_t* r2, const uint8_t* valid,
                                       const float* ufront, uint32_t n, const float* score, const uint32_t* actPrev,
                                       uint32_t* actNext, int32_t* total, int32_t* validc, uint8_t* fnext,
