@@ -73,6 +73,7 @@ struct QueryDesc
     uint32_t rowOff;                 // first obstacle row (2 * wdim floats) of the query in the scene's source rows
     uint32_t masks;                  // the scene has box masks (the query's tiles run the mask check)
     int32_t wdim;                    // workspace dimension W_DIM: 2 (planar: x y, z = 0) or 3
+    uint32_t hostPathOff;            // float offset in a batch's host-mapped path rows (min(max_iter+2, kWaveRows)*D)
 };
 
 // Where a region's counter lies: consecutive regions go to different 128-byte
@@ -108,6 +109,9 @@ __host__ __device__ constexpr uint32_t region_word(uint32_t r, uint32_t shift, u
 {
     return (actW <= 2u ? region_slot(r, shift) : r) * actW;
 }
+
+// path rows that one wave writes together (walk_path_wave)
+constexpr uint32_t kWaveRows = 64;
 
 // words of a flagged-child row: parent and grandparent indices + D sample
 // words, padded to whole float4s

@@ -166,6 +166,7 @@ int dev_alloc(T*& p, size_t count, std::vector<void*>& owned)
 // bound, 21.3 never, 20.5 always.
 constexpr uint32_t kRefill = 1u << 17;
 constexpr size_t kHostPathFloats = size_t(1) << 20;  // host-mapped path rows of a single query (4 MiB)
+constexpr size_t kHostPoolFloats = size_t(1) << 22;  // host-mapped path rows of a batch (16 MiB)
 // launch units the host stays ahead of the GPU: one for a plan's first
 // kLongAfter iterations (every launch is queued while the one before runs,
 // and a plan that finishes leaves one unit behind), two after them (a plan
@@ -259,6 +260,12 @@ struct Engine
     bool counterDirty = false;  // W.counter may be non-zero (a plan did not complete)
     HostResult* hostRes = nullptr;  // host-mapped result of a single-query plan
     float* hostPath     = nullptr;  // host-mapped path rows of that plan
+    // Host-mapped rows of a batch's paths, the first kWaveRows of each (null:
+    // more than kHostPoolFloats): the last kernel of a plan writes them, so
+    // that reading a path is a memory copy on the host (from the device it was
+    // 16 us a path, 6.8 of 36 ms with the 425 paths of 512 queries; now 3).
+    float* hostPaths  = nullptr;
+    float* dHostPaths = nullptr;  // its device address
     uint32_t maxPairs = 0;   // largest per-query scene (pairs) of the current plan
     int model       = -1;    // common model or -1
     uint32_t maxIter = 0;
@@ -297,6 +304,7 @@ struct Engine
         if(pinned) (void)hipHostFree(pinned);
         if(hostRes) (void)hipHostFree(hostRes);
         if(hostPath) (void)hipHostFree(hostPath);
+        if(hostPaths) (void)hipHostFree(hostPaths);
         for(void* p : owned) (void)hipFree(p);
         if(ownStream && stream) (void)hipStreamDestroy(stream);
     }
@@ -309,7 +317,7 @@ struct Engine
         HIP_TRY(hipGetDevice(&device));
         nq = n;
         if(!hq.resize(n) || !hs.resize(n)) return fail(KGMT_E_NOMEM, "pinned host allocation failed");
-        uint64_t samples = 0, rows = 0, nodes = 0, paths = 0;
+        uint64_t samples = 0, rows = 0, nodes = 0, paths = 0, hostRows = 0;
         uint32_t chunks = 0, regs = 0, subs = 0;
         model = cfgs[0].model;
         for(uint32_t q = 0; q < n; ++q)
@@ -325,6 +333,7 @@ struct Engine
                 qd.regOff    = regs;
                 qd.subOff    = subs;
                 qd.pathOff   = (uint32_t)paths;
+                qd.hostPathOff = (uint32_t)std::min<uint64_t>(hostRows, kHostPoolFloats);
                 samples += (uint64_t)qd.D * qd.cap;
                 rows += (uint64_t)row_words(qd.D) * qd.cap;
                 nodes += ((uint64_t)qd.cap + kNodeAlign - 1) / kNodeAlign * kNodeAlign;
@@ -332,6 +341,7 @@ struct Engine
                 regs += 16u << qd.regShift;
                 subs += (uint32_t)qd.R2words;
                 paths += (uint64_t)(cfgs[q].max_iter + 2) * qd.D;
+                hostRows += (uint64_t)std::min<uint32_t>(cfgs[q].max_iter + 2, kWaveRows) * qd.D;
                 if(paths > 0xffffffffull) return fail(KGMT_E_CAPACITY, "path pool too large");
                 if(cfgs[q].model != model) model = -1;
                 if(qd.wdim != hq[0].wdim)
@@ -378,6 +388,11 @@ struct Engine
                 HIP_TRY(hipHostGetDevicePointer((void**)&W.result, hostRes, 0));
                 HIP_TRY(hipHostMalloc((void**)&hostPath, pathFloats * sizeof(float), hipHostMallocMapped));
                 HIP_TRY(hipHostGetDevicePointer((void**)&W.hostPath, hostPath, 0));
+            }
+        else if(hostRows <= kHostPoolFloats)
+            {
+                HIP_TRY(hipHostMalloc((void**)&hostPaths, hostRows * sizeof(float), hipHostMallocMapped));
+                HIP_TRY(hipHostGetDevicePointer((void**)&dHostPaths, hostPaths, 0));
             }
         // launch shape: persistent workgroups sized to the device
         hipDeviceProp_t prop;
@@ -663,7 +678,7 @@ struct Engine
                 itersRun     = std::min(it, maxIter);
                 return device_error();
             }
-        HIP_TRY(launch_paths(dq, ds, P, nq, stream));
+        HIP_TRY(launch_paths(dq, ds, P, nq, dHostPaths, stream));
         HIP_TRY(hipMemcpyAsync(hs.data(), ds, sizeof(QueryState) * nq, hipMemcpyDeviceToHost, stream));
         HIP_TRY(hipStreamSynchronize(stream));
         counterDirty = false;
@@ -737,7 +752,7 @@ struct Engine
         if(all || stepItr >= maxIter)
             {
                 // goal paths of solved queries (a single query has walked its own)
-                HIP_TRY(launch_paths(dq, ds, P, nq, stream));
+                HIP_TRY(launch_paths(dq, ds, P, nq, dHostPaths, stream));
                 HIP_TRY(hipMemcpyAsync(hs.data(), ds, sizeof(QueryState) * nq, hipMemcpyDeviceToHost, stream));
                 HIP_TRY(hipStreamSynchronize(stream));
                 if(hostRes && hs[0].success && hostRes->pathRows) hs[0].pathRows = hostRes->pathRows;
@@ -815,24 +830,34 @@ struct Engine
 
     int get_tree(uint32_t q, float* samples, int32_t* parents, float* costs, uint32_t cap, uint32_t* n)
     {
-        HIP_TRY(hipStreamSynchronize(stream));  // a plan returns before its trailing launches drain
         const QueryDesc& qd = hq[q];
         const uint32_t ts   = hs[q].treeSize;
         if(n) *n = ts;
-        if(!samples && !parents && !costs) return KGMT_OK;
-        if(cap < ts) return fail(KGMT_E_CAPACITY, "tree output buffer too small");
-        if(samples)
+        if(!samples && !parents && !costs)
             {
-                std::vector<float> soa((size_t)qd.D * ts);
-                for(int d = 0; d < qd.D; ++d)
-                    HIP_TRY(hipMemcpy(soa.data() + (size_t)d * ts, P.treeS + qd.sampleOff + (size_t)d * qd.cap,
-                                      sizeof(float) * ts, hipMemcpyDeviceToHost));
-                for(uint32_t i = 0; i < ts; ++i)
-                    for(int d = 0; d < qd.D; ++d) samples[(size_t)i * qd.D + d] = soa[(size_t)d * ts + i];
+                HIP_TRY(hipStreamSynchronize(stream));  // a plan returns before its trailing launches drain
+                return KGMT_OK;
             }
-        if(parents)
-            HIP_TRY(hipMemcpy(parents, P.parent + qd.nodeOff, sizeof(int32_t) * ts, hipMemcpyDeviceToHost));
-        if(costs) HIP_TRY(hipMemcpy(costs, P.cost + qd.nodeOff, sizeof(float) * ts, hipMemcpyDeviceToHost));
+        if(cap < ts) return fail(KGMT_E_CAPACITY, "tree output buffer too small");
+        // rows made on the device, in the flagged-child rows of the plan's last
+        // iteration (wider than D floats and dead between iterations), so that
+        // they leave in one copy: 43601 nodes of 10 floats with parents and
+        // costs 208 us, 340 as one copy per dimension transposed on the host
+        float* rows  = P.childR + qd.rowOffC;
+        hipError_t e = hipSuccess;
+        auto copy    = [&](void* to, const void* from, size_t bytes) {
+            if(to && e == hipSuccess) e = hipMemcpyAsync(to, from, bytes, hipMemcpyDeviceToHost, stream);
+        };
+        if(samples)
+            e = launch_tree_rows(P.treeS + qd.sampleOff, nullptr, nullptr, qd.cap, ts, qd.D, ts, rows, nullptr, nullptr,
+                                 stream);
+        copy(samples, rows, sizeof(float) * qd.D * ts);
+        copy(parents, P.parent + qd.nodeOff, sizeof(int32_t) * ts);
+        copy(costs, P.cost + qd.nodeOff, sizeof(float) * ts);
+        // (also after an error: no copy into the caller's memory stays in flight)
+        const hipError_t w = hipStreamSynchronize(stream);
+        HIP_TRY(e);
+        HIP_TRY(w);
         return KGMT_OK;
     }
 
@@ -849,7 +874,7 @@ struct Engine
         if(!mirValid)
             {
                 HIP_TRY(launch_tree_rows(P.treeS + qd.sampleOff, P.parent + qd.nodeOff, P.cost + qd.nodeOff, qd.cap,
-                                         qd.D, ts, mirRows, mirPar, mirCost, stream));
+                                         qd.cap, qd.D, ts, mirRows, mirPar, mirCost, stream));
                 HIP_TRY(hipStreamSynchronize(stream));
                 mirValid = true;
             }
@@ -877,8 +902,14 @@ struct Engine
                 std::memcpy(rows, (const void*)hostPath, sizeof(float) * r * qd.D);
                 return KGMT_OK;
             }
+        // the first rows from host memory (the plan waited for the kernel that
+        // wrote them)
+        const uint32_t h = hostPaths ? std::min(r, kWaveRows) : 0u;
+        if(h) std::memcpy(rows, hostPaths + qd.hostPathOff, sizeof(float) * h * qd.D);
+        if(h == r) return KGMT_OK;
         HIP_TRY(hipStreamSynchronize(stream));  // a plan returns before its trailing launches drain
-        HIP_TRY(hipMemcpy(rows, P.path + qd.pathOff, sizeof(float) * r * qd.D, hipMemcpyDeviceToHost));
+        HIP_TRY(hipMemcpy(rows + (size_t)h * qd.D, P.path + qd.pathOff + (size_t)h * qd.D,
+                          sizeof(float) * (r - h) * qd.D, hipMemcpyDeviceToHost));
         return KGMT_OK;
     }
 };

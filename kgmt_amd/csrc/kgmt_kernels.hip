@@ -1243,11 +1243,13 @@ __device__ __forceinline__ void static_for(F&& f)
 
 // goal -> root rows of a solved query by one wave (every lane): the chain is
 // followed six levels per round of loads (parent, grandparent and the
-// ancestors at 3..6), lane l takes the row of the l-th node, and up to 64 rows
-// go out together; cost and length (of the edge durations and of the segments
-// between node positions) are summed in walk order.
-__device__ __forceinline__ void walk_path_wave(const QueryDesc& qd, QueryState& st, const Pools& P,
-                                               float* __restrict__ out, int32_t goal)
+// ancestors at 3..6), lane l takes the row of the l-th node, and kWaveRows rows
+// go out together, the first ones to `first`, those after them to `out` (both
+// as if they held the whole path); cost and length (of the edge durations and
+// of the segments between node positions) are summed in walk order. stage:
+// null, or LDS for kWaveRows rows, through which they go out as whole lines.
+__device__ __forceinline__ void walk_path_wave(const QueryDesc& qd, QueryState& st, const Pools& P, float* first,
+                                               float* out, float* stage, int32_t goal)
 {
     const uint32_t lane    = lane_id();
     const uint32_t cap     = qd.cap;
@@ -1262,7 +1264,7 @@ __device__ __forceinline__ void walk_path_wave(const QueryDesc& qd, QueryState& 
     float pc = 0.0f, pl = 0.0f, px = 0.0f, py = 0.0f, pz = 0.0f;
     while(true)
         {
-            const uint32_t lim = maxRows - rows < 64u ? maxRows - rows : 64u;
+            const uint32_t lim = maxRows - rows < kWaveRows ? maxRows - rows : kWaveRows;
             int32_t mine = lane == 0 ? head : -1;  // this lane's node
             int32_t f    = head;                    // the last node found
             uint32_t cnt = 1;                       // nodes found
@@ -1296,10 +1298,18 @@ __device__ __forceinline__ void walk_path_wave(const QueryDesc& qd, QueryState& 
             const uint32_t node = mine < 0 ? (uint32_t)f : (uint32_t)mine;
             static_for<KGMT_MAX_SAMPLE>([&](auto K) { r[K] = T[(size_t)(K < D ? K : 0) * cap + node]; });
             const float dn = T[(size_t)(D - 1) * cap + node];
+            float* to = rows == 0u ? first : out + rows * D;
             if(lane < cnt)
                 static_for<KGMT_MAX_SAMPLE>([&](auto K) {
-                    if(K < D) out[(rows + lane) * D + K] = r[K];
+                    if(K < D) (stage ? stage : to)[lane * D + K] = r[K];
                 });
+            if(stage)
+                {
+                    // (one wave: its LDS writes come before its reads)
+                    __builtin_amdgcn_wave_barrier();
+                    for(uint32_t i = lane; i < cnt * (uint32_t)D; i += 64u) to[i] = stage[i];
+                    __builtin_amdgcn_wave_barrier();
+                }
             // segment length from the row before (lane l - 1, or the last of
             // the rows before) to this one
             float qx = __shfl_up(r[0], 1, 64), qy = __shfl_up(r[1], 1, 64), qz = __shfl_up(r[2], 1, 64);
@@ -2002,7 +2012,7 @@ __device__ __forceinline__ void update_job(const UpdateArgs& A0, uint32_t q, uin
     // into host memory before its first lane publishes the result
     if(nq == 1 && jobGoal != kLbNone && goalBefore == kLbNone && W.result != nullptr && threadIdx.x < 64 &&
        st.pathRows == 0u)
-        walk_path_wave(qd, st, P, W.hostPath, (int32_t)jobGoal);
+        walk_path_wave(qd, st, P, W.hostPath, W.hostPath, nullptr, (int32_t)jobGoal);
     // The last job's look-back has seen a word of every other job, each
     // published after that job read the chunk counts: they start at zero
     // again for the next propagate.
@@ -2108,15 +2118,19 @@ __global__ __launch_bounds__(kBlock) void k_finish(const QueryDesc* __restrict__
 // per query (512 mixed queries: 40.4 us with one thread per query and two
 // levels a round)
 // ---------------------------------------------------------------------------
+// hostPaths: the host-mapped pool of the first kWaveRows rows of every path,
+// which the host reads without a copy (null: all rows go to the device pool)
 __global__ __launch_bounds__(64) void k_paths(const QueryDesc* __restrict__ qds, QueryState* __restrict__ sts,
-                                              Pools P, uint32_t nq)
+                                              Pools P, uint32_t nq, float* __restrict__ hostPaths)
 {
+    __shared__ float stage[kWaveRows * KGMT_MAX_SAMPLE];
     const uint32_t q = blockIdx.x;
     QueryState& st   = sts[q];
     if(threadIdx.x == 0) commit_state(st);  // the closed last iteration
     if(!st.successN || st.pathRows) return;
     const QueryDesc& qd = qds[q];
-    walk_path_wave(qd, st, P, P.path + qd.pathOff, st.goalIdx);
+    float* rows         = P.path + qd.pathOff;
+    walk_path_wave(qd, st, P, hostPaths ? hostPaths + qd.hostPathOff : rows, rows, stage, st.goalIdx);
 }
 
 // ---------------------------------------------------------------------------
@@ -2362,14 +2376,15 @@ __global__ __launch_bounds__(kBlock) void k_build_scene(const float* __restrict_
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(kBlock) void k_tree_rows(const float* __restrict__ treeS,
                                                       const int32_t* __restrict__ parent,
-                                                      const float* __restrict__ cost, uint32_t cap, int D,
+                                                      const float* __restrict__ cost, uint32_t cap, uint32_t n, int D,
                                                       uint32_t treeSize, float* __restrict__ rows,
                                                       int32_t* __restrict__ parents, float* __restrict__ costs)
 {
     const uint32_t i = blockIdx.x * kBlock + threadIdx.x;
-    if(i >= cap) return;
+    if(i >= n) return;
     const bool in = i < treeSize;
     for(int d = 0; d < D; ++d) rows[(size_t)i * D + d] = in ? treeS[(size_t)d * cap + i] : 0.0f;
+    if(!parents) return;
     parents[i] = in ? parent[i] : -1;
     costs[i]   = in ? cost[i] : 0.0f;
 }
@@ -2925,18 +2940,19 @@ hipError_t launch_finish(const QueryDesc* qds, QueryState* sts, const WorkLists&
     return hipGetLastError();
 }
 
-hipError_t launch_paths(const QueryDesc* qds, QueryState* sts, const Pools& P, uint32_t nq, hipStream_t s)
+hipError_t launch_paths(const QueryDesc* qds, QueryState* sts, const Pools& P, uint32_t nq, float* hostPaths,
+                        hipStream_t s)
 {
     if(nq == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_paths, dim3(nq), dim3(64), 0, s, qds, sts, P, nq);
+    hipLaunchKernelGGL(k_paths, dim3(nq), dim3(64), 0, s, qds, sts, P, nq, hostPaths);
     return hipGetLastError();
 }
 
-hipError_t launch_tree_rows(const float* treeS, const int32_t* parent, const float* cost, uint32_t cap, int D,
-                            uint32_t treeSize, float* rows, int32_t* parents, float* costs, hipStream_t s)
+hipError_t launch_tree_rows(const float* treeS, const int32_t* parent, const float* cost, uint32_t cap, uint32_t n,
+                            int D, uint32_t treeSize, float* rows, int32_t* parents, float* costs, hipStream_t s)
 {
-    if(cap == 0) return hipSuccess;
-    hipLaunchKernelGGL(k_tree_rows, dim3((cap + kBlock - 1) / kBlock), dim3(kBlock), 0, s, treeS, parent, cost, cap,
+    if(n == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_tree_rows, dim3((n + kBlock - 1) / kBlock), dim3(kBlock), 0, s, treeS, parent, cost, cap, n,
                        D, treeSize, rows, parents, costs);
     return hipGetLastError();
 }

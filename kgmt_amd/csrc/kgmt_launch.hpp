@@ -47,12 +47,15 @@ hipError_t launch_update(const QueryDesc* qds, QueryState* sts, const Pools& P, 
                          uint32_t parity, const Launch& L, bool own, hipStream_t s);
 hipError_t launch_finish(const QueryDesc* qds, QueryState* sts, const WorkLists& W, uint32_t parity, hipStream_t s);
 // goal paths of the solved queries, once a plan has ended
-hipError_t launch_paths(const QueryDesc* qds, QueryState* sts, const Pools& P, uint32_t nq, hipStream_t s);
+// goal paths of the solved queries; hostPaths: device address of the
+// host-mapped pool of path rows (null: none)
+hipError_t launch_paths(const QueryDesc* qds, QueryState* sts, const Pools& P, uint32_t nq, float* hostPaths,
+                        hipStream_t s);
 
-// a query's tree as rows of D floats, parents and costs (entries past the
-// tree: 0, -1, 0)
-hipError_t launch_tree_rows(const float* treeS, const int32_t* parent, const float* cost, uint32_t cap, int D,
-                            uint32_t treeSize, float* rows, int32_t* parents, float* costs, hipStream_t s);
+// the first n of a query's nodes as rows of D floats and, unless null, their
+// parents and costs (entries past the tree: 0, -1, 0)
+hipError_t launch_tree_rows(const float* treeS, const int32_t* parent, const float* cost, uint32_t cap, uint32_t n,
+                            int D, uint32_t treeSize, float* rows, int32_t* parents, float* costs, hipStream_t s);
 
 // stage-level kernels (one query, caller buffers)
 hipError_t launch_stage_draw(const QueryDesc* qd, int C, uint32_t query, uint32_t itr, uint32_t u0, uint32_t n,
