@@ -152,9 +152,9 @@ typedef struct kgmt_result {
  * around every launch of the plain, non-graph iteration loop). Kernel order:
  * 0 propagate, 1 update (region scores, tree append, re-activation, goal
  * test and next expansion list in one launch), 2 finish (closes the
- * iteration of every query and builds the next iteration's work lists; a
- * single-query context has no finish launch: its last update job does
- * that); slots 3 and 4 are unused. */
+ * iteration of every query and builds the next iteration's work lists; up to
+ * 256 queries have no finish launch: their last update jobs do that); slots
+ * 3 and 4 are unused. */
 #define KGMT_PROFILE_KERNELS 5
 typedef struct kgmt_profile {
     uint64_t launches[KGMT_PROFILE_KERNELS];

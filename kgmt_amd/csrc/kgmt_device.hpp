@@ -149,7 +149,7 @@ struct QueryState
     uint32_t finishItr;
     uint32_t pad[3];
     // The next iteration's values, written when an iteration closes (by the
-    // last update job of a single-query plan, by k_finish for a batch);
+    // query's last update job, by k_finish for more than kFewQueries queries);
     // propagate reads them and its first workgroup copies them to the fields
     // above (k_paths after the last iteration), which the update kernel reads.
     uint32_t itrN, treeSizeN, nChildrenN, perN, doneN, successN, finishItrN, padN;
@@ -211,11 +211,20 @@ struct HostResult
 // Work lists over queries, double-buffered by iteration parity: the kernels
 // of iteration i read buffer (i-1)&1 while the last finisher of that
 // iteration writes the other one. Prefix sums of nq + 1 entries each.
+// Most queries whose work lists every workgroup makes for itself: each query's
+// last update job leaves its tiles and jobs in one word, and a workgroup scans
+// the words into LDS (33 queries: k_propagate 16.6 to 16.2 us, k_update 10.6 to
+// 10.9, and k_finish's 4.3 are gone). More queries' lists are made by k_finish:
+// 256 words are one load of a propagate workgroup, 5.9 us are little beside an
+// iteration of that many, and the list would take LDS from the scene.
+constexpr uint32_t kFewQueries = 256;
+
 struct WorkLists
 {
-    uint32_t* tileStart;   // 2 x (nq + 1): propagate tiles
-    uint32_t* jobStart;    // 2 x (nq + 1): update jobs
-    uint32_t* active;      // 2: queries not done in each list
+    uint32_t* tileStart;   // 2 x (nq + 1): propagate tiles (more than kFewQueries queries)
+    uint32_t* jobStart;    // 2 x (nq + 1): update jobs (the same)
+    uint64_t* work;        // 2 x nq: a query's tiles (low word) and jobs (2 to kFewQueries queries)
+    uint32_t* ended;       // queries done in this plan (2 to kFewQueries queries)
     uint32_t* counter;     // arrivals of k_init's workgroups (the last builds the first work lists)
     uint32_t* tileClaim;   // 2 (by parity): propagate tiles taken past the first of each workgroup
     uint32_t* claim;       // 2 (by parity): update jobs taken in a launch (the launch before zeroes it)
@@ -230,6 +239,9 @@ struct WorkLists
     uint32_t quads;        // 1 when a query is a quadcopter's
     uint32_t refill;       // children from which a quadcopter query's tiles hold twice as many (0: never)
 
+    uint32_t listOff;      // offset (4-byte words) of a propagate workgroup's list of tile starts in its dynamic LDS
+
+    __host__ __device__ __forceinline__ bool few() const { return nq > 1 && nq <= kFewQueries; }
     __device__ __forceinline__ const uint32_t* tiles(uint32_t parity) const { return tileStart + parity * (nq + 1); }
     __device__ __forceinline__ const uint32_t* jobs(uint32_t parity) const { return jobStart + parity * (nq + 1); }
 };
@@ -1608,19 +1620,22 @@ __device__ __forceinline__ uint32_t count_bits(const uint32_t* words, uint32_t s
     return cnt;
 }
 
-// index of the query owning global job t (prefix array of nq + 1 entries)
+// query of work item t, t < prefix[nq] (prefix sums of the queries' items; the
+// same for every lane, all of them active): the last query that starts at or
+// before t, 64 starts a round
 __device__ __forceinline__ uint32_t locate(const uint32_t* prefix, uint32_t nq, uint32_t t)
 {
-    uint32_t lo = 0, hi = nq;  // prefix[lo] <= t < prefix[hi]
-    while(hi - lo > 1)
+    const uint32_t lane = (uint32_t)__lane_id();
+    uint32_t lo = 0, n = nq;
+    while(true)
         {
-            const uint32_t mid = (lo + hi) >> 1;
-            if(prefix[mid] <= t)
-                lo = mid;
-            else
-                hi = mid;
+            const uint32_t step = (n + 63u) / 64u, at = lane * step;
+            const uint64_t m    = __ballot(at < n && prefix[lo + (at < n ? at : 0u)] <= t);
+            const uint32_t k    = ((uint32_t)__popcll(m) - 1u) * step;
+            lo += k;
+            if(step == 1u) return lo;
+            n = n - k < step ? n - k : step;
         }
-    return lo;
 }
 
 }  // namespace kgmt

@@ -361,7 +361,8 @@ struct Engine
            (rc = dev_alloc(P.score, regs, owned)) ||
            (rc = dev_alloc(P.actPrev, subs, owned)) || (rc = dev_alloc(P.actNext, subs, owned)) ||
            (rc = dev_alloc(P.path, paths, owned)) || (rc = dev_alloc(W.tileStart, 2 * (size_t)(n + 1), owned)) ||
-           (rc = dev_alloc(W.jobStart, 2 * (size_t)(n + 1), owned)) || (rc = dev_alloc(W.active, 2, owned)) ||
+           (rc = dev_alloc(W.jobStart, 2 * (size_t)(n + 1), owned)) || (rc = dev_alloc(W.work, 2 * (size_t)n, owned)) ||
+           (rc = dev_alloc(W.ended, 1, owned)) ||
            (rc = dev_alloc(W.counter, 1, owned)) || (rc = dev_alloc(W.claim, 2, owned)) || (rc = dev_alloc(W.tileClaim, 2, owned)) ||
            (rc = dev_alloc(W.closedDev, 1, owned)))
             return rc;
@@ -472,7 +473,7 @@ struct Engine
         return KGMT_OK;
     }
 
-    // One iteration: 2 launches for one query, 3 for a batch (k_finish).
+    // One iteration: 2 launches, 3 for more than kFewQueries queries (k_finish).
     // marks: timing events around them (profiling).
     int enqueue_iteration(uint32_t parity, hipEvent_t* marks = nullptr)
     {
@@ -482,8 +483,8 @@ struct Engine
         if(marks) HIP_TRY(hipEventRecord(marks[1], stream));
         HIP_TRY(launch_update(dq, ds, P, W, parity, L, true, stream));
         if(all) HIP_TRY(hipEventRecord(marks[2], stream));
-        // a single query's last update job closes the iteration itself
-        if(nq > 1)
+        // the last update jobs of one query or a few close the iteration
+        if(nq > kFewQueries)
             {
                 HIP_TRY(launch_finish(dq, ds, W, parity, stream));
                 if(all) HIP_TRY(hipEventRecord(marks[3], stream));
@@ -511,9 +512,9 @@ struct Engine
         for(uint32_t it = 0; it < iters; ++it)
             {
                 hipEvent_t* m = &profEv[(size_t)it * (KGMT_PROFILE_KERNELS + 1)];
-                // propagate, update and (batches) finish; the last two
+                // propagate, update and (many queries) finish; the last two
                 // profile slots stay unused
-                const int nk = profiling > 1 ? (nq > 1 ? 3 : 2) : 1;
+                const int nk = profiling > 1 ? (nq > kFewQueries ? 3 : 2) : 1;
                 for(int k = 0; k < nk; ++k)
                     {
                         float ms = 0.0f;
@@ -595,8 +596,9 @@ struct Engine
         if(hostRes) hostRes->iterations = 0;
         bool published = false;
         auto seen      = [&]() { return early && __atomic_load_n(pinned, __ATOMIC_ACQUIRE) != 0; };
-        // The closing job of every iteration (k_finish for a batch) writes the
-        // number of iterations closed so far into host-mapped memory; the host
+        // The closing job of every iteration (for a few queries the next
+        // propagate, for many k_finish) writes the number of iterations
+        // closed so far into host-mapped memory; the host
         // stays at most kLag launch units ahead of it. No event between the
         // units: an event record is a system-scope release on the stream.
         iterMs.assign(maxIter + 2, 0.0);
@@ -1568,7 +1570,7 @@ int kgmt_frontier_update(const kgmt_config* cfg, uint32_t itr, uint32_t tree_siz
        (rc = a.get(P.fnext, nodes)) || (rc = a.get(P.react, nodes)) || (rc = a.get(P.repIdx, nodes)) ||
        (rc = a.get(P.partA, h.nChunks + 1)) || (rc = a.get(P.look, 4 * ((size_t)h.nChunks + 1))) ||
        (rc = a.get(P.cnt, 16u << h.regShift)) || (rc = a.get(P.score, h.R1)) || (rc = a.get(W.tileStart, 4)) ||
-       (rc = a.get(W.jobStart, 4)) || (rc = a.get(W.active, 2)) || (rc = a.get(W.counter, 1)) ||
+       (rc = a.get(W.jobStart, 4)) || (rc = a.get(W.counter, 1)) ||
        (rc = a.get(W.claim, 2)) || (rc = a.get(W.allDone, 1)) || (rc = a.get(W.error, 1)) ||
        (rc = a.get(W.closed, 1)) || (rc = a.get(W.closedDev, 1)))
         return rc;

@@ -1,7 +1,7 @@
 // kgmt_kernels.hip — HIP kernels of the KGMT per-iteration expansion path (gfx950).
 //
-// One iteration of the planner is three launches over a table of queries, two
-// for a single query (its last k_update job does k_finish's work):
+// One iteration of the planner is two launches over a table of queries, three
+// over more than 256:
 //   k_propagate  persistent over tiles of children: Philox draws, per-wave
 //                sort by step count, RK4 rollout, AABB test against the
 //                obstacles staged in LDS (candidate boxes per wave), region
@@ -17,7 +17,7 @@
 //                and goal test, and the next expansion list (segmented
 //                repeat) at offsets found by a decoupled look-back.
 //                (Graph.cu:207-358, KGMT.cu:170-181, 305-403, Planner.cu:52-80)
-//   k_finish     (batches) one workgroup: closes the iteration of every query (tree
+//   k_finish     (more than 256 queries) one workgroup: closes the iteration of every query (tree
 //                size, stop rules, next launch regime; KGMT.cu:84-95, 183-201,
 //                399-402) and builds the next iteration's work lists.
 // Per plan: k_init (scene build and first iteration's state) before the first
@@ -347,10 +347,66 @@ __device__ void build_worklists(const QueryDesc* __restrict__ qds, const QuerySt
         {
             tileStart[nq]     = carryT;
             jobStart[nq]      = carryJ;
-            W.active[parity]  = carryA;
             *W.counter        = 0;
             __hip_atomic_store(W.allDone, carryA == 0 ? 1u : 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
         }
+}
+
+// One more iteration closed in this plan: the count for the host, which
+// stays a few launch units ahead of it (one thread per iteration: the closing
+// job of a single query, k_finish for many queries)
+__device__ __forceinline__ void count_closed(const WorkLists& W)
+{
+    const uint32_t n = *W.closedDev + 1u;
+    *W.closedDev     = n;
+    __hip_atomic_store(W.closed, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// The same for a few queries, whose iterations no one thread closes: the next
+// propagate counts the one before it as it starts.
+__device__ __forceinline__ void count_started(const WorkLists& W)
+{
+    const uint32_t n = *W.closedDev;
+    *W.closedDev     = n + 1u;
+    __hip_atomic_store(W.closed, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Tiles and jobs of a query's next iteration as one word (0 once it is done).
+__device__ __forceinline__ uint64_t query_work(const QueryDesc& qd, const QueryState& st, const WorkLists& W)
+{
+    if(st.doneN) return 0ull;
+    const uint32_t nc = st.nChildrenN, tr = st.treeSizeN, tc = tile_children(qd, W, nc);
+    return (uint64_t)((nc + kChunk - 1) / kChunk + (tr + kChunk - 1) / kChunk) << 32 | (nc + tc - 1) / tc;
+}
+
+// Starts of the queries' items (tiles: shift 0, jobs: 32) into list (nq + 1
+// words of LDS) by a block of NT threads; returns their number.
+template <int NT>
+__device__ __forceinline__ uint32_t few_starts(const WorkLists& W, uint32_t parity, uint32_t shift, uint32_t* list,
+                                               uint32_t* sbuf)
+{
+    constexpr uint32_t I = kFewQueries > NT ? kFewQueries / NT : 1;
+    const uint32_t nq    = W.nq;
+    const uint64_t* work = W.work + parity * nq;
+    uint32_t v[I], sum = 0;
+#pragma unroll
+    for(uint32_t i = 0; i < I; ++i)
+        {
+            const uint32_t q = threadIdx.x * I + i;
+            v[i]             = q < nq ? (uint32_t)(work[q] >> shift) : 0u;
+            sum += v[i];
+        }
+    uint32_t tot;
+    uint32_t at = block_excl_scan<NT>(sum, sbuf, tot);
+#pragma unroll
+    for(uint32_t i = 0; i < I; ++i)
+        {
+            const uint32_t q = threadIdx.x * I + i;
+            if(q < nq) list[q] = at;
+            at += v[i];
+        }
+    __syncthreads();
+    return tot;
 }
 
 // Returns true in every thread of the last workgroup to arrive (all writes of
@@ -1085,10 +1141,35 @@ __global__ __launch_bounds__(NT, 4) void k_propagate(const QueryDesc* __restrict
     // the first workgroup commits the next-state fields (written when the
     // last iteration closed) to the current ones, which the update kernel
     // reads; propagate itself reads only the next-state fields
+    // (a done query's word for the iteration after the next stays empty)
+    const bool few = W.few();
     if(blockIdx.x == 0)
-        for(uint32_t q = threadIdx.x; q < nq; q += NT) commit_state(sts[q]);
-    const uint32_t* tileList = W.tiles(parity);
-    const uint32_t nTiles    = tileList[nq];
+        {
+            for(uint32_t q = threadIdx.x; q < nq; q += NT)
+                {
+                    commit_state(sts[q]);
+                    if(few && sts[q].doneN) W.work[(parity ^ 1u) * nq + q] = 0ull;
+                }
+            if(few && threadIdx.x == 0) count_started(W);
+        }
+    // the tiles: one query's straight from its state, a few queries' scanned
+    // by every workgroup, more queries' from the list
+    const uint32_t* starts = W.tiles(parity);
+    uint32_t nTiles;
+    if(nq == 1)
+        {
+            const uint32_t nc = sts[0].nChildrenN, tc = tile_children(qds[0], W, nc);
+            nTiles            = sts[0].doneN ? 0u : (nc + tc - 1) >> __builtin_ctz(tc);  // a power of two
+        }
+    else if(few)
+        {
+            __shared__ uint32_t sbuf[NT / 64];
+            uint32_t* list = reinterpret_cast<uint32_t*>(sObs) + W.listOff;
+            nTiles         = few_starts<NT>(W, parity, 0u, list, sbuf);
+            starts         = list;
+        }
+    else
+        nTiles = starts[nq];
     uint32_t staged          = 0xffffffffu;
     uint32_t fb              = 0;  // flag buffer of the next tile
     // the tables and both flag buffers start empty (each tile empties them
@@ -1113,7 +1194,8 @@ __global__ __launch_bounds__(NT, 4) void k_propagate(const QueryDesc* __restrict
                                                                                       __ATOMIC_RELAXED,
                                                                                       __HIP_MEMORY_SCOPE_AGENT)
                                                  : nTiles;
-            const uint32_t q    = locate(tileList, nq, t);
+            const uint32_t q     = nq == 1 ? 0u : locate(starts, nq, t);
+            const uint32_t first = nq == 1 ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane((int)starts[q]);
             if(sts[q].doneN)
                 {
                     if(claim) __syncthreads();
@@ -1129,7 +1211,7 @@ __global__ __launch_bounds__(NT, 4) void k_propagate(const QueryDesc* __restrict
                 if(model == KGMT_MODEL_QUADCOPTER)
                     {
                         const uint32_t tile = tile_children(qd, W, sts[q].nChildrenN);
-                        quad_tile<NT>(qd, sts[q], (t - tileList[q]) * tile, tile, P, sObs, L.quad, stage);
+                        quad_tile<NT>(qd, sts[q], (t - first) * tile, tile, P, sObs, L.quad, stage);
                         used = true;
                         continue;
                     }
@@ -1142,7 +1224,7 @@ __global__ __launch_bounds__(NT, 4) void k_propagate(const QueryDesc* __restrict
                             __syncthreads();
                             used = false;
                         }
-                    const uint32_t base = (t - tileList[q]) * (NT / K);
+                    const uint32_t base = (t - first) * (NT / K);
                     if constexpr(MODEL >= 0)
                         child_tile<MODEL, NT, K>(qd, sts[q], base, P, sObs, L.tile, fb, stage);
                     else
@@ -1199,33 +1281,6 @@ __device__ void finish_query(const QueryDesc& qd, QueryState& st, uint32_t R)
     st.doneN      = done;
     st.successN   = success;
     st.finishItrN = fin;
-}
-
-// One more iteration closed in this plan: the count for the host, which
-// stays a few launch units ahead of it (one thread per iteration: the closing
-// job of a single query, k_finish for a batch)
-__device__ __forceinline__ void count_closed(const WorkLists& W)
-{
-    const uint32_t n = *W.closedDev + 1u;
-    *W.closedDev     = n;
-    __hip_atomic_store(W.closed, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-}
-
-// Work lists of a single-query table for its next iteration (parity
-// buffer), from the next-state fields (one thread).
-template <bool QUADS>
-__device__ __forceinline__ void single_worklists(const QueryDesc& qd, const QueryState& st, const WorkLists& W,
-                                                 uint32_t parity)
-{
-    uint32_t* tileStart = W.tileStart + parity * 2;
-    uint32_t* jobStart  = W.jobStart + parity * 2;
-    const bool alive    = st.doneN == 0;
-    tileStart[0]        = 0;
-    jobStart[0]         = 0;
-    const uint32_t tc   = QUADS ? tile_children(qd, W, st.nChildrenN) : W.tile;
-    tileStart[1]        = alive ? (st.nChildrenN + tc - 1) / tc : 0u;
-    jobStart[1] = alive ? (st.nChildrenN + kChunk - 1) / kChunk + (st.treeSizeN + kChunk - 1) / kChunk : 0u;
-    W.active[parity] = alive ? 1u : 0u;
 }
 
 // f(0), .., f(N - 1) with constant indices from the start: an array that only
@@ -2031,7 +2086,8 @@ __device__ __forceinline__ void update_job(const UpdateArgs& A0, uint32_t q, uin
                 }
             // the last job knows the list size and the goal: it closes the
             // iteration of a single query (the next-state fields and work
-            // lists, read from the next kernel on), k_finish those of a batch
+            // lists, read from the next kernel on), and that of each of a few
+            // queries; k_finish those of more
             if(last)
                 {
                     const uint32_t R = before + total;
@@ -2040,10 +2096,16 @@ __device__ __forceinline__ void update_job(const UpdateArgs& A0, uint32_t q, uin
                     st.nAcc          = nAcc;
                     st.next          = next;
                     st.fAccept       = faccept(qd, st.itr, tree, next);
+                    if(W.few())
+                        {
+                            finish_query(qd, st, R);
+                            W.work[(parity ^ 1u) * nq + q] = query_work(qd, st, W);
+                            if(st.doneN && atomicAdd(W.ended, 1u) == nq - 1u)
+                                __hip_atomic_store(W.allDone, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+                        }
                     if(nq == 1)
                         {
                             finish_query(qd, st, R);
-                            single_worklists<QUADS>(qd, st, W, parity ^ 1u);
                             count_closed(W);
                             if(st.doneN && !st.successN)
                                 {
@@ -2066,13 +2128,21 @@ __global__ __launch_bounds__(kUpd) void k_update(UpdateArgs)
     QueryState* __restrict__ sts      = A.sts;
     const uint32_t parity             = A.parity;
     const uint32_t nq       = W.nq;
-    const uint32_t* jobList = W.jobs(parity);
-    // one query: its jobs 0 .. nJ-1 straight from its state (the list holds
-    // the same), without waiting for the list first
+    // the jobs: one query's straight from its state, a few queries' scanned by
+    // every workgroup, more queries' from the list
+    __shared__ uint32_t list[kFewQueries + 1];
     const QueryState& st0 = sts[0];
-    const uint32_t nJobs  = nq > 1 ? jobList[nq]
-                            : st0.done ? 0u
-                                       : (st0.treeSize + kChunk - 1) / kChunk + (st0.nChildren + kChunk - 1) / kChunk;
+    const uint32_t* starts = W.jobs(parity);
+    uint32_t nJobs;
+    if(nq == 1)
+        nJobs = st0.done ? 0u : (st0.treeSize + kChunk - 1) / kChunk + (st0.nChildren + kChunk - 1) / kChunk;
+    else if(W.few())
+        {
+            nJobs  = few_starts<kUpd>(W, parity, 32u, list, L.sbuf);
+            starts = list;
+        }
+    else
+        nJobs = starts[nq];
     // with no more jobs than workgroups, workgroup j does job j; with more,
     // every job comes from the counter (the other parity's counter starts at
     // zero for the next launch)
@@ -2090,9 +2160,10 @@ __global__ __launch_bounds__(kUpd) void k_update(UpdateArgs)
                     j = L.job;
                     if(j >= nJobs) return;
                 }
-            const uint32_t q = nq > 1 ? (uint32_t)__builtin_amdgcn_readfirstlane((int)locate(jobList, nq, j)) : 0u;
+            const uint32_t q     = nq == 1 ? 0u : locate(starts, nq, j);
+            const uint32_t first = nq == 1 ? 0u : (uint32_t)__builtin_amdgcn_readfirstlane((int)starts[q]);
             // (a stale list entry of a finished query has nothing to do)
-            if(!sts[q].done) update_job<QUADS>(A, q, nq > 1 ? j - jobList[q] : j, L);
+            if(!sts[q].done) update_job<QUADS>(A, q, j - first, L);
             if(!more) return;
             __syncthreads();  // L is rewritten by the next job
         }
@@ -2331,6 +2402,13 @@ __global__ __launch_bounds__(kBlock) void k_init(const QueryDesc* __restrict__ q
     root_query(qd, sts[q], P);
     if(q == 0 && threadIdx.x < 2) W.claim[threadIdx.x] = W.tileClaim[threadIdx.x] = 0u;
     if(q == 0 && threadIdx.x == 0) *W.closedDev = 0u;
+    if(q == 0 && threadIdx.x == 0) *W.ended = 0u;
+    if(W.few())
+        {
+            // (the first thread wrote the state)
+            if(threadIdx.x == 0) W.work[q] = query_work(qd, sts[q], W);
+            return;
+        }
     if(last_arrival(W.counter, nq, &sflag)) build_worklists<kBlock>(qds, sts, W, 0, sbuf);
 }
 
@@ -2353,12 +2431,7 @@ __global__ __launch_bounds__(kBlock) void k_init_one(const QueryDesc qd, QueryDe
     if(rows && qd.nObs) build_query_scene<MASKS>(qd, rows, P, L);
     root_query(qd, sts[0], P);
     if(threadIdx.x < 2) W.claim[threadIdx.x] = W.tileClaim[threadIdx.x] = 0u;
-    // the first thread wrote the state: it builds the first work lists
-    if(threadIdx.x == 0)
-        {
-            *W.closedDev = 0u;
-            single_worklists<MASKS>(qd, sts[0], W, 0u);
-        }
+    if(threadIdx.x == 0) *W.closedDev = 0u;
 }
 
 template <int W>
@@ -2700,12 +2773,6 @@ __global__ __launch_bounds__(kBlock) void k_stage_fu_state(const QueryDesc* __re
     for(uint32_t i = 0; i < jobs; ++i) P.look[i] = 0ull;  // parity 0's words
     W.claim[0] = W.claim[1] = 0u;
     *W.error   = 0u;
-    for(uint32_t par = 0; par < 2; ++par)
-        {
-            W.jobStart[2 * par] = 0, W.jobStart[2 * par + 1] = jobs;
-            W.tileStart[2 * par] = 0, W.tileStart[2 * par + 1] = 0;
-            W.active[par] = 1;
-        }
 }
 
 // info[4] = {appended, expansion multiset size, goal node or -1, re-activated}
@@ -2863,10 +2930,11 @@ hipError_t launch_init_one(const QueryDesc& qd, QueryDesc* dq, QueryState* sts, 
 
 template <int NT, int K>
 static hipError_t launch_propagate_nt(int model, const QueryDesc* qds, QueryState* sts, const Pools& P,
-                                      const WorkLists& W, uint32_t parity, uint32_t maxPairs, const Launch& L,
-                                      hipStream_t s)
+                                      WorkLists W, uint32_t parity, uint32_t maxPairs, const Launch& L, hipStream_t s)
 {
-    const size_t lds = (size_t)maxPairs * 2 * sizeof(float4);
+    const size_t scene = (size_t)maxPairs * 2 * sizeof(float4);
+    const size_t lds   = scene + (W.few() ? (kFewQueries + 1) * sizeof(uint32_t) : 0u);
+    W.listOff          = (uint32_t)(scene / sizeof(uint32_t));
     const dim3 g(L.propGrid), b(NT);
     switch(model)
         {
