@@ -1569,8 +1569,7 @@ int kgmt_frontier_update(const kgmt_config* cfg, uint32_t itr, uint32_t tree_siz
        (rc = a.get(P.frontier, nodes)) || (rc = a.get(P.r1node, nodes)) || (rc = a.get(P.r1child, nodes)) ||
        (rc = a.get(P.fnext, nodes)) || (rc = a.get(P.react, nodes)) || (rc = a.get(P.repIdx, nodes)) ||
        (rc = a.get(P.partA, h.nChunks + 1)) || (rc = a.get(P.look, 4 * ((size_t)h.nChunks + 1))) ||
-       (rc = a.get(P.cnt, 16u << h.regShift)) || (rc = a.get(P.score, h.R1)) || (rc = a.get(W.tileStart, 4)) ||
-       (rc = a.get(W.jobStart, 4)) || (rc = a.get(W.counter, 1)) ||
+       (rc = a.get(P.cnt, 16u << h.regShift)) || (rc = a.get(P.score, h.R1)) || (rc = a.get(W.counter, 1)) ||
        (rc = a.get(W.claim, 2)) || (rc = a.get(W.allDone, 1)) || (rc = a.get(W.error, 1)) ||
        (rc = a.get(W.closed, 1)) || (rc = a.get(W.closedDev, 1)))
         return rc;

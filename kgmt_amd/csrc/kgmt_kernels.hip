@@ -823,8 +823,9 @@ __device__ __forceinline__ void child_tile(const QueryDesc& qd, const QueryState
 // not change its result. With the mask check in place of the group bounds:
 // three configured quadcopter queries 29.2 -> 19.9 ms a plan, the mixed batch
 // of 512 queries 112 -> 35.7 ms (propagate launches 444 -> 295 and 1154 ->
-// about 340 us); bound by vector issue (63 % of its slots in the single
-// query's launches), then by the length of the longest edge.
+// about 340 us, 239 and 295 with quad_ode's shorter divisions and roots); bound
+// by vector issue (63 % of its slots in the single query's launches), then by
+// the length of the longest edge.
 constexpr int kQuadSteps = 4;
 constexpr int kMoveWords = 20;  // a running child: state, controls, frontier uniform, steps left, index and steps, parent
 
@@ -2123,15 +2124,14 @@ __global__ __launch_bounds__(kUpd) void k_update(UpdateArgs)
 {
     __shared__ UpdateLds L;
     const UpdateArgs& A = *(const UpdateArgs*)__builtin_amdgcn_kernarg_segment_ptr();
-    const WorkLists& W  = A.W;
-    const QueryDesc* __restrict__ qds = A.qds;
-    QueryState* __restrict__ sts      = A.sts;
-    const uint32_t parity             = A.parity;
-    const uint32_t nq       = W.nq;
+    const WorkLists& W           = A.W;
+    QueryState* __restrict__ sts = A.sts;
+    const uint32_t parity        = A.parity;
+    const uint32_t nq            = W.nq;
     // the jobs: one query's straight from its state, a few queries' scanned by
     // every workgroup, more queries' from the list
     __shared__ uint32_t list[kFewQueries + 1];
-    const QueryState& st0 = sts[0];
+    const QueryState& st0  = sts[0];
     const uint32_t* starts = W.jobs(parity);
     uint32_t nJobs;
     if(nq == 1)
