@@ -302,6 +302,17 @@ __device__ __forceinline__ void draw_child(const kgmt_config& c, uint32_t q, uin
     ufront = u01(d[7]);
 }
 
+// its steps alone
+template <int C>
+__device__ __forceinline__ int32_t draw_steps(const kgmt_config& c, uint32_t q, uint32_t itr, uint32_t u)
+{
+    uint32_t d[4];
+    draw_block(c, q, itr, u, C / 4, d);
+    const int32_t n = c.steps_max - c.steps_min + 1;
+    const int32_t k = (int32_t)(u01(d[C % 4]) * (float)n);
+    return c.steps_min + (k > n - 1 ? n - 1 : k);
+}
+
 __device__ __forceinline__ float draw_react(const kgmt_config& c, uint32_t q, uint32_t itr, uint32_t node)
 {
     uint32_t d[4];

@@ -159,12 +159,17 @@ int dev_alloc(T*& p, size_t count, std::vector<void*>& owned)
     return KGMT_OK;
 }
 
-// children from which a quadcopter query's tiles hold two per lane (fewer
+// Children from which a quadcopter query's tiles hold two per lane (fewer
 // idle lanes: 1.3 to 1.4 times the steps needed instead of 1.5 to 1.6); below
-// it, tiles of one child per lane spread the work over more workgroups. Three
-// configured queries of 0.1 to 0.45 M children a launch: 20.36 ms with this
-// bound, 21.3 never, 20.5 always.
-constexpr uint32_t kRefill = 1u << 17;
+// it, tiles of one child per lane spread the work over more workgroups. One
+// query: 211 us a propagate launch with 2^12 to 2^17 (launches of 0.1 to 0.45 M
+// children). The queries of a batch fill the chip together, 2^18 children
+// being 512 such tiles: 512 mixed queries 291 us a launch with 2^17 for each,
+// 279 with 2^15, 268 with 2^12, 274 with 2^10; plans of 33 queries of 20000
+// nodes 8.94 to 7.80 ms, of 8 of 80000 9.29 to 8.08; but of 8 of 30000 5.08 to
+// 5.45 with 2^14, which they keep short of here. Four per lane are slower (one
+// query's launches 211 to 270 us).
+constexpr uint32_t kRefill = 1u << 17, kRefillAll = 1u << 18, kRefillLeast = 1u << 12;
 constexpr size_t kHostPathFloats = size_t(1) << 20;  // host-mapped path rows of a single query (4 MiB)
 constexpr size_t kHostPoolFloats = size_t(1) << 22;  // host-mapped path rows of a batch (16 MiB)
 // launch units the host stays ahead of the GPU: one for a plan's first
@@ -408,7 +413,7 @@ struct Engine
     {
         W.tile   = L.propBlock / L.lanes;
         W.quads  = model == -1 || model == KGMT_MODEL_QUADCOPTER ? 1u : 0u;
-        W.refill = L.lanes == 1 && W.quads ? kRefill : 0u;
+        W.refill = L.lanes == 1 && W.quads ? std::clamp(kRefillAll / W.nq, kRefillLeast, kRefill) : 0u;
     }
 
     int set_stream(void* s)
