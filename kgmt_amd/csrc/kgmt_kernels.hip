@@ -823,9 +823,9 @@ __device__ __forceinline__ void child_tile(const QueryDesc& qd, const QueryState
 // not change its result. With the mask check in place of the group bounds:
 // three configured quadcopter queries 29.2 -> 19.9 ms a plan, the mixed batch
 // of 512 queries 112 -> 35.7 ms (propagate launches 444 -> 295 and 1154 ->
-// about 340 us, 239 and 295 with quad_ode's shorter divisions and roots); bound
-// by vector issue (63 % of its slots in the single query's launches), then by
-// the length of the longest edge.
+// about 340 us, 239 and 295 with quad_ode's shorter divisions and roots, 211 and
+// 268 with the longest edges first); bound by vector issue, then by the length
+// of the longest edge.
 constexpr int kQuadSteps = 4;
 constexpr int kMoveWords = 20;  // a running child: state, controls, frontier uniform, steps left, index and steps, parent
 
