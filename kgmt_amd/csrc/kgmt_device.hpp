@@ -214,9 +214,9 @@ struct HostResult
 // Most queries whose work lists every workgroup makes for itself: each query's
 // last update job leaves its tiles and jobs in one word, and a workgroup scans
 // the words into LDS (33 queries: k_propagate 16.6 to 16.2 us, k_update 10.6 to
-// 10.9, and k_finish's 4.3 are gone). More queries' lists are made by k_finish:
-// 256 words are one load of a propagate workgroup, 5.9 us are little beside an
-// iteration of that many, and the list would take LDS from the scene.
+// 10.9, and k_finish's 4.3 are gone). More queries' lists are made by k_finish,
+// 5.9 us beside an iteration of that many: a longer list costs LDS (512 mixed
+// queries with one of 512: a workgroup less on a CU, k_propagate 268 to 297 us).
 constexpr uint32_t kFewQueries = 256;
 
 struct WorkLists
