@@ -141,16 +141,27 @@ __device__ __forceinline__ void box_penalty(float4 lo, float4 hi, float px, floa
     const float d2 = ox * ox + oy * oy + oz * oz;
     const float id = __builtin_amdgcn_rsqf(d2);
     float sd       = d2 * id;
-    // outside: (ox, oy, oz) / distance; inside (rare: one vote of the active
-    // lanes skips it): the axis of the nearest face, the first of the largest
+    // outside: (ox, oy, oz) / distance; inside: the axis of the nearest face,
+    // the first of the largest. The unit's reciprocal root holds for normal d2
+    // alone: a face or a corner within 1e-19 and a box farther than 1.8e19
+    // take a scaled root, as inside does (rare: one vote of the active lanes
+    // skips it; the other lanes keep what they have)
     float vx = ox * id, vy = oy * id, vz = oz * id;
-    if(__any(!(d2 > 0.0f) | __builtin_isunordered(qx, qy) | (qz != qz)))
+    const bool tiny = !(d2 >= 0x1p-126f), huge = !(d2 <= 0x1.fffffep127f);
+    const bool odd  = tiny | huge | __builtin_isunordered(qx, qy) | (qz != qz);
+    if(__any(odd))
         {
-            const bool out = d2 > 0.0f;
+            const float k  = tiny ? 0x1p100f : huge ? 0x1p-100f : 1.0f;
+            const float rk = tiny ? 0x1p-100f : huge ? 0x1p100f : 1.0f;
+            const float kx = ox * k, ky = oy * k, kz = oz * k;
+            const float root = __builtin_sqrtf(kx * kx + ky * ky + kz * kz), len = root * rk;
+            const float ux = kx / root, uy = ky / root, uz = kz / root;
+            const bool out = root > 0.0f;
             const bool xy = qx >= qy, ax = xy & (qx >= qz), ay = !xy & (qy >= qz);
-            sd = (out ? sd : 0.0f) + fminf(ax ? qx : ay ? qy : qz, 0.0f);
-            vx = out ? vx : ax ? 1.0f : 0.0f, vy = out ? vy : ay ? 1.0f : 0.0f;
-            vz = out ? vz : (ax | ay) ? 0.0f : 1.0f;
+            sd = odd ? (out ? len : 0.0f) + fminf(ax ? qx : ay ? qy : qz, 0.0f) : sd;
+            vx = odd ? (out ? ux : ax ? 1.0f : 0.0f) : vx;
+            vy = odd ? (out ? uy : ay ? 1.0f : 0.0f) : vy;
+            vz = odd ? (out ? uz : (ax | ay) ? 0.0f : 1.0f) : vz;
         }
     const float z = (margin - sd) * itau;
     const float e = __builtin_amdgcn_exp2f(-1.44269504f * fabsf(z));
