@@ -206,6 +206,7 @@ int kgmt_set_graph(kgmt_ctx* ctx, int32_t on);
  * workgroup (128, 256 or 512), lanes per child (1; or 2 or 4 with 256
  * threads: the lanes split the child's box tests), and the workgroup counts
  * of the propagate and update kernels (0 keeps the current value).
+ * Taken by the next plan: one in progress (kgmt_plan_step) keeps its own.
  * Results do not depend on it. No counterpart in the reference (fixed launch
  * shapes at KGMT.cu:183-211). */
 int kgmt_set_launch(kgmt_ctx* ctx, uint32_t propagate_block, uint32_t lanes_per_child, uint32_t propagate_grid,

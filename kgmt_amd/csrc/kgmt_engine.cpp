@@ -278,7 +278,8 @@ struct Engine
     bool ownStream     = false;
     uint32_t* pinned   = nullptr;  // host-mapped words written by the kernels: completion, look-back error,
                                    // iterations closed
-    Launch L;
+    Launch L;     // shape of the plan in progress, or of the last one
+    Launch wanted;  // shape that the next plan takes
     hipGraph_t graph         = nullptr;
     hipGraphExec_t graphExec = nullptr;
     uint32_t graphObs        = 0xffffffffu;
@@ -406,7 +407,17 @@ struct Engine
         const uint32_t cus = (uint32_t)std::max(prop.multiProcessorCount, 1);
         L.propGrid         = cus * 4;
         L.chunkGrid        = cus * 4;
+        wanted             = L;
         return KGMT_OK;
+    }
+
+    // The shape of the plan that starts. A quadcopter's scene (with or without
+    // box masks), the LDS of its tiles and the work lists follow from it, so a
+    // plan keeps it to its end.
+    void use_launch()
+    {
+        L = wanted;
+        set_tile();
     }
 
     void set_tile()
@@ -1063,16 +1074,16 @@ int kgmt_set_seed(kgmt_ctx* ctx, uint64_t seed)
 static int set_launch(Engine& e, uint32_t propagate_block, uint32_t lanes_per_child, uint32_t propagate_grid,
                       uint32_t chunk_grid)
 {
-    const uint32_t blk = propagate_block ? propagate_block : e.L.propBlock;
-    const uint32_t ln  = lanes_per_child ? lanes_per_child : e.L.lanes;
+    const uint32_t blk = propagate_block ? propagate_block : e.wanted.propBlock;
+    const uint32_t ln  = lanes_per_child ? lanes_per_child : e.wanted.lanes;
     if(!launch_supported(blk, ln))
         return fail(KGMT_E_UNSUPPORTED, "propagate shape must be 128/256/512 threads with 1 lane per child, "
                                         "or 256 threads with 2 or 4 lanes per child");
     if(propagate_grid > (1u << 20) || chunk_grid > (1u << 20)) return fail(KGMT_E_ARG, "grid too large");
-    e.L.propBlock = blk, e.L.lanes = ln;
-    e.set_tile();
-    if(propagate_grid) e.L.propGrid = propagate_grid;
-    if(chunk_grid) e.L.chunkGrid = chunk_grid;
+    Launch& L   = e.wanted;  // (use_launch)
+    L.propBlock = blk, L.lanes = ln;
+    if(propagate_grid) L.propGrid = propagate_grid;
+    if(chunk_grid) L.chunkGrid = chunk_grid;
     return KGMT_OK;
 }
 
@@ -1132,10 +1143,18 @@ static int upload_obstacles(Engine& e, const float* obstacles, const uint32_t* o
             const uint32_t off = offsets ? offsets[q] : 0;
             if(c > kMaxObs) return fail(KGMT_E_CAPACITY, "more than 1500 obstacles in one query");
             if((uint64_t)off + c > (uint64_t)total) return fail(KGMT_E_ARG, "obstacle range out of bounds");
-            pairs += pool_pairs(c, mask_check(e.hq[q].cfg.model, e.L.lanes));
+            pairs += pool_pairs(c, mask_check(e.hq[q].cfg.model, e.wanted.lanes));
         }
-    int rc = e.ensure_obstacles(pairs);
+    int rc = total && onDevice ? check_device_rows(obstacles) : KGMT_OK;
     if(rc) return rc;
+    // (a step-by-step plan in progress goes on after the refusals above; the
+    // calls below may drop its scene)
+    if((rc = e.ensure_obstacles(pairs)) || (total && !onDevice && (rc = e.ensure_rows(total))))
+        {
+            e.stepping = false;
+            return rc;
+        }
+    e.use_launch();
     // scenes are built on the device (run()) from the caller's device rows or
     // from a device copy of the host rows
     e.sceneRows  = nullptr;
@@ -1143,13 +1162,9 @@ static int upload_obstacles(Engine& e, const float* obstacles, const uint32_t* o
     if(total)
         {
             if(onDevice)
-                {
-                    if((rc = check_device_rows(obstacles))) return rc;
-                    e.sceneRows = obstacles;
-                }
+                e.sceneRows = obstacles;
             else
                 {
-                    if((rc = e.ensure_rows(total))) return rc;
                     const size_t rowW = 2 * (size_t)e.hq[0].wdim;
                     HIP_TRY(hipMemcpyAsync(e.rowsBuf, obstacles, (size_t)total * rowW * sizeof(float),
                                            hipMemcpyHostToDevice, e.stream));
