@@ -423,7 +423,10 @@ int kgmt_repeat(const uint32_t* d_ids, const uint32_t* d_counts, uint32_t n, uin
  *   steps [n] int32 (T_k <= max_steps), x0 [12][n], goal [3][n],
  *   u / grad [max_steps][4][n] (element (t, c, k) at (t*4 + c)*n + k),
  *   obstacles: 6 floats per box (shared by all trajectories).
- * cfg supplies the quad parameters, dt and (for clamping) ctrl_min/max. */
+ * cfg supplies the quad parameters, dt and (for clamping) ctrl_min/max.
+ * A trajectory's results follow from its own inputs, bit for bit: not from
+ * rows of u past T_k, which are not read, nor from the other trajectories or
+ * their number. */
 /* J_k -> cost[n] and dJ_k/du -> grad (zero past T_k). */
 int kgmt_rk4_adjoint(const kgmt_config* cfg, const kgmt_adjoint_params* ap, uint32_t n, uint32_t max_steps,
                      const int32_t* d_steps, const float* d_x0, const float* d_goal, const float* d_u,
