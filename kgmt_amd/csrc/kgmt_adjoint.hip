@@ -142,29 +142,40 @@ __device__ __forceinline__ float quad_scatter(const float (&v)[4], int lane)
     return (b0 ? y : x) + dpp<0xB1>(b0 ? x : y);
 }
 
-// tau * softplus((margin - sd) / tau) of one box at p, and its gradient
-// (times -w): softplus(z) = max(z, 0) + log1p(e) and its derivative
-// (1 or e) / (1 + e) with e = exp(-|z|); log1p(e) = 2 atanh(e / (2 + e)).
-// The error of z (of the position, over tau) is larger than that of exp2
-// of the rounded product.
+// tau * softplus(x / tau), x = margin - sd, of one box at p, and its gradient:
+// max(x, 0) + tau log1p(e) and (1 or e) / (1 + e) with e = exp(-|x| / tau);
+// log1p(e) = 2 atanh(t), t = e / (2 + e), the polynomial by Chebyshev
+// interpolation over t^2 <= 1/9. The root, the reciprocal and the exponential
+// of the units are within an ulp; each is followed by the step that takes its
+// error out (the residuals of the root and of the quotients, the rest of the
+// exponent's product): one box's penalty is 0.7 to 1.05 times as far from 64
+// bits as by the library's sqrt, division, expf and log1pf (its gradient 0.75
+// to 1.1 times), 1.0 to 2.2 times without. That costs 8 %: refine of 4096
+// trajectories among 50 boxes 7.48 to 8.00 ms. acc: half the logarithms, and
+// the gradient; flat: the max(x, 0).
 __device__ __forceinline__ void box_penalty(float4 lo, float4 hi, float px, float py, float pz, float margin,
-                                            float itau, float tau, float w, float (&acc)[4])
+                                            float tau, const RolloutK& K, float (&acc)[4], float& flat)
 {
     const float lx = lo.x - px, hx = px - hi.x, ly = lo.y - py, hy = py - hi.y, lz = lo.z - pz, hz = pz - hi.z;
     const bool nx = lx > hx, ny = ly > hy, nz = lz > hz;  // nearer the low face
     const float qx = nx ? lx : hx, qy = ny ? ly : hy, qz = nz ? lz : hz;
     const float ox = fmaxf(qx, 0.0f), oy = fmaxf(qy, 0.0f), oz = fmaxf(qz, 0.0f);
     const float d2 = ox * ox + oy * oy + oz * oz;
-    const float id = __builtin_amdgcn_rsqf(d2);
-    float sd       = d2 * id;
+    const float id = __builtin_amdgcn_rsqf(d2), s0 = d2 * id;
+    float sd       = __builtin_fmaf(__builtin_fmaf(-s0, s0, d2), 0.5f * id, s0);
+    float x        = margin - sd;
+    // -|x| / tau in base 2: rounded, and what the rounding leaves
+    float y  = -fabsf(x) * K.eHi;
+    float yl = __builtin_fmaf(-fabsf(x), K.eLo, __builtin_fmaf(-fabsf(x), K.eHi, -y));
     // outside: (ox, oy, oz) / distance; inside: the axis of the nearest face,
     // the first of the largest. The unit's reciprocal root holds for normal d2
     // alone: a face or a corner within 1e-19 and a box farther than 1.8e19
-    // take a scaled root, as inside does (rare: one vote of the active lanes
-    // skips it; the other lanes keep what they have)
+    // take a scaled root, as inside does, and the plain quotient by tau (rare:
+    // one vote of the active lanes skips it; the other lanes keep what they
+    // have; K.plain: tau or margin out of the range of the short form)
     float vx = ox * id, vy = oy * id, vz = oz * id;
     const bool tiny = !(d2 >= 0x1p-126f), huge = !(d2 <= 0x1.fffffep127f);
-    const bool odd  = tiny | huge | __builtin_isunordered(qx, qy) | (qz != qz);
+    const bool odd  = tiny | huge | __builtin_isunordered(qx, qy) | (qz != qz) | (K.plain != 0u);
     if(__any(odd))
         {
             const float k  = tiny ? 0x1p100f : huge ? 0x1p-100f : 1.0f;
@@ -178,24 +189,28 @@ __device__ __forceinline__ void box_penalty(float4 lo, float4 hi, float px, floa
             vx = odd ? (out ? ux : ax ? 1.0f : 0.0f) : vx;
             vy = odd ? (out ? uy : ay ? 1.0f : 0.0f) : vy;
             vz = odd ? (out ? uz : (ax | ay) ? 0.0f : 1.0f) : vz;
+            x  = margin - sd;
+            const float z = fabsf(x / tau), c = z > 110.0f ? 110.0f : z;  // (e^-104 is 0; NaN stays)
+            const float w = c * -0x1.715476p+0f;
+            yl = odd ? __builtin_fmaf(c, -0x1.4ae0cp-26f, __builtin_fmaf(c, -0x1.715476p+0f, -w)) : yl;
+            y  = odd ? w : y;
         }
-    const float z = (margin - sd) * itau;
-    const float e = __builtin_amdgcn_exp2f(-1.44269504f * fabsf(z));
+    const float e0 = __builtin_amdgcn_exp2f(y), e = __builtin_fmaf(e0, 0.693147181f * yl, e0);
     // one reciprocal for 1 / (2 + e) and 1 / (1 + e)
-    const float e1 = 1.0f + e, e2 = 2.0f + e, re = recip(e1 * e2);
-    const float s = e * e1 * re, s2 = s * s;
-    float at      = __builtin_fmaf(s2, 2.0f / 15.0f, 2.0f / 13.0f);
-    at            = __builtin_fmaf(s2, at, 2.0f / 11.0f);
-    at            = __builtin_fmaf(s2, at, 2.0f / 9.0f);
-    at            = __builtin_fmaf(s2, at, 2.0f / 7.0f);
-    at            = __builtin_fmaf(s2, at, 2.0f / 5.0f);
-    at            = __builtin_fmaf(s2, at, 2.0f / 3.0f);
-    at            = __builtin_fmaf(s2, at, 2.0f);
-    acc[0]        = __builtin_fmaf(tau, __builtin_fmaf(s, at, fmaxf(z, 0.0f)), acc[0]);
-    const float ds = -w * (z >= 0.0f ? 1.0f : e) * e2 * re;
-    acc[1]         = __builtin_fmaf(nx ? -ds : ds, vx, acc[1]);
-    acc[2]         = __builtin_fmaf(ny ? -ds : ds, vy, acc[2]);
-    acc[3]         = __builtin_fmaf(nz ? -ds : ds, vz, acc[3]);
+    const float e1 = 1.0f + e, e2 = 2.0f + e, el = e - (e2 - 2.0f);
+    const float re = recip(e1 * e2), r1 = e2 * re, r2 = e1 * re;
+    const float t0 = e * r2, tr = __builtin_fmaf(-t0, el, __builtin_fmaf(-t0, e2, e)) * r2, t = t0 + tr, u = t * t;
+    float at       = __builtin_fmaf(u, 0x1.dba25ep-4f, 0x1.bc8cf8p-4f);
+    at             = __builtin_fmaf(u, at, 0x1.24c926p-3f);
+    at             = __builtin_fmaf(u, at, 0x1.9998d4p-3f);
+    at             = __builtin_fmaf(u, at, 0x1.555556p-2f);
+    acc[0]         = __builtin_fmaf(tau, t0 + __builtin_fmaf(t * u, at, tr), acc[0]);  // (half of it)
+    flat += fmaxf(x, 0.0f);
+    const float n  = x >= 0.0f ? 1.0f : e;
+    const float g0 = n * r1, g = __builtin_fmaf(__builtin_fmaf(-g0, e1, n), r1, g0);
+    acc[1]         = __builtin_fmaf(nx ? g : -g, vx, acc[1]);
+    acc[2]         = __builtin_fmaf(ny ? g : -g, vy, acc[2]);
+    acc[3]         = __builtin_fmaf(nz ? g : -g, vz, acc[3]);
 }
 
 constexpr int kRowWords   = 12;   // a row of coefficients: constant, then those of a3 a4 a6 a7 a8 a9 a10 a11
@@ -273,7 +288,6 @@ __global__ __launch_bounds__(64) void k_rollout(RolloutK K, kgmt_adjoint_params 
     const float uscale = s == 0 ? K.minv : s == 1 ? K.bx : s == 2 ? K.by : K.bz;
     const float umin   = s == 0 ? K.cmin[0] : s == 1 ? K.cmin[1] : s == 2 ? K.cmin[2] : K.cmin[3];
     const float umax   = s == 0 ? K.cmax[0] : s == 1 ? K.cmax[1] : s == 2 ? K.cmax[2] : K.cmax[3];
-    const float itau   = 1.0f / ap.tau;
     const float hS     = s == 0 || s == 3 ? K.h6 : K.h3;  // weight of stage s in the step
     const float* uF    = Wg + 4 + ((s + 1) & 3);  // forward: lane c takes control c + 1, lane 3 control 0
     const uint32_t iters = REFINE ? ap.iterations : 0;
@@ -434,18 +448,19 @@ __global__ __launch_bounds__(64) void k_rollout(RolloutK K, kgmt_adjoint_params 
                     rx = __shfl(rx, LPT - 1, LPT), ry = __shfl(ry, LPT - 1, LPT), rz = __shfl(rz, LPT - 1, LPT);
                     // boxes s, s + 4, ... against this lane's step, each read
                     // while the one before it is worked on
-                    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+                    float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f}, flat = 0.0f;
                     float4 lo = sBox[s], hi = sBox[nBox + s];
                     for(uint32_t o = s; o < nObs; o += 4)
                         {
                             const float4 l1 = sBox[o + 4], h1 = sBox[nBox + o + 4];
-                            box_penalty(lo, hi, qx, qy, qz, ap.margin, itau, ap.tau, ap.w_obstacle, acc);
+                            box_penalty(lo, hi, qx, qy, qz, ap.margin, ap.tau, K, acc, flat);
                             lo = l1, hi = h1;
                         }
-                    const float mine = quad_scatter(acc, l);
+                    acc[0] += acc[0] + flat;
+                    const float mine = ap.w_obstacle * quad_scatter(acc, l);
                     if(on)
                         {
-                            const float Jt = (s == 0 ? ap.w_obstacle * mine : 0.0f) + ap.w_effort * d * d;
+                            const float Jt = (s == 0 ? mine : 0.0f) + ap.w_effort * d * d;
 #pragma unroll
                             for(int k = 0; k < 64 / LPT; ++k)
                                 if(k == ((t0 / CH) & (64 / LPT - 1))) Jp[k] += Jt;

@@ -1690,8 +1690,11 @@ static int adjoint_common(bool refine, const kgmt_config* cfg, const kgmt_adjoin
     QueryDesc qd;
     fill_desc(qd, *cfg);
     RolloutK K{cfg->dt, 0.5f * cfg->dt, cfg->dt / 6.0f, cfg->dt / 3.0f, cfg->gravity, qd.qminv, cfg->quad_nu,
-               cfg->quad_mu, qd.qax, qd.qbx, qd.qay, qd.qby, qd.qaz, qd.qbz, {}, {}};
+               cfg->quad_mu, qd.qax, qd.qbx, qd.qay, qd.qby, qd.qaz, qd.qbz, {}, {}, 0.0f, 0.0f, 0u};
     for(int k = 0; k < 4; ++k) K.cmin[k] = cfg->ctrl_min[k], K.cmax[k] = cfg->ctrl_max[k];
+    const double le = 1.4426950408889634 / (double)ap->tau;
+    K.plain = !(ap->tau >= 0x1p-40f && ap->tau <= 0x1p60f && std::fabs(ap->margin) <= 1e18f) ? 1u : 0u;
+    if(!K.plain) K.eHi = (float)le, K.eLo = (float)(le - (double)K.eHi);
     AsyncBuffers a((hipStream_t)stream);  // released on every return path
     size_t floats       = 0;
     const uint32_t slab = rollout_slab(refine, n, max_steps, &floats);

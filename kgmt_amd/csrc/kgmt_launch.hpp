@@ -98,6 +98,10 @@ struct RolloutK
     float g, minv, nu, mu;
     float ax, bx, ay, by, az, bz;
     float cmin[4], cmax[4];
+    // log2(e) / tau in two parts, the penalty's exponent; plain: tau or margin
+    // where it is not formed this way
+    float eHi, eLo;
+    uint32_t plain;
 };
 // trajectories per launch and the floats of work space they take
 uint32_t rollout_slab(bool refine, uint32_t n, uint32_t maxT, size_t* floats);

@@ -94,3 +94,52 @@ def test_faces_at_a_hair_from_the_position(gap, axis, low, orc):
         J, w = orc.traj_grad_f64(cfg, ap, x0[:, k], u[:, :, k], goal[:, k], box)
         assert abs(c[k] - J) <= RTOL * max(J, 1e-30), (k, c[k], J)
         assert np.abs(g[:, :, k] - w).max() <= RTOL * np.abs(w).max(), (k, g[:, :, k], w)
+
+
+def _one_box(z, tau, margin, orc):
+    """(cost, gradient, 64-bit cost, 64-bit gradient, position) of trajectories
+    at rest above the face z = 0 of one box, the thrust along z."""
+    cfg = W.config("quad12d", dt=0.1, gravity=0.0)
+    ap = W.refine_params(cfg, "hover")
+    ap.w_effort, ap.w_goal, ap.w_obstacle, ap.margin, ap.tau = 0.0, 0.0, 1.0, margin, tau
+    n = len(z)
+    x0 = np.zeros((12, n), np.float32)
+    x0[2] = z
+    box = np.array([[-1.0, -1.0, -1.0, 1.0, 1.0, 0.0]], np.float32)
+    u, goal, steps = np.zeros((1, 4, n), np.float32), np.zeros((3, n), np.float32), np.ones(n, np.int32)
+    c, g = A.cost_and_grad(_d(u), _d(x0), _d(goal), _d(steps), _d(box), cfg, ap)
+    J, w = np.zeros(n), np.zeros(n)
+    for k in range(n):
+        J[k], e = orc.traj_grad_f64(cfg, ap, x0[:, k], u[:, :, k], goal[:, k], box)
+        w[k] = e[0, 0]
+    return c.cpu().numpy().astype(np.float64), g.cpu().numpy()[0, 0].astype(np.float64), J, w, x0[2].astype(np.float64)
+
+
+@pytest.mark.parametrize("tau", [0.5, 0.05, 0.01, 0.002])
+def test_one_box_to_the_last_bits(tau, orc):
+    """The distance is the position: exact but for the square's rounding and
+    the root's (0.75 of 2^-24), which the exponent multiplies by z; beside it a
+    few roundings of 2^-24 (the exponential 2, the logarithm's quotient, its
+    sum and the product with tau 1 each, for the gradient the quotient and the
+    backward chain's eight products)."""
+    rng = np.random.default_rng(int(1 / tau))
+    z = np.exp(rng.uniform(np.log(1e-4), np.log(min(60.0 * tau, 1.0)), 3000)).astype(np.float32)
+    c, g, J, w, p = _one_box(z, tau, 0.0, orc)
+    ulp = 2.0**-24
+    zz = p / float(np.float32(tau))
+    worst = (np.abs(c - J) / J / ulp - zz).max(), (np.abs(g - w) / np.abs(w) / ulp - zz).max()
+    print(f"tau {tau}: error less z, in 2^-24: cost {worst[0]:.2f}, gradient {worst[1]:.2f}", flush=True)
+    assert (np.abs(c - J) <= (zz + 5.0) * ulp * J).all()
+    assert (np.abs(g - w) <= (zz + 11.0) * ulp * np.abs(w)).all()
+
+
+@pytest.mark.parametrize("tau,margin", [(1e-13, 0.02), (1e-39, 0.02), (1e19, 0.02), (3e38, 0.02), (0.01, 1e19),
+                                        (0.01, -1e19), (0.01, 3e38)])
+def test_ends_of_tau_and_margin(tau, margin, orc):
+    z = np.array([1e-3, 0.01, 0.0199, 0.0201, 0.3, 2.0], np.float32)
+    c, g, J, w, _ = _one_box(z, tau, margin, orc)
+    # (a cost past the largest float is infinite)
+    J32 = J.astype(np.float32).astype(np.float64)
+    same = (c == J32) | (np.abs(c - J) <= RTOL * np.maximum(np.abs(J), 1e-30))
+    assert same.all(), (c, J)
+    assert (np.abs(g - w) <= RTOL * np.maximum(np.abs(w), 1e-30)).all(), (g, w)
