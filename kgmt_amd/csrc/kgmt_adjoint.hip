@@ -663,14 +663,22 @@ static uint32_t rollout_lanes(uint32_t n)
     return n <= 1024 ? 64 : n <= 2048 ? 32 : 16;
 }
 
+// Trajectories per launch, and the floats of work space they take. The launches
+// of a call share one work space: 1 GiB, or, of long rollouts, 12 floats a step
+// and trajectory (20 with moments) where that is more: a launch lasts as long
+// as the longest chain, however few trajectories it holds, so at most five
+// launches do the call (4096 trajectories of 8000 and 20000 steps: 74 and 484 ms
+// in launches of 1 GiB, 47 and 117 in five; 77 and 193 in one launch of a kernel
+// that kept 12 floats a step and ran the whole step in every lane).
 uint32_t rollout_slab(bool refine, uint32_t n, uint32_t maxT, size_t* floats)
 {
-    const size_t per = std::max<size_t>(rollout_words(refine, maxT), 1);
-    // trajectories per launch: whole waves, the work space within 1 GiB
-    const size_t most = std::max<size_t>((size_t(1) << 28) / per / 64 * 64, 64);
-    const uint32_t slab = (uint32_t)std::min<size_t>(((size_t)n + 63) / 64 * 64, most);
+    const size_t per  = std::max<size_t>(rollout_words(refine, maxT), 1);
+    const size_t most = std::max<size_t>(size_t(1) << 28, ((size_t)maxT * (refine ? 20 : 12) + 12) * n) / per;
+    const size_t wave = 64 / rollout_lanes(n), all = ((size_t)n + wave - 1) / wave * wave;
+    // whole waves: four trajectories at most
+    const size_t slab = most >= all ? all : most >= 4 ? most / 4 * 4 : std::max<size_t>(most, 1);
     *floats = per * slab;
-    return slab;
+    return (uint32_t)slab;
 }
 
 template <bool REFINE, int LPT>
