@@ -352,7 +352,8 @@ enum {
     KGMT_CHECK_CANDIDATES = 1, /* two-phase: the wave's candidate list, each lane its  */
                                /* own candidates inside its edge box                  */
     KGMT_CHECK_DRY_RUN    = 2, /* two-phase: no box near the wave, the dry run decides */
-    KGMT_CHECK_ONE_PASS   = 3  /* quadcopter: one pass against every box             */
+    KGMT_CHECK_ONE_PASS   = 3  /* quadcopter: one pass, every step against the boxes  */
+                               /* that its box masks leave                            */
 };
 /* Propagate + collide through the planner's own per-child path, for checking
  * it on identical inputs: children in waves of 64 consecutive indices, sorted
@@ -362,8 +363,11 @@ enum {
  * unicycle (an edge box from a dry run, or for the Dubins models from an
  * interval bound of the edge; the wave's candidate boxes = boxes meeting some
  * lane's edge box; each lane tests only its own candidates; the whole scene
- * when a box is not finite or the candidates exceed 128), the one-pass check
- * for the quadcopter. Same arguments and outputs as kgmt_propagate_collide
+ * when a box is not finite or the candidates exceed 128). A quadcopter's
+ * children run as the planner's tiles with one lane per child run them (512
+ * children of a tile sorted over its 256 lanes, then 256 as they come, in
+ * turn; lanes refilled and moved together, a quad of lanes for each of the
+ * last) with the one-pass check on the planner's scene and masks. Same arguments and outputs as kgmt_propagate_collide
  * (isMotionValid, collisionCheck.cu:49-62, per step), plus two optional
  * outputs (NULL: not written): d_check[n], the KGMT_CHECK_* that decided
  * each child, and d_edge_box [6][n], each child's edge box (lo xyz, hi xyz;

@@ -1542,13 +1542,15 @@ int kgmt_propagate_collide_planner(const kgmt_config* cfg, const int32_t* d_pare
     if(n_obs && (rc = check_device_rows(d_obstacles))) return rc;
     const uint32_t nGrp = scene_groups(n_obs);
     float4* d_scene     = nullptr;
-    HIP_TRY(hipMallocAsync((void**)&d_scene, (size_t)std::max<uint32_t>(scene_pairs(n_obs), 1) * 2 * sizeof(float4),
-                           sd.s));
-    hipError_t e = launch_build_scene(d_obstacles, n_obs, nGrp, d_scene, model_wdim(cfg->model), sd.s);
+    const bool masks    = mask_check(cfg->model, 1);
+    HIP_TRY(hipMallocAsync((void**)&d_scene,
+                           (size_t)std::max<uint32_t>(pool_pairs(n_obs, masks), 1) * 2 * sizeof(float4), sd.s));
+    hipError_t e = masks ? launch_build_mask_scene(sd.d, d_obstacles, n_obs, nGrp, d_scene, sd.s)
+                         : launch_build_scene(d_obstacles, n_obs, nGrp, d_scene, model_wdim(cfg->model), sd.s);
     if(e == hipSuccess)
         e = launch_stage_propagate_planner(cfg->model, sd.d, d_parent_idx, d_parent_states, n_parents, d_controls,
-                                           d_steps, n_children, d_scene, nGrp, d_child_samples, d_valid, d_r1, d_r2,
-                                           d_check, d_edge_box, sd.s);
+                                           d_steps, n_children, d_scene, nGrp, n_obs, d_child_samples, d_valid, d_r1,
+                                           d_r2, d_check, d_edge_box, sd.s);
     (void)hipFreeAsync(d_scene, sd.s);
     if(e != hipSuccess) return fail(KGMT_E_HIP, std::string("propagate: ") + hipGetErrorString(e));
     return KGMT_OK;

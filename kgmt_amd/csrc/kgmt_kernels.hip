@@ -2489,6 +2489,16 @@ __global__ __launch_bounds__(kBlock) void k_build_scene(const float* __restrict_
     build_scene_wg<W>(rows, n, nGrp, out, L);
 }
 
+// a caller's boxes as the planner's scene of a query with box masks
+__global__ __launch_bounds__(kBlock) void k_build_mask_scene(const QueryDesc* __restrict__ qdp,
+                                                             const float* __restrict__ rows, uint32_t n, uint32_t nGrp,
+                                                             float4* __restrict__ out)
+{
+    __shared__ SceneLds L;
+    build_scene_wg<3, true>(rows, n, nGrp, out, L, reinterpret_cast<uint32_t*>(out + 2 * (size_t)nGrp * (1 + kGroup)),
+                            qdp->cfg.ws_min, qdp->slabScale);
+}
+
 // ---------------------------------------------------------------------------
 // a query's tree in the reference's layout: rows of D floats
 // (d_treeSamples_), parents and costs; entries past the tree are 0, -1, 0 as
@@ -2568,30 +2578,40 @@ __device__ __forceinline__ MaskScene stage_scene_masks(const QueryDesc& qd, cons
     return MaskScene{lo, hi, mask, (int)mask_row(n), (int)n};
 }
 
-// kgmt_propagate_collide: one launch. Every workgroup builds the scene's
-// masks in its LDS (about 2 us for 200 boxes; a scene kernel before this one
-// took 10.6 and the sort its group bounds need grows with the square of the
-// boxes) and takes every gridDim.x-th tile of kBlock children: one per lane,
-// or, for the quadcopter, as the planner's tiles do. 100003 quadcopter edges
-// among 200 boxes: kernels 539 + 10.6 -> 235 us, the call 580 -> 233; 100003 of
-// the other models 102 to 246 -> 22 to 47 us, 1000 of them 55 to 65 -> 12 to 20.
+// A caller's edges: parent, control and steps in, child, verdict and regions
+// out.
 template <int MODEL>
-__global__ __launch_bounds__(kBlock, 4) void k_stage_propagate(const QueryDesc qd, const int32_t* __restrict__ parentIdx,
-                                                               const float* __restrict__ parentStates,
-                                                               uint32_t nParents, const float* __restrict__ controls,
-                                                               const int32_t* __restrict__ steps, uint32_t n,
-                                                               const float* __restrict__ rows, uint32_t nObs,
-                                                               float* __restrict__ child, uint8_t* __restrict__ valid,
-                                                               int32_t* __restrict__ r1o, int32_t* __restrict__ r2o)
+struct StageEdges
 {
-    constexpr int S = ModelDims<MODEL>::S, C = ModelDims<MODEL>::C, D = S + C + 1;
-    extern __shared__ float4 sObs[];
-    const MaskScene sc = stage_scene_masks<MODEL == KGMT_MODEL_UNICYCLE ? 2 : 3>(qd, rows, nObs, sObs);
-    auto parent = [&](uint32_t i) {
+    static constexpr int S = ModelDims<MODEL>::S, C = ModelDims<MODEL>::C, D = S + C + 1;
+    const int32_t* __restrict__ parentIdx;
+    const float* __restrict__ parentStates;
+    uint32_t nParents;
+    const float* __restrict__ controls;
+    const int32_t* __restrict__ steps;
+    uint32_t n;
+    float* __restrict__ child;
+    uint8_t* __restrict__ valid;
+    int32_t* __restrict__ r1o;
+    int32_t* __restrict__ r2o;
+
+    // -1: out of range
+    __device__ __forceinline__ int32_t parent(uint32_t i) const
+    {
         const int32_t p = parentIdx[i];
         return p >= 0 && (uint32_t)p < nParents ? p : -1;
-    };
-    auto write = [&](uint32_t i, int32_t p, const float* s, const float* u, bool ok) {
+    }
+    // start state and control of edge i
+    __device__ __forceinline__ void read(uint32_t i, int32_t p, float* s, float* u) const
+    {
+#pragma unroll
+        for(int d = 0; d < S; ++d) s[d] = p < 0 ? 0.0f : parentStates[(size_t)d * nParents + p];
+#pragma unroll
+        for(int k = 0; k < C; ++k) u[k] = controls[(size_t)k * n + i];
+    }
+    __device__ __forceinline__ void write(const QueryDesc& qd, uint32_t i, int32_t p, const float* s, const float* u,
+                                          bool ok) const
+    {
         if(p < 0)
             {
                 // caller index out of range: no state is read; flagged by r1 = r2 = -1
@@ -2611,49 +2631,72 @@ __global__ __launch_bounds__(kBlock, 4) void k_stage_propagate(const QueryDesc q
         valid[i]     = ok ? 1 : 0;
         r1o[i]       = r1;
         r2o[i]       = subregion_of(qd, s[0], s[1], s[2], r1, ix, iy, iz);
-    };
+    }
+};
+
+// Quadcopter edges base .. base + count - 1 as a planner's tile of NT threads
+// (at most 2 NT edges; barriers inside).
+template <int NT>
+__device__ __forceinline__ void stage_quad_tile(const QueryDesc& qd, const StageEdges<KGMT_MODEL_QUADCOPTER>& E,
+                                                uint32_t base, uint32_t count, const MaskScene& sc, QuadRunLds<NT>& L)
+{
+    quad_run<NT>(
+      qd, count, sc, L, [&](uint32_t k) { return E.steps[base + k]; },
+      [&](uint32_t k, QuadChild& ch) {
+          const uint32_t i = base + k;
+          const int32_t p  = E.parent(i);
+          ch.p             = (uint32_t)p;
+          E.read(i, p, ch.s, ch.u);
+          const int32_t st = E.steps[i];
+          ch.uf            = 0.0f;
+          ch.left          = p < 0 || st < 0 ? 0 : st;
+      },
+      [&](const QuadChild& ch) { E.write(qd, base + (ch.meta & 1023u), (int32_t)ch.p, ch.s, ch.u, ch.left == 0); });
+}
+
+// kgmt_propagate_collide: one launch. Every workgroup builds the scene's
+// masks in its LDS (about 2 us for 200 boxes; a scene kernel before this one
+// took 10.6 and the sort its group bounds need grows with the square of the
+// boxes) and takes every gridDim.x-th tile of kBlock children: one per lane,
+// or, for the quadcopter, as the planner's tiles do. 100003 quadcopter edges
+// among 200 boxes: kernels 539 + 10.6 -> 235 us, the call 580 -> 233; 100003 of
+// the other models 102 to 246 -> 22 to 47 us, 1000 of them 55 to 65 -> 12 to 20.
+template <int MODEL>
+__global__ __launch_bounds__(kBlock, 4) void k_stage_propagate(const QueryDesc qd, const int32_t* __restrict__ parentIdx,
+                                                               const float* __restrict__ parentStates,
+                                                               uint32_t nParents, const float* __restrict__ controls,
+                                                               const int32_t* __restrict__ steps, uint32_t n,
+                                                               const float* __restrict__ rows, uint32_t nObs,
+                                                               float* __restrict__ child, uint8_t* __restrict__ valid,
+                                                               int32_t* __restrict__ r1o, int32_t* __restrict__ r2o)
+{
+    constexpr int S = ModelDims<MODEL>::S, C = ModelDims<MODEL>::C;
+    extern __shared__ float4 sObs[];
+    const MaskScene sc = stage_scene_masks<MODEL == KGMT_MODEL_UNICYCLE ? 2 : 3>(qd, rows, nObs, sObs);
+    const StageEdges<MODEL> E{parentIdx, parentStates, nParents, controls, steps, n, child, valid, r1o, r2o};
     if constexpr(MODEL == KGMT_MODEL_QUADCOPTER)
         {
             __shared__ QuadRunLds<kBlock> L;
             for(uint32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock)
                 {
-                    quad_run<kBlock>(
-                      qd, n - base < kBlock ? n - base : kBlock, sc, L, [&](uint32_t k) { return steps[base + k]; },
-                      [&](uint32_t k, QuadChild& ch) {
-                          const uint32_t i = base + k;
-                          const int32_t p  = parent(i);
-                          ch.p             = (uint32_t)p;
-#pragma unroll
-                          for(int d = 0; d < S; ++d) ch.s[d] = p < 0 ? 0.0f : parentStates[(size_t)d * nParents + p];
-#pragma unroll
-                          for(int c = 0; c < C; ++c) ch.u[c] = controls[(size_t)c * n + i];
-                          const int32_t st = steps[i];
-                          ch.uf            = 0.0f;
-                          ch.left          = p < 0 || st < 0 ? 0 : st;
-                      },
-                      [&](const QuadChild& ch) {
-                          write(base + (ch.meta & 1023u), (int32_t)ch.p, ch.s, ch.u, ch.left == 0);
-                      });
+                    stage_quad_tile<kBlock>(qd, E, base, n - base < kBlock ? n - base : kBlock, sc, L);
                     __syncthreads();  // L is used again
                 }
         }
     else
         for(uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock)
             {
-                const int32_t p = parent(i);
+                const int32_t p = E.parent(i);
                 float s[S], u[C];
                 bool ok = false;
-#pragma unroll
-                for(int d = 0; d < S; ++d) s[d] = p < 0 ? 0.0f : parentStates[(size_t)d * nParents + p];
-#pragma unroll
-                for(int k = 0; k < C; ++k) u[k] = controls[(size_t)k * n + i];
+                E.read(i, p, s, u);
                 if(p >= 0)
                     {
                         MaskCheck chk{qd, sc, MaskWalk{0, 0, 0}};
                         chk.walk.start(qd, s[0], s[1], pos_z<MODEL>(s));
                         ok = propagate_with<MODEL>(qd, s, u, steps[i], chk);
                     }
-                write(i, p, s, u, ok);
+                E.write(qd, i, p, s, u, ok);
             }
 }
 
@@ -2661,9 +2704,8 @@ __global__ __launch_bounds__(kBlock, 4) void k_stage_propagate(const QueryDesc q
 // consecutive indices, handed to the wave's lanes longest-first by the same
 // counting sort child_tile runs with one lane per child, then
 // propagate_two_phase called by every lane of the wave as child_tile calls it
-// (lanes without a child take part with an empty box), or the one-pass check
-// for the quadcopter. check / box (optional) receive the check that decided
-// each child and its edge box.
+// (lanes without a child take part with an empty box). check / box (optional)
+// receive the check that decided each child and its edge box.
 template <int MODEL>
 __global__ __launch_bounds__(kBlock) void k_stage_propagate_planner(
   const QueryDesc* __restrict__ qdp, const int32_t* __restrict__ parentIdx, const float* __restrict__ parentStates,
@@ -2671,7 +2713,7 @@ __global__ __launch_bounds__(kBlock) void k_stage_propagate_planner(
   const float4* __restrict__ obs, uint32_t nGrp, float* child, uint8_t* valid, int32_t* r1o, int32_t* r2o,
   uint8_t* checkOut, float* boxOut)
 {
-    constexpr int S = ModelDims<MODEL>::S, C = ModelDims<MODEL>::C, D = S + C + 1;
+    constexpr int S = ModelDims<MODEL>::S, C = ModelDims<MODEL>::C;
     extern __shared__ float4 sObs[];
     __shared__ float4 cand[kBlock / 64][2 * kCand];
     __shared__ uint32_t hist[kBlock];
@@ -2702,46 +2744,47 @@ __global__ __launch_bounds__(kBlock) void k_stage_propagate_planner(
         slot[hist[bucket] + rank] = (uint16_t)t;
         wave_sync();
     }
+    const StageEdges<MODEL> E{parentIdx, parentStates, nParents, controls, steps, n, child, valid, r1o, r2o};
     const uint32_t i = base + slot[t];
-    const int32_t p  = i < n ? parentIdx[i] : -1;
-    const bool has   = i < n && p >= 0 && (uint32_t)p < nParents;
-    float s[S], uc[C];
+    const int32_t p  = i < n ? E.parent(i) : -1;
+    const bool has   = p >= 0;
+    float s[S] = {}, uc[C] = {};
     int32_t st = 0;
-#pragma unroll
-    for(int d = 0; d < S; ++d) s[d] = has ? parentStates[(size_t)d * nParents + p] : 0.0f;
-#pragma unroll
-    for(int k = 0; k < C; ++k) uc[k] = has ? controls[(size_t)k * n + i] : 0.0f;
-    if(has) st = steps[i];
+    if(has) E.read(i, p, s, uc), st = steps[i];
     const Scene sc{sObs, (int)nGrp, 0};
-    bool ok = false;
-    TwoPhaseTrace tr{KGMT_CHECK_ONE_PASS, {0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}};
-    if constexpr(MODEL != KGMT_MODEL_QUADCOPTER)
-        ok = propagate_two_phase<MODEL>(qd, s, uc, st, sc, cand[t / 64], has, &tr);  // every lane
-    else if(has)
-        ok = propagate<MODEL>(qd, s, uc, st, sc);
+    TwoPhaseTrace tr{KGMT_CHECK_SCENE, {0.0f, 0.0f, 0.0f}, {0.0f, 0.0f, 0.0f}};
+    const bool ok = propagate_two_phase<MODEL>(qd, s, uc, st, sc, cand[t / 64], has, &tr);  // every lane
     if(i >= n) return;
-    if(!has)
-        {
-            // caller index out of range: no state is read; flagged by r1 = r2 = -1
-            for(int d = 0; d < D; ++d) child[(size_t)d * n + i] = 0.0f;
-            valid[i] = 0;
-            r1o[i]   = -1;
-            r2o[i]   = -1;
-            return;
-        }
-#pragma unroll
-    for(int d = 0; d < S; ++d) child[(size_t)d * n + i] = s[d];
-#pragma unroll
-    for(int k = 0; k < C; ++k) child[(size_t)(S + k) * n + i] = uc[k];
-    child[(size_t)(D - 1) * n + i] = qd.cfg.dt * (float)st;
-    int ix, iy, iz;
-    const int r1 = region_of(qd, s[0], s[1], s[2], ix, iy, iz);
-    valid[i]     = ok ? 1 : 0;
-    r1o[i]       = r1;
-    r2o[i]       = subregion_of(qd, s[0], s[1], s[2], r1, ix, iy, iz);
+    E.write(qd, i, p, s, uc, ok);
+    if(!has) return;
     if(checkOut) checkOut[i] = (uint8_t)tr.path;
-    if(boxOut && MODEL != KGMT_MODEL_QUADCOPTER)
+    if(boxOut)
         for(int d = 0; d < 3; ++d) boxOut[(size_t)d * n + i] = tr.lo[d], boxOut[(size_t)(3 + d) * n + i] = tr.hi[d];
+}
+
+// The same for the quadcopter: tiles of the planner's workgroup with one lane
+// per child (quad_run) on the planner's scene, in turn a tile of twice as many
+// children as lanes (sorted, refilled) and one of as many.
+__global__ __launch_bounds__(kTile, 4) void k_stage_quad_planner(
+  const QueryDesc* __restrict__ qdp, const int32_t* __restrict__ parentIdx, const float* __restrict__ parentStates,
+  uint32_t nParents, const float* __restrict__ controls, const int32_t* __restrict__ steps, uint32_t n,
+  const float4* __restrict__ obs, uint32_t nGrp, uint32_t nObs, float* __restrict__ child, uint8_t* __restrict__ valid,
+  int32_t* __restrict__ r1o, int32_t* __restrict__ r2o, uint8_t* __restrict__ checkOut)
+{
+    extern __shared__ float4 sObs[];
+    __shared__ QuadRunLds<kTile> L;
+    const QueryDesc& qd = *qdp;
+    const StageEdges<KGMT_MODEL_QUADCOPTER> E{parentIdx, parentStates, nParents, controls, steps, n,
+                                              child,     valid,        r1o,      r2o};
+    const MaskScene sc  = stage_masks(obs, 0, nGrp, nObs, sObs, true);
+    const uint32_t two  = blockIdx.x & 1u ? 0u : kTile;
+    const uint32_t base = (blockIdx.x >> 1) * 3u * kTile + (two ? 0u : 2u * kTile);
+    if(base >= n) return;
+    const uint32_t count = n - base < kTile + two ? n - base : kTile + two;
+    stage_quad_tile<kTile>(qd, E, base, count, sc, L);
+    if(checkOut)
+        for(uint32_t k = threadIdx.x; k < count; k += kTile)
+            if(E.parent(base + k) >= 0) checkOut[base + k] = KGMT_CHECK_ONE_PASS;
 }
 
 // Frontier update stage: the caller's tree and children staged into a
@@ -3049,6 +3092,14 @@ hipError_t launch_build_scene(const float* rows, uint32_t n, uint32_t nGrp, floa
     return hipGetLastError();
 }
 
+hipError_t launch_build_mask_scene(const QueryDesc* qd, const float* rows, uint32_t n, uint32_t nGrp, float4* out,
+                                   hipStream_t s)
+{
+    if(n == 0) return hipSuccess;
+    hipLaunchKernelGGL(k_build_mask_scene, dim3(1), dim3(kBlock), 0, s, qd, rows, n, nGrp, out);
+    return hipGetLastError();
+}
+
 hipError_t launch_finish(const QueryDesc* qds, QueryState* sts, const WorkLists& W, uint32_t parity, hipStream_t s)
 {
     hipLaunchKernelGGL(k_finish, dim3(1), dim3(kBlock), 0, s, qds, sts, W, parity);
@@ -3116,11 +3167,19 @@ hipError_t launch_stage_propagate(int model, const QueryDesc& qd, const int32_t*
 hipError_t launch_stage_propagate_planner(int model, const QueryDesc* qd, const int32_t* parentIdx,
                                           const float* parentStates, uint32_t nParents, const float* controls,
                                           const int32_t* steps, uint32_t n, const float4* obs, uint32_t nGrp,
-                                          float* child, uint8_t* valid, int32_t* r1, int32_t* r2, uint8_t* check,
-                                          float* box, hipStream_t s)
+                                          uint32_t nObs, float* child, uint8_t* valid, int32_t* r1, int32_t* r2,
+                                          uint8_t* check, float* box, hipStream_t s)
 {
     if(n == 0) return hipSuccess;
-    const dim3 g((n + kBlock - 1) / kBlock), b(kBlock);
+    if(model == KGMT_MODEL_QUADCOPTER)
+        {
+            const size_t ldsQ = (size_t)std::max<uint32_t>(nGrp * kGroup + mask_pairs(nObs), 1) * 2 * sizeof(float4);
+            hipLaunchKernelGGL(k_stage_quad_planner, dim3(2 * ((n - 1) / (3 * kTile) + 1)), dim3(kTile), ldsQ, s, qd,
+                               parentIdx, parentStates, nParents, controls, steps, n, obs, nGrp, nObs, child, valid, r1,
+                               r2, check);
+            return hipGetLastError();
+        }
+    const dim3 g((n - 1) / kBlock + 1), b(kBlock);
     const size_t lds = (size_t)(nGrp ? nGrp * (1 + kGroup) : 1) * 2 * sizeof(float4);
 #define KGMT_STAGE_PROP(M)                                                                                        \
     hipLaunchKernelGGL(k_stage_propagate_planner<M>, g, b, lds, s, qd, parentIdx, parentStates, nParents, controls, \
@@ -3130,7 +3189,6 @@ hipError_t launch_stage_propagate_planner(int model, const QueryDesc* qd, const 
             case KGMT_MODEL_DOUBLE_INTEGRATOR: KGMT_STAGE_PROP(KGMT_MODEL_DOUBLE_INTEGRATOR); break;
             case KGMT_MODEL_DUBINS_AIRPLANE: KGMT_STAGE_PROP(KGMT_MODEL_DUBINS_AIRPLANE); break;
             case KGMT_MODEL_DUBINS_5D: KGMT_STAGE_PROP(KGMT_MODEL_DUBINS_5D); break;
-            case KGMT_MODEL_QUADCOPTER: KGMT_STAGE_PROP(KGMT_MODEL_QUADCOPTER); break;
             case KGMT_MODEL_UNICYCLE: KGMT_STAGE_PROP(KGMT_MODEL_UNICYCLE); break;
             default: return hipErrorInvalidValue;
         }

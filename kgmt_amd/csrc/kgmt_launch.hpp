@@ -26,6 +26,9 @@ uint32_t scene_groups(uint32_t n);
 uint32_t scene_pairs(uint32_t n);
 // rows of 2 * wdim floats (wdim 2: planar boxes, z range [-1, 1])
 hipError_t launch_build_scene(const float* rows, uint32_t n, uint32_t nGrp, float4* out, int wdim, hipStream_t s);
+// with its box masks behind it (mask_pairs(n) more), for a 3D query
+hipError_t launch_build_mask_scene(const QueryDesc* qd, const float* rows, uint32_t n, uint32_t nGrp, float4* out,
+                                   hipStream_t s);
 
 // propagate launch shapes that are built
 bool launch_supported(uint32_t block, uint32_t lanes);
@@ -65,12 +68,13 @@ hipError_t launch_stage_propagate(int model, const QueryDesc& qd, const int32_t*
                                   uint32_t nParents, const float* controls, const int32_t* steps, uint32_t n,
                                   const float* rows, uint32_t nObs, float* child, uint8_t* valid, int32_t* r1,
                                   int32_t* r2, hipStream_t s);
-// the planner's per-child path (wave sort, two-phase or one-pass check)
+// the planner's per-child path (wave sort and two-phase check; quadcopter: its
+// tiles, obs with box masks)
 hipError_t launch_stage_propagate_planner(int model, const QueryDesc* qd, const int32_t* parentIdx,
                                           const float* parentStates, uint32_t nParents, const float* controls,
                                           const int32_t* steps, uint32_t n, const float4* obs, uint32_t nGrp,
-                                          float* child, uint8_t* valid, int32_t* r1, int32_t* r2, uint8_t* check,
-                                          float* box, hipStream_t s);
+                                          uint32_t nObs, float* child, uint8_t* valid, int32_t* r1, int32_t* r2,
+                                          uint8_t* check, float* box, hipStream_t s);
 // frontier update of one iteration on a one-query pool (the caller's tree
 // already in P.treeS / parent / cost / frontier, the scores in P.score; valid:
 // its R1 valid counts): staging kernels, then the planner's k_update;
