@@ -2677,16 +2677,19 @@ __global__ __launch_bounds__(kBlock, 4) void k_stage_propagate(const QueryDesc q
     if constexpr(MODEL == KGMT_MODEL_QUADCOPTER)
         {
             __shared__ QuadRunLds<kBlock> L;
-            for(uint32_t base = blockIdx.x * kBlock; base < n; base += gridDim.x * kBlock)
+            // (64 bits: the turn after the last can pass 2^32)
+            for(uint64_t at = blockIdx.x * kBlock; at < n; at += gridDim.x * kBlock)
                 {
+                    const uint32_t base = (uint32_t)at;
                     stage_quad_tile<kBlock>(qd, E, base, n - base < kBlock ? n - base : kBlock, sc, L);
                     __syncthreads();  // L is used again
                 }
         }
     else
-        for(uint32_t i = blockIdx.x * kBlock + threadIdx.x; i < n; i += gridDim.x * kBlock)
+        for(uint64_t at = blockIdx.x * kBlock + threadIdx.x; at < n; at += gridDim.x * kBlock)
             {
-                const int32_t p = E.parent(i);
+                const uint32_t i = (uint32_t)at;
+                const int32_t p  = E.parent(i);
                 float s[S], u[C];
                 bool ok = false;
                 E.read(i, p, s, u);
