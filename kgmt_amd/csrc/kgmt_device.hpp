@@ -901,7 +901,9 @@ __device__ __forceinline__ bool prop_dubins(const QueryDesc& qd, float* s, const
 }
 
 // a / b rounded correctly, y: 1 / b after one Newton step (no operand or
-// intermediate result near the ends of the exponent range)
+// intermediate result near the ends of the exponent range). From any
+// approximation within one unit in the last place, but for a divisor just below
+// a power of two, where it has to be the nearest float, as the unit gives it.
 __device__ __forceinline__ float quotient(float a, float b, float y)
 {
     float q = a * y;
