@@ -28,8 +28,10 @@ constexpr uint32_t kMaxObs  = 1500;  // obstacles a query may carry
 constexpr uint32_t kGroup   = 8;     // boxes per bounding group of a scene
 constexpr uint32_t kGroupBatch = 4;  // groups tested together (scenes pad to a multiple)
 // LDS of one scene: G groups + 8 G boxes, G = ceil(n / 32) * 4, as (lo, hi)
-// float4 pairs: at most 1692 pairs = 54.1 KB (+ 58.5 KB of tile state and
-// candidate lists for a 512-thread propagate tile: 113 KB of gfx950's 160 KB)
+// float4 pairs: at most 1692 pairs = 54.1 KB; of a quadcopter's with box masks
+// the boxes and the masks, at most 2080 pairs = 66.6 KB (+ 58.6 KB of tile state
+// and candidate lists for a 512-thread propagate tile of mixed models + 1 KB of
+// tile starts: 126 KB of gfx950's 160 KB)
 constexpr int32_t kNoGoal   = 0x7fffffff;
 // Box masks of a scene: the workspace cut into kSlabs slabs per axis; row
 // (axis, side, slab) has one bit per box: side 0, the boxes whose low face

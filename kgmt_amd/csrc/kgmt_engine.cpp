@@ -1484,12 +1484,12 @@ int kgmt_build_scene(const float* d_rows, uint32_t n, float* d_out, uint32_t out
 static int propagate_collide(const kgmt_config* cfg, const int32_t* d_parent_idx, const float* d_parent_states,
                              uint32_t n_parents, const float* d_controls, const int32_t* d_steps, uint32_t n_children,
                              const float* d_obstacles, uint32_t n_obs, float* d_child_samples, uint8_t* d_valid,
-                             int32_t* d_r1, int32_t* d_r2, void* stream, const char* too_many)
+                             int32_t* d_r1, int32_t* d_r2, void* stream)
 {
     if(n_children && (!d_parent_idx || !d_parent_states || !d_controls || !d_steps || !d_child_samples || !d_valid ||
                       !d_r1 || !d_r2))
         return fail(KGMT_E_ARG, "null buffer");
-    if(n_obs > kMaxObs) return fail(KGMT_E_CAPACITY, too_many);
+    if(n_obs > kMaxObs) return fail(KGMT_E_CAPACITY, "more than 1500 obstacles");
     if(n_obs && !d_obstacles) return fail(KGMT_E_ARG, "obstacles pointer is null");
     int rc = check_config(cfg);
     if(rc) return rc;
@@ -1509,8 +1509,7 @@ int kgmt_propagate_collide(const kgmt_config* cfg, const int32_t* d_parent_idx, 
                            int32_t* d_r1, int32_t* d_r2, void* stream)
 {
     return propagate_collide(cfg, d_parent_idx, d_parent_states, n_parents, d_controls, d_steps, n_children,
-                             d_obstacles, n_obs, d_child_samples, d_valid, d_r1, d_r2, stream,
-                             "more than 1500 obstacles");
+                             d_obstacles, n_obs, d_child_samples, d_valid, d_r1, d_r2, stream);
 }
 
 int kgmt_propagate_collide_noalloc(const kgmt_config* cfg, const int32_t* d_parent_idx, const float* d_parent_states,
@@ -1521,8 +1520,7 @@ int kgmt_propagate_collide_noalloc(const kgmt_config* cfg, const int32_t* d_pare
 {
     if(!cfg) return fail(KGMT_E_ARG, "null configuration");
     return propagate_collide(cfg, d_parent_idx, d_parent_states, n_parents, d_controls, d_steps, n_children,
-                             d_obstacles, n_obs, d_child_samples, d_valid, d_r1, d_r2, stream,
-                             "more than 1500 obstacles: the scratch scene holds at most 1500 boxes");
+                             d_obstacles, n_obs, d_child_samples, d_valid, d_r1, d_r2, stream);
 }
 
 int kgmt_propagate_collide_planner(const kgmt_config* cfg, const int32_t* d_parent_idx,

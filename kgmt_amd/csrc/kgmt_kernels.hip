@@ -601,6 +601,7 @@ __device__ __forceinline__ void child_tile(const QueryDesc& qd, const QueryState
                                            bool stage)
 {
     constexpr int S = ModelDims<MODEL>::S, C = ModelDims<MODEL>::C;
+    static_assert(K > 1 || MODEL != KGMT_MODEL_QUADCOPTER, "one lane per child: quad_tile");
     constexpr uint32_t TC = NT / K;
     const uint32_t nC  = st.nChildrenN;
     const uint32_t cap = qd.cap;
@@ -743,7 +744,7 @@ __device__ __forceinline__ void child_tile(const QueryDesc& qd, const QueryState
         }
     if constexpr(K == 1) wave_sync();  // the stage is read before the check writes candidates
     const Scene sc{sObs, (int)qd.nGrp, (int)(t % K)};
-    if constexpr(K == 1 && MODEL != KGMT_MODEL_QUADCOPTER)
+    if constexpr(K == 1)
         ok = propagate_two_phase<MODEL>(qd, s, uc, steps, sc, L.cand[t / 64], has);  // every lane
     else if(has)
         ok = propagate<MODEL, K>(qd, s, uc, steps, sc);
