@@ -150,11 +150,12 @@ __device__ __forceinline__ float quad_scatter(const float (&v)[4], int lane)
 // error out (the residuals of the root and of the quotients, the rest of the
 // exponent's product): one box's penalty is 0.7 to 1.05 times as far from 64
 // bits as by the library's sqrt, division, expf and log1pf (its gradient 0.75
-// to 1.1 times), 1.0 to 2.2 times without. That costs 8 %: refine of 4096
-// trajectories among 50 boxes 7.48 to 8.00 ms. acc: half the logarithms, and
+// to 1.1 times), 1.0 to 2.2 times without. That costs 4 %: refine of 4096
+// trajectories among 50 boxes 7.48 to 7.77 ms. acc: half the logarithms, and
 // the gradient; flat: the max(x, 0).
 __device__ __forceinline__ void box_penalty(float4 lo, float4 hi, float px, float py, float pz, float margin,
-                                            float tau, const RolloutK& K, float (&acc)[4], float& flat)
+                                            float tau, const RolloutK& K, bool plain, uint64_t anyPlain,
+                                            float (&acc)[4], float& flat)
 {
     const float lx = lo.x - px, hx = px - hi.x, ly = lo.y - py, hy = py - hi.y, lz = lo.z - pz, hz = pz - hi.z;
     const bool nx = lx > hx, ny = ly > hy, nz = lz > hz;  // nearer the low face
@@ -172,12 +173,14 @@ __device__ __forceinline__ void box_penalty(float4 lo, float4 hi, float px, floa
     // alone: a face or a corner within 1e-19 and a box farther than 1.8e19
     // take a scaled root, as inside does, and the plain quotient by tau (rare:
     // one vote of the active lanes skips it; the other lanes keep what they
-    // have; K.plain: tau or margin out of the range of the short form)
+    // have; plain: a position or a scene that is not finite, or tau or margin
+    // out of the range of the short form)
     float vx = ox * id, vy = oy * id, vz = oz * id;
-    const bool tiny = !(d2 >= 0x1p-126f), huge = !(d2 <= 0x1.fffffep127f);
-    const bool odd  = tiny | huge | __builtin_isunordered(qx, qy) | (qz != qz) | (K.plain != 0u);
-    if(__any(odd))
+    const bool edge = __builtin_amdgcn_classf(d2, 0x2ff);  // not a positive normal
+    if((__builtin_amdgcn_ballot_w64(edge) | anyPlain) != 0u)
         {
+            const bool odd  = plain | edge;
+            const bool tiny = !(d2 >= 0x1p-126f), huge = !(d2 <= 0x1.fffffep127f);
             const float k  = tiny ? 0x1p100f : huge ? 0x1p-100f : 1.0f;
             const float rk = tiny ? 0x1p-100f : huge ? 0x1p100f : 1.0f;
             const float kx = ox * k, ky = oy * k, kz = oz * k;
@@ -205,8 +208,9 @@ __device__ __forceinline__ void box_penalty(float4 lo, float4 hi, float px, floa
     at             = __builtin_fmaf(u, at, 0x1.9998d4p-3f);
     at             = __builtin_fmaf(u, at, 0x1.555556p-2f);
     acc[0]         = __builtin_fmaf(tau, t0 + __builtin_fmaf(t * u, at, tr), acc[0]);  // (half of it)
-    flat += fmaxf(x, 0.0f);
-    const float n  = x >= 0.0f ? 1.0f : e;
+    const bool up  = x >= 0.0f;
+    flat += up ? x : 0.0f;
+    const float n  = up ? 1.0f : e;
     const float g0 = n * r1, g = __builtin_fmaf(__builtin_fmaf(-g0, e1, n), r1, g0);
     acc[1]         = __builtin_fmaf(nx ? g : -g, vx, acc[1]);
     acc[2]         = __builtin_fmaf(ny ? g : -g, vy, acc[2]);
@@ -251,12 +255,18 @@ __global__ __launch_bounds__(64) void k_rollout(RolloutK K, kgmt_adjoint_params 
     __shared__ RolloutLds L;
     const int lane = (int)threadIdx.x;
     const uint32_t nBox = box_slots(nObs);  // the read ahead ends inside the slots (unused ones hold anything)
+    bool odd            = K.plain != 0u;
     for(uint32_t k = lane; k < nObs; k += 64)
         {
             const float* r = rows + 6 * (size_t)k;
-            sBox[k]        = make_float4(r[0], r[1], r[2], 0.0f);
-            sBox[nBox + k] = make_float4(r[3], r[4], r[5], 0.0f);
+            const float4 lo = make_float4(r[0], r[1], r[2], 0.0f), hi = make_float4(r[3], r[4], r[5], 0.0f);
+            sBox[k]        = lo;
+            sBox[nBox + k] = hi;
+            // (0 x: NaN unless x is finite)
+            const float f = 0.0f * lo.x + 0.0f * lo.y + 0.0f * lo.z + 0.0f * hi.x + 0.0f * hi.y + 0.0f * hi.z;
+            odd |= f != 0.0f;
         }
+    const bool scenePlain = __any(odd);
     __syncthreads();
     const uint32_t slot = (blockIdx.x * 64 + lane) / LPT;
     const uint32_t i    = i0 + slot < n ? i0 + slot : n - 1;  // lanes past the end read the last trajectory
@@ -449,11 +459,14 @@ __global__ __launch_bounds__(64) void k_rollout(RolloutK K, kgmt_adjoint_params 
                     // boxes s, s + 4, ... against this lane's step, each read
                     // while the one before it is worked on
                     float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f}, flat = 0.0f;
+                    const bool plain = scenePlain | !(fmaxf(fmaxf(fabsf(qx), fabsf(qy)), fabsf(qz)) < INFINITY) |
+                                       __builtin_isunordered(qx, qy) | (qz != qz);
+                    const uint64_t anyPlain = __builtin_amdgcn_ballot_w64(plain);
                     float4 lo = sBox[s], hi = sBox[nBox + s];
                     for(uint32_t o = s; o < nObs; o += 4)
                         {
                             const float4 l1 = sBox[o + 4], h1 = sBox[nBox + o + 4];
-                            box_penalty(lo, hi, qx, qy, qz, ap.margin, ap.tau, K, acc, flat);
+                            box_penalty(lo, hi, qx, qy, qz, ap.margin, ap.tau, K, plain, anyPlain, acc, flat);
                             lo = l1, hi = h1;
                         }
                     acc[0] += acc[0] + flat;
