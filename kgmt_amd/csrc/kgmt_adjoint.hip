@@ -19,8 +19,9 @@
 //      step takes a quarter of the instructions that one lane would need. The
 //      four stages' states are kept for the passes below.
 //   2. positions, penalties and J, lane = (step, stage): the stages' world
-//      velocities, their sum over a step by quad permutations, a scan over the
-//      steps, then the boxes spread over the trajectory's lanes.
+//      velocities, their sum over a step by quad permutations, a scan over
+//      groups of four steps and a sum over the groups, then the boxes spread
+//      over a step's four lanes.
 //   3. backward, lane = (step, stage): the stage's vector-Jacobian product as
 //      eight rows of coefficients in LDS (the adjoints of the positions and of
 //      psi do not depend on the others: suffix sums over the steps, folded
@@ -29,9 +30,9 @@
 //      broadcast operands.
 // The kernel that ran the whole step in every lane of a trajectory took
 // 47.2 ms for 4096 trajectories (20..80 steps, 50 Adam steps, 50 boxes),
-// 1.18 ms for one cost and gradient of them and 1.42 ms for 333 trajectories
-// among 301 boxes; this one takes 7.33, 0.21 and 0.11 ms, and its error
-// against 64 bits is smaller (gradient of the 333: 2.2e-6 to 5.8e-7).
+// 1.28 ms for one cost and gradient of them and 1.51 ms for 333 trajectories
+// among 301 boxes; this one takes 7.78, 0.23 and 0.13 ms, and its error
+// against 64 bits is smaller (gradient of the 333: 2.4e-6 to 2.7e-7).
 #include <algorithm>
 
 #include "kgmt_launch.hpp"

@@ -812,7 +812,7 @@ __device__ __forceinline__ void child_tile(const QueryDesc& qd, const QueryState
 // ---------------------------------------------------------------------------
 // Most edges of a quadcopter end long before their drawn 10 to 50 steps (out
 // of the workspace, past a speed bound, in a box: 8 to 16 steps on average on
-// the configured queries), and a step is about 1300 instructions, so a wave
+// the configured queries), and a step is about 1090 instructions, so a wave
 // that runs until its longest edge ends leaves more than half of its lanes
 // idle (2.0 to 2.5 times the steps needed). A tile's lanes are therefore
 // looked over every kQuadSteps steps: with children left, once 64 lanes are
