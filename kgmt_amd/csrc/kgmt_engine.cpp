@@ -805,29 +805,31 @@ struct Engine
     // sparse_valid_below or not), 0 otherwise (KGMT.cu:336-339, 373)
     int get_frontier(uint32_t q, uint8_t* frontier, uint32_t* repeat, uint32_t cap, uint32_t* n)
     {
-        HIP_TRY(hipStreamSynchronize(stream));  // a plan returns before its trailing launches drain
-        QueryState st;
-        HIP_TRY(hipMemcpy(&st, ds + q, sizeof(QueryState), hipMemcpyDeviceToHost));
         const QueryDesc& qd = hq[q];
-        const uint32_t ts   = st.treeSizeN;
+        const uint32_t ts   = hs[q].treeSize;
         if(n) *n = ts;
         if(!frontier && !repeat) return KGMT_OK;
         if(cap < ts) return fail(KGMT_E_CAPACITY, "frontier output buffer too small");
+        HIP_TRY(hipStreamSynchronize(stream));  // a plan returns before its trailing launches drain
+        QueryState st;
+        HIP_TRY(hipMemcpy(&st, ds + q, sizeof(QueryState), hipMemcpyDeviceToHost));
         if(frontier) HIP_TRY(hipMemcpy(frontier, P.frontier + qd.nodeOff, ts, hipMemcpyDeviceToHost));
-        if(repeat)
+        if(!repeat) return KGMT_OK;
+        const uint32_t next = std::min(st.next, ts), old = ts - next;
+        std::vector<uint8_t> react(old);
+        std::vector<int32_t> r1(next);
+        std::vector<uint64_t> cnt(next ? 16u << qd.regShift : 0u);
+        if(old) HIP_TRY(hipMemcpy(react.data(), P.react + qd.nodeOff, old, hipMemcpyDeviceToHost));
+        if(next)
             {
-                const uint32_t next = std::min(st.next, ts), old = ts - next;
-                std::vector<uint8_t> react(old);
-                std::vector<int32_t> r1(next), valid;
-                if(old) HIP_TRY(hipMemcpy(react.data(), P.react + qd.nodeOff, old, hipMemcpyDeviceToHost));
-                if(next)
-                    HIP_TRY(hipMemcpy(r1.data(), P.r1node + qd.nodeOff + old, sizeof(int32_t) * next,
-                                      hipMemcpyDeviceToHost));
-                if(int rc = region_counts(q, nullptr, &valid)) return rc;
-                for(uint32_t i = 0; i < old; ++i) repeat[i] = react[i] ? 1u : 0u;
-                for(uint32_t j = 0; j < next; ++j)
-                    repeat[old + j] = valid[r1[j]] < qd.cfg.sparse_valid_below ? qd.cfg.repeat_sparse
-                                                                                  : qd.cfg.repeat_dense;
+                HIP_TRY(hipMemcpy(r1.data(), P.r1node + qd.nodeOff + old, sizeof(int32_t) * next, hipMemcpyDeviceToHost));
+                HIP_TRY(hipMemcpy(cnt.data(), P.cnt + qd.regOff, sizeof(uint64_t) * cnt.size(), hipMemcpyDeviceToHost));
+            }
+        for(uint32_t i = 0; i < old; ++i) repeat[i] = react[i] ? 1u : 0u;
+        for(uint32_t j = 0; j < next; ++j)
+            {
+                const int32_t valid = (int32_t)(cnt[region_slot((uint32_t)r1[j], qd.regShift)] >> 32);
+                repeat[old + j]     = valid < qd.cfg.sparse_valid_below ? qd.cfg.repeat_sparse : qd.cfg.repeat_dense;
             }
         return KGMT_OK;
     }
